@@ -734,7 +734,7 @@ def exact(case, seed):
     n, _, nb, steps = _count(case)
     if case["kind"] == "ensemble":
         # one run after another; the largest decides
-        if case["runs"]*steps*case["n_hi"]**2 > 6.0e12:
+        if case["runs"]*steps*case["n_hi"]**2 > 4.0e11:
             return None
         out = []
         for p in _ensemble(case, seed):
