@@ -315,7 +315,7 @@ int spx_run_set_end_of_step_omega(spx_run* run, int32_t eager);
    compatible-energy update (sizes[0..3), each 4 or 8: how many neighbours' loads a lane
    issues before using them).  Every size gives the same result bits.  By default (sizes null
    or sizes[0] <= 0) the engine measures: after two warm-up steps it alternates 4 and 8 per
-   pass over six steps, timing each, moves a pass off its default (4, 8, 8) only when the
+   pass over six steps, timing each, moves a pass off its default (8, 8, 8) only when the
    other size is at least 3 % faster, and measures again once the active particle count has
    changed by more than 2x. */
 int spx_run_set_group_sizes(spx_run* run, const int32_t* sizes);

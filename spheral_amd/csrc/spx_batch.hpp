@@ -13,7 +13,7 @@
 // code), then the finished runs, then removed runs until they are squeezed out.
 //
 // Neighbour lists are filtered every step from per-run candidate lists (k_candidates,
-// k_neighbor_filter).  A run re-sorts and rebuilds its candidates only when its own nodes
+// k_density_dt).  A run re-sorts and rebuilds its candidates only when its own nodes
 // have moved or grown enough that the list might miss a pair (measured in k_full_update), so the
 // rebuild schedule of a run, and with it every bit of its results, does not depend on
 // the other runs of the batch.
@@ -60,6 +60,14 @@ static inline double choose_skin(double rate, int D) {
   }
   return best;
 }
+
+// Active particles up to which the grad-h pass takes four lanes per node (one lane beyond): KH 2-D
+// 4096 mixed 24 -> 11.6 us, Sod 3-D 25k mixed 71 -> 32.5, KH 65536 FP64 27.4 -> 20.4, Evrard 250k
+// mixed 118 -> 118, Taylor-Green 96^3 mixed 170 -> 185, 128^3 FP64 392 -> 493 (the kernel table is
+// staged by four times the blocks, and one lane per node already fills the GPU).
+constexpr int64_t kOmegaWideNodes = 250000;
+// Entries in flight per lane of the package-level calls' passes.
+constexpr int kFilterLoads = 2, kUpdateLoads = 2;
 
 // Value of an order-preserving bit key written by a max-reduction (0: nothing measured).
 static inline double skin_value(unsigned long long b) { return b == 0ull ? 0.0 : ord_value(b); }
@@ -181,7 +189,7 @@ class Batch {
   // count and the particle count.  The batch measures instead of guessing: once a composition
   // has run two warm-up steps it alternates sizes 4 and 8 of every pass over six steps (HIP
   // events around each pass, three samples per size), and moves a pass off its default size
-  // (4, 8, 8: measured on Taylor-Green 128^3) only when the other size's fastest sample is at
+  // (8, 8, 8: measured on Taylor-Green 128^3) only when the other size's fastest sample is at
   // least 3 % faster; it measures again once the active particle count has changed by more
   // than 2x.  Callers may fix the sizes (setGroupSizes).
   struct GroupTuner {
@@ -1151,18 +1159,17 @@ class Batch {
     bool ok = false;
     for (int attempt = 0; attempt < 3 && !ok; ++attempt) {
       HIP_CHECK(hipMemsetAsync(dOverflow, 0, sizeof(int), stream));
-      const unsigned nbx = xcd_grid(nActive, kBlock);
       if (withDensityDt) {
         // the step's sum density and dt vote ride on the filter
         hipLaunchKernelGGL(k_reset_dt, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns);
         tuneMark(0);
-        launchFilter(nbx, dOverflow);
+        launchFilter(dOverflow);
         tuneMark(1);
       } else {
         launchD([&](auto d) {
           constexpr int DD = decltype(d)::value;
-          hipLaunchKernelGGL((k_neighbor_filter<DD, kGroup>), dim3(nbx), dim3(kBlock), 0, stream, f, geo, ph,
-                             (int)nActive, dOverflow);
+          hipLaunchKernelGGL((k_density_dt<DD, false, false, double, kFilterLoads, true>), dim3(nodeGrid()),
+                             dim3(kBlock), 0, stream, f, geo, ph, dtab, (int)nActive, dsc, dOverflow, 0);
         });
       }
       HIP_CHECK(hipGetLastError());
@@ -1225,36 +1232,44 @@ class Batch {
       if (mid) packMid(true);
       return;
     }
-    const int nb = (int)xcd_grid(nActive, kBlock);
     // midpoint: the record k_midstep wrote; state: the connectivity record (k_pack), or the
     // end-of-step position k_full_update left in it
     if (mid) tuneMark(2);
-    if (groupSize(1) == 8) launchOmega<8>(mid, nb, runMask);
-    else launchOmega<4>(mid, nb, runMask);
+    if (groupSize(1) == 8) launchOmega<8>(mid, runMask);
+    else launchOmega<4>(mid, runMask);
     if (mid) tuneMark(3);
   }
+  // Grid of a pass with kNodeLanes lanes per node.
+  int nodeGrid() const { return (int)xcd_grid(nActive*kNodeLanes, kBlock); }
+  // G neighbours of a node in flight: with one lane per node G entries per lane, with four G/4.
   template <int G>
-  void launchOmega(bool mid, int nb, const int* runMask) {
+  void launchOmega(bool mid, const int* runMask) {
     launchD([&](auto d) {
       constexpr int DD = decltype(d)::value;
-      if (mid)
-        launchPrecTable(k_omega<DD, double, true, G>, k_omega<DD, float, true, G>, nb, f, geo, dtab, (int)nActive,
-                        (const double*)f.xhm, f.omegam, runMask);
-      else
-        launchPrecTable(k_omega<DD, double, false, G>, k_omega<DD, float, false, G>, nb, f, geo, dtab, (int)nActive,
-                        (const double*)f.xh, f.omega, runMask);
+      auto go = [&](auto lanes, auto m) {
+        constexpr int L = decltype(lanes)::value, U = G/L;
+        constexpr bool M = decltype(m)::value;
+        launchPrecTable(k_omega<DD, double, M, U, L>, k_omega<DD, float, M, U, L>, (int)xcd_grid(nActive*L, kBlock), f,
+                        geo, dtab, (int)nActive, (const double*)(M ? f.xhm : f.xh), M ? f.omegam : f.omega, runMask);
+      };
+      auto pick = [&](auto m) {
+        if (nActive <= kOmegaWideNodes) go(std::integral_constant<int, kNodeLanes>{}, m);
+        else go(std::integral_constant<int, 1>{}, m);
+      };
+      if (mid) pick(std::true_type{});
+      else pick(std::false_type{});
     });
   }
   // The step's filtering sum-density + dt pass (see buildConnectivity).
-  void launchFilter(unsigned nbx, int* overflow) {
+  void launchFilter(int* overflow) {
     launchD([&](auto d) {
       constexpr int DD = decltype(d)::value;
       if (groupSize(0) == 8)
-        launchPrecTable(k_density_dt<DD, true, true, double, 8, true>, k_density_dt<DD, true, true, float, 8, true>,
-                        (int)nbx, f, geo, ph, dtab, (int)nActive, dsc, overflow);
+        launchPrecTable(k_density_dt<DD, true, true, double, 2, true>, k_density_dt<DD, true, true, float, 2, true>,
+                        nodeGrid(), f, geo, ph, dtab, (int)nActive, dsc, overflow);
       else
-        launchPrecTable(k_density_dt<DD, true, true, double, 4, true>, k_density_dt<DD, true, true, float, 4, true>,
-                        (int)nbx, f, geo, ph, dtab, (int)nActive, dsc, overflow);
+        launchPrecTable(k_density_dt<DD, true, true, double, 1, true>, k_density_dt<DD, true, true, float, 1, true>,
+                        nodeGrid(), f, geo, ph, dtab, (int)nActive, dsc, overflow);
     });
   }
 
@@ -1343,18 +1358,18 @@ class Batch {
   // which must describe the current state (pack()).
   void densityDt(bool dens, bool dtv) {
     if (nActive == 0) return;
-    const int nb = (int)xcd_grid(nActive, kBlock);
+    const int nb = nodeGrid();
     if (dtv) hipLaunchKernelGGL(k_reset_dt, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns);
     launchD([&](auto d) {
       constexpr int DD = decltype(d)::value;
       if (dens && dtv)
-        launchPrecTable(k_density_dt<DD, true, true, double, kGroup>, k_density_dt<DD, true, true, float, kGroup>, nb, f,
+        launchPrecTable(k_density_dt<DD, true, true, double, kFilterLoads>, k_density_dt<DD, true, true, float, kFilterLoads>, nb, f,
                         geo, ph, dtab, (int)nActive, dsc, (int*)nullptr);
       else if (dens)
-        launchPrecTable(k_density_dt<DD, true, false, double, kGroup>, k_density_dt<DD, true, false, float, kGroup>, nb,
+        launchPrecTable(k_density_dt<DD, true, false, double, kFilterLoads>, k_density_dt<DD, true, false, float, kFilterLoads>, nb,
                         f, geo, ph, dtab, (int)nActive, dsc, (int*)nullptr);
       else
-        launchPrecTable(k_density_dt<DD, false, true, double, kGroup>, k_density_dt<DD, false, true, float, kGroup>, nb,
+        launchPrecTable(k_density_dt<DD, false, true, double, kFilterLoads>, k_density_dt<DD, false, true, float, kFilterLoads>, nb,
                         f, geo, ph, dtab, (int)nActive, dsc, (int*)nullptr);
     });
   }
@@ -1641,7 +1656,7 @@ class Batch {
     if (overlap) gravityPass(true, false, true);
     mark("sph");
     joinGravity();
-    fullStep(nb);
+    fullStep();
   }
 
   // Integrator::step with SynchronousRK2::step and the SPH package (Integrator/SynchronousRK2.cc:
@@ -1680,7 +1695,7 @@ class Batch {
     // trial half step, then the midpoint postStateUpdate (grad-h Omega and the records)
     launchD([&](auto d) {
       constexpr int DD = decltype(d)::value;
-      launchPrec(k_half_update<DD, double, kGroupUpdate>, k_half_update<DD, float, kGroupUpdate>, nb, f, geo, ph,
+      launchPrec(k_half_update<DD, double, kUpdateLoads>, k_half_update<DD, float, kUpdateLoads>, nodeGrid(), f, geo, ph,
                  (const Scalars*)dsc, (int)nActive);
     });
     mark("update");
@@ -1691,13 +1706,13 @@ class Batch {
     sphPass(false, true, true);
     copyQVelocityGradient();
     mark("sph");
-    fullStep(nb);
+    fullStep();
   }
 
   // The full step from the start-of-step state with the midpoint derivatives (compatible energy
   // first), the end-of-step grad-h Omega and the time advance; shared by both integrators.
-  void fullStep(int nb) {
-    fullStepLaunches(nb);
+  void fullStep() {
+    fullStepLaunches();
     omegaStale = cfg.gradh_correction != 0;
     if (eagerOmega) ensureOmega();
     download(hsc, dsc, sizeof(Scalars)*maxRuns);
@@ -1708,16 +1723,16 @@ class Batch {
   }
   // The full step's launches: update (compatible energy first), velocity buffer swap, end-of-step
   // grad-h Omega, time advance.
-  void fullStepLaunches(int nb) {
+  void fullStepLaunches() {
     tuneMark(6);
     launchD([&](auto d) {
       constexpr int DD = decltype(d)::value;
       if (groupSize(2) == 8)
-        launchPrec(k_full_update<DD, false, double, 8>, k_full_update<DD, false, float, 8>, nb, f, geo, ph, dsc, 0.0,
-                   (int)nActive);
+        launchPrec(k_full_update<DD, false, double, 2>, k_full_update<DD, false, float, 2>, nodeGrid(), f, geo, ph, dsc,
+                   0.0, (int)nActive);
       else
-        launchPrec(k_full_update<DD, false, double, 4>, k_full_update<DD, false, float, 4>, nb, f, geo, ph, dsc, 0.0,
-                   (int)nActive);
+        launchPrec(k_full_update<DD, false, double, 1>, k_full_update<DD, false, float, 1>, nodeGrid(), f, geo, ph, dsc,
+                   0.0, (int)nActive);
     });
     tuneMark(7);
     for (int a = 0; a < D; ++a) {
@@ -1807,7 +1822,7 @@ class Batch {
     pack();
     hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, stream, dOverflowG, 1, 0);
     hipLaunchKernelGGL(k_reset_dt, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns);
-    launchFilter(xcd_grid(nActive, kBlock), dOverflowG);
+    launchFilter(dOverflowG);
     const int nb = (int)xcd_grid(nActive, kBlock);
     hipLaunchKernelGGL(k_select_dt, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns, ph, cfg.dt_min,
                        cfg.dt_max, cfg.dt_growth, cfg.gravity);
@@ -1819,7 +1834,7 @@ class Batch {
     HIP_CHECK(hipGetLastError());
     omegaPass(true);
     sphPass(false, true, true);
-    fullStepLaunches(nb);
+    fullStepLaunches();
   }
   void graphStep() {
     connectivityPrep(false);
@@ -1997,8 +2012,8 @@ class Batch {
       constexpr int DD = decltype(d)::value;
       hipLaunchKernelGGL(k_v12<DD>, dim3(nblocks(nActive)), dim3(kBlock), 0, stream, f, (const Scalars*)nullptr,
                          0.5*multiplier, (int)nActive);
-      launchPrec(k_full_update<DD, true, double, kGroupUpdate>, k_full_update<DD, true, float, kGroupUpdate>,
-                 (int)xcd_grid(nActive, kBlock), f, geo, ph, dsc, multiplier, (int)nActive);
+      launchPrec(k_full_update<DD, true, double, kUpdateLoads>, k_full_update<DD, true, float, kUpdateLoads>,
+                 nodeGrid(), f, geo, ph, dsc, multiplier, (int)nActive);
     });
     eos();
     HIP_CHECK(hipStreamSynchronize(stream));

@@ -25,20 +25,17 @@ __host__ __device__ __forceinline__ size_t ell_at(int k, int i, size_t ld) {
   return (((size_t)(k >> 3)*ld + (size_t)i) << 3) + (size_t)(k & 7);
 }
 
-// Neighbour entries are consumed in groups of G (4 or 8): one or two 16-byte loads of the
-// blocked list, then every neighbour read of the group is issued before any is used, so a
-// wavefront waits on memory once per group instead of twice per neighbour.  Positions past the end of the list
-// (k0 + u >= nn) become the lane's own slot with no image, and are skipped by the caller.
-// The filtering sum-density + dt pass: 4 in flight (137 VGPRs, 3 waves/SIMD) 1.28 ms per step on
-// FP64 Taylor-Green 128^3; 8 in flight (219 VGPRs, 2 waves) 1.32 ms.
-constexpr int kGroup = 4;
-// The compatible-energy update does little arithmetic per neighbour; it keeps 8 in flight.
-// FP64 Taylor-Green 128^3 per step: 8 in flight (184 VGPRs, 2 waves/SIMD) 0.96 ms; 4 in flight
-// (102 VGPRs, 4 waves) 1.16 ms; 8 capped at 3 waves (167 VGPRs, no spills) 1.04 ms.
+// Neighbour entries of a node are consumed in groups of G (4 or 8): every record of the group is
+// requested before any is used, so a wavefront waits on memory once per group instead of twice per
+// neighbour.  With four lanes per node a group is G/4 entries of each lane.  Defaults of the
+// filtering sum-density pass, the energy update and the grad-h passes (a batch measures 4 against 8);
+// Taylor-Green 128^3 FP64 per step: filter 8 -> 1.08 ms, 4 -> 1.40; update 0.82 / 0.83; grad-h (one
+// lane per node there) 0.39 / 0.44.
+constexpr int kGroup = 8;
 constexpr int kGroupUpdate = 8;
-// The grad-h passes read 32 bytes per neighbour and evaluate one kernel lookup: 8 in flight
-// (88 VGPRs, 5 waves/SIMD) measured 0.92 -> 0.906 ms FP64 per step on Taylor-Green 128^3.
 constexpr int kGroupOmega = 8;
+// With one lane per node the group's entries come in one or two 16-byte loads of the blocked list;
+// positions past the end of the list (k0 + u >= nn) become the lane's own slot with no image.
 template <int G>
 __device__ __forceinline__ void ell_group(const uint32_t* nbr, size_t ld, int k0, int i, int nn, int* js, int* codes) {
   uint32_t e[G];
@@ -62,6 +59,129 @@ __device__ __forceinline__ void ell_group(const uint32_t* nbr, size_t ld, int k0
     js[u] = ok ? (int)(e[u] & kIdxMask) : i;
     codes[u] = ok ? (int)(e[u] >> kImgShift) : 0;
   }
+}
+
+// Lanes per node of the pair passes: four lanes of a quad share node i, lane `sub` taking the list
+// entries k = sub, sub + 4, ...  One lane per node leaves a small run's passes bound by a lane
+// walking its 40 to 120 neighbours in turn (Kelvin-Helmholtz 4096 mixed: the filtering pass 70.7 ->
+// 24.2 us, the energy update 33.3 -> 13.6 us).
+constexpr int kNodeLanes = 4;
+
+// Value of lane Q of each quad, in every lane of the quad (quad_perm [Q, Q, Q, Q]).
+template <int Q>
+__device__ __forceinline__ int quad_lane(int v) { return __builtin_amdgcn_mov_dpp(v, Q*0x55, 0xf, 0xf, false); }
+template <int Q>
+__device__ __forceinline__ float quad_lane(float v) { return __int_as_float(quad_lane<Q>(__float_as_int(v))); }
+template <int Q>
+__device__ __forceinline__ double quad_lane(double v) {
+  return __hiloint2double(quad_lane<Q>(__double2hiint(v)), quad_lane<Q>(__double2loint(v)));
+}
+// quad_perm CTRL of a double: 0xB1 swaps neighbouring lanes, 0x4E swaps the halves of a quad.
+template <int CTRL>
+__device__ __forceinline__ double quad_swap(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+
+// A node's sum over its list, L lanes per node.  Ordered: terms are added in list order, as one lane
+// alone would add them, so the lane count never shows in the bits (every lane of the quad adds all
+// four lanes' terms, passed along by DPP).  Otherwise each lane keeps its own partial sum and the
+// four are joined at the end.  Mixed precision is always ordered: there a last-bit change of an FP64
+// sum flips FP32 roundings of later steps' pair terms.  Every lane of a quad must call add()
+// together, with a zero term where it has none (adding it changes nothing).
+template <int L, bool ORDERED>
+struct NodeSum {
+  double a;
+  __device__ __forceinline__ NodeSum(double first, int sub) : a(ORDERED || L == 1 || sub == 0 ? first : 0.0) {}
+  template <typename T>
+  __device__ __forceinline__ void add(T t) {
+    if (L == 1 || !ORDERED) {
+      a += (double)t;
+    } else {
+      a += (double)quad_lane<0>(t);
+      a += (double)quad_lane<1>(t);
+      a += (double)quad_lane<2>(t);
+      a += (double)quad_lane<3>(t);
+    }
+  }
+  template <typename T>
+  __device__ __forceinline__ void add(double m, T t) {
+    if (L == 1 || !ORDERED) {
+      a += m*(double)t;
+    } else {
+      a += quad_lane<0>(m)*(double)quad_lane<0>(t);
+      a += quad_lane<1>(m)*(double)quad_lane<1>(t);
+      a += quad_lane<2>(m)*(double)quad_lane<2>(t);
+      a += quad_lane<3>(m)*(double)quad_lane<3>(t);
+    }
+  }
+  __device__ __forceinline__ double total() const {
+    if (L == 1 || ORDERED) return a;
+    double v = a;
+    v += quad_swap<0xB1>(v);
+    return v + quad_swap<0x4E>(v);
+  }
+};
+
+// The list entries k0 + sub, k0 + sub + L, ... (U of them) of node i.  One lane per node: U entries in
+// one or two 16-byte loads.  Past the end of the list: the node itself, with no image and in[] false.
+template <int U, int L>
+__device__ __forceinline__ void lane_entries(const uint32_t* nbr, size_t ld, int k0, int sub, int i, int nn, int* js,
+                                             int* codes, bool* in) {
+  if constexpr (L == 1) {
+    ell_group<U>(nbr, ld, k0, i, nn, js, codes);
+#pragma unroll
+    for (int u = 0; u < U; ++u) in[u] = k0 + u < nn;
+  } else {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + u*L + sub;
+      in[u] = k < nn;
+      const uint32_t e = in[u] ? nbr[ell_at(k, i, ld)] : (uint32_t)i;
+      js[u] = (int)(e & kIdxMask);
+      codes[u] = (int)(e >> kImgShift);
+    }
+  }
+}
+
+// Expressions whose rounding must not depend on where they are compiled (a contraction the compiler
+// may choose either way moves a result by a last bit, and one kernel's variants must agree):
+// a product rounded by itself, and e0^2 + e1^2 + ... as one fused chain in that order (norm2) or
+// starting from e1 (norm2_second).
+template <typename R>
+__device__ __forceinline__ R rounded_product(R a, R b) {
+#pragma clang fp contract(off)
+  return a*b;
+}
+__device__ __forceinline__ float fused(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fused(double a, double b, double c) { return __builtin_fma(a, b, c); }
+template <int D, typename R>
+__device__ __forceinline__ R norm2(const R* e) {
+  R s = rounded_product(e[0], e[0]);
+#pragma unroll
+  for (int a = 1; a < D; ++a) s = fused(e[a], e[a], s);
+  return s;
+}
+
+template <int D, typename R>
+__device__ __forceinline__ R norm2_second(const R* e) {
+  const R t[3] = {e[1 % D], e[0], e[2 % D]};
+  return D == 1 ? rounded_product(e[0], e[0]) : norm2<D>(t);
+}
+
+// 1/x and 1/sqrt(x) from the hardware's estimate and one third-order correction (relative error
+// of the estimate cubed, far below FP64 rounding): for normal, positive x of the pair passes,
+// where a division's scaling and special cases never arise.
+__device__ __forceinline__ double fast_rcp(double x) {
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = __builtin_fma(-x, y, 1.0);
+  return __builtin_fma(y, __builtin_fma(e, e, e), y);
+}
+__device__ __forceinline__ double fast_rsqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-x*y, y, 1.0);
+  return __builtin_fma(y*e, __builtin_fma(e, 0.375, 0.5), y);
 }
 
 // The command processor hands workgroup b to XCD b % 8, and each XCD has its own L2.

@@ -280,8 +280,8 @@ __device__ __forceinline__ void flush_chunk(uint32_t* nbr, int k, int i, size_t 
 // with the criterion widened to ext (1 + skin): one lane per particle walks the 3^D cells
 // (of side >= the widened support) around its own; lanes of a wavefront mostly share a
 // cell, so candidate reads are wave-uniform.  It records the positions and h^-1 the list
-// was built from.  k_neighbor_filter applies the exact criterion to the candidates every
-// step.  The candidates stay complete while no pair can have closed in from beyond the
+// was built from.  The filtering pass (k_density_dt) applies the exact criterion to the
+// candidates every step.  The candidates stay complete while no pair can have closed in from beyond the
 // widened radius: with D = max |x - xb| hb/ext and G = max hb/h^-1 over the run's nodes,
 // |rij(now)| <= max(Si, Sj)(now) implies |rij(built)| <= max(Si, Sj)(built) (G + 2D), so a
 // list is valid while G + 2D <= 1 + skin (the full update measures both after every step).
@@ -517,66 +517,6 @@ __global__ void __launch_bounds__(kBlock) k_candidates_merge(Fields f, const int
   if (ok) f.ccnt[me] = c0 + t;
 }
 
-// The exact criterion over each active node's candidates; writes the ELL neighbour list in
-// candidate order.  Periodic image codes are re-chosen from the current positions (nearest
-// copy); reflecting codes are kept.
-template <int D, int G>
-__global__ void __launch_bounds__(kBlock) k_neighbor_filter(Fields f, Geo g, Phys ph, int n, int* overflow) {
-  const int i = xcd_block()*blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double xi[D];
-#pragma unroll
-  for (int a = 0; a < D; ++a) xi[a] = f.x[a][i];
-  const double hi = f.hinv[i];
-  const size_t ld = (size_t)f.ld;
-  const int cap = f.cap;
-  const int nc = f.ccnt[i];
-  int count = 0;
-  uint32_t chunk[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int k0 = 0; k0 < nc; k0 += G) {
-    int js[G], codes[G];
-    ell_group<G>(f.cand, ld, k0, i, nc, js, codes);
-    double xj[G][D], hj[G];
-#pragma unroll
-    for (int u = 0; u < G; ++u) load_xh<D>(f.xh, js[u], xj[u], hj[u]);
-#pragma unroll
-    for (int u = 0; u < G; ++u) {
-      if (k0 + u >= nc) continue;
-      int code = codes[u];
-#pragma unroll
-      for (int a = 0; a < D; ++a) {
-        if ((g.permask >> a) & 1) {
-          const double half = 0.5*(g.xmax[a] - g.xmin[a]);
-          const double d = xj[u][a] - xi[a];
-          const int c = d > half ? 1 : (d < -half ? 2 : 0);
-          code = (code & ~(3 << (2*a))) | (c << (2*a));
-        }
-      }
-      if (js[u] == i && code == 0) continue;
-      if (code) image_pos<D>(g, code, xj[u]);
-      double e2i = 0.0, e2j = 0.0;
-#pragma unroll
-      for (int a = 0; a < D; ++a) {
-        const double rr = dsub(xi[a], xj[u][a]);
-        const double ei = dmul(hi, rr), ej = dmul(hj[u], rr);
-        e2i = a == 0 ? dmul(ei, ei) : dadd(e2i, dmul(ei, ei));
-        e2j = a == 0 ? dmul(ej, ej) : dadd(e2j, dmul(ej, ej));
-      }
-      if (e2i <= ph.ext2 || e2j <= ph.ext2) {
-        const uint32_t e = (uint32_t)js[u] | ((uint32_t)code << kImgShift);
-        const int s = count & 7;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) chunk[q] = s == q ? e : chunk[q];
-        ++count;
-        if (s == 7 && count <= cap) flush_chunk(f.nbr, count - 1, i, ld, chunk);
-      }
-    }
-  }
-  if ((count & 7) && count <= cap) flush_chunk(f.nbr, count - 1, i, ld, chunk);
-  f.cnt[i] = count;
-  if (count > cap) atomicMax(overflow, count);
-}
-
 // Per-run maximum of an order-preserving double key: a wavefront whose lanes share a run
 // reduces first, and an atomic is issued only when it would raise the running maximum
 // (most wavefronts do not: reading first keeps them off the contended word).
@@ -629,29 +569,70 @@ __global__ void __launch_bounds__(kBlock) k_remap_candidates(const uint32_t* src
 // -- node i receives m_j W(|Hj ri - Hj rj|, det Hj) -- fused with the GenericHydro::dt
 // vote (Physics/GenericHydro.cc:112-381): per-node limits on the new density and the
 // pairwise velocity-difference limit, min-reduced per run.
-// FILT: the pass walks the candidate lists instead, applies the neighbour criterion of
-// k_neighbor_filter to each candidate and writes the ELL neighbour list as it goes, so the
-// connectivity filter and the first pair pass of the step read the neighbours once.
+// FILT: the pass walks the candidate lists instead, applies the neighbour criterion to each
+// candidate and writes the ELL neighbour list as it goes, so the connectivity filter and the first
+// pair pass of the step read the neighbours once.  Without DENS and DT it only filters.
+//
+// Bound by the latency and the rate of the records' gathers (the L1 takes a 64-lane gather of 16
+// bytes at about 1.4 lanes per clock).  kNodeLanes lanes per node: KH 2-D 4096 mixed 70.7 -> 26.5 us,
+// 65536 FP64 80 -> 46 us, Sod 3-D 25k mixed 232 -> 92 us, Evrard 250k mixed 478 -> 417 us,
+// Taylor-Green 96^3 mixed 494 -> 449 us, 128^3 FP64 1137 -> 1077 us (one lane per node before).
 // ---------------------------------------------------------------------------
-template <int D, bool DENS, bool DT, typename R, int G, bool FILT, typename CP>
+//
+// The neighbour criterion: |Hi rij|^2 <= ext^2 or |Hj rij|^2 <= ext^2 in the reference's rounding.
+// (h r)^2 with each product and sum rounded is non-decreasing in h, so the test with the smaller
+// h^-1 decides both.  half[a]: half the box on a periodic axis (the nearest copy of j is taken),
+// otherwise larger than any separation; only a pair that needs an image pays for one.  Returns
+// whether j is a neighbour; code and rr = xi - xj are those of the image taken.
+template <int D>
+__device__ __forceinline__ bool neighbor_test(const Geo& g, double ext2, const double* half, const double* xi, double hi,
+                                              const double* xj, double hj, bool self, int& code, double* rr) {
+  code &= ~(((g.permask & 1) ? 3 : 0) | ((g.permask & 2) ? 12 : 0) | ((g.permask & 4) ? 48 : 0));
+  bool far = code != 0;
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    rr[a] = dsub(xi[a], xj[a]);
+    far |= fabs(rr[a]) > half[a];
+  }
+  if (far) {
+    double xk[D];
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+      xk[a] = xj[a];
+      if ((g.permask >> a) & 1) code |= (rr[a] < -half[a] ? 1 : (rr[a] > half[a] ? 2 : 0)) << (2*a);
+    }
+    image_pos<D>(g, code, xk);
+#pragma unroll
+    for (int a = 0; a < D; ++a) rr[a] = dsub(xi[a], xk[a]);
+  }
+  const double hm = fmin(hi, hj);
+  double e2 = 0.0;
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    const double e = dmul(hm, rr[a]);
+    e2 = a == 0 ? dmul(e, e) : dadd(e2, dmul(e, e));
+  }
+  return e2 <= ext2 && !(self && code == 0);
+}
+
+// U: entries in flight per lane.
+template <int D, bool DENS, bool DT, typename R, int U, bool FILT, typename CP>
 __device__ __forceinline__ void density_dt_node(const Fields& f, const Geo& g, const Phys& ph, const DevTable& tab,
                                                 CP coef, int n, Scalars* sc, int* overflow) {
-  const int i = xcd_block()*blockDim.x + threadIdx.x;
+  constexpr int L = kNodeLanes;
+  const int gl = xcd_block()*blockDim.x + threadIdx.x;
+  const int i = gl/L, sub = gl & (L - 1);
   double dtmin = 1.7976931348623157e308;
   const bool valid = i < n;
   int r = 0;
   if (valid) {
-    r = f.run[i];
-    double xi[D], vi[D];
+    if (DT) r = f.run[i];
+    double xi[D], vi[D], half[D];
 #pragma unroll
-    for (int a = 0; a < D; ++a) { xi[a] = f.x[a][i]; vi[a] = f.v[a][i]; }
-    const double nsi = f.ns[i];
-    double rho = 0.0;
-    if (DENS) {
-      const R hi = (R)f.hinv[i];
-      R w, gw, graw;
-      kernel_wgw_c<R>(coef, tab, (R)0, hdet_iso<D, R>(hi), w, gw, graw);   // self term W(|Hi ri - Hi ri|) = W(0)
-      rho = f.m[i]*(double)w;
+    for (int a = 0; a < D; ++a) {
+      xi[a] = f.x[a][i];
+      vi[a] = DT ? f.v[a][i] : 0.0;
+      half[a] = ((g.permask >> a) & 1) ? 0.5*(g.xmax[a] - g.xmin[a]) : 1.7976931348623157e308;
     }
     // pairwise limit min(ns_i, ns_j)/|v_ij| (GenericHydro.cc:196-210).  For isotropic H the
     // nodeScale is 1/(h^-1 nPerh) (lambda_max(h^-1 I) = h^-1; the reference's eigen-solver may
@@ -659,128 +640,117 @@ __device__ __forceinline__ void density_dt_node(const Fields& f, const Geo& g, c
     // max |v_ij|^2 max(h_i^-1, h_j^-1)^2, scaled by nPerh^2 at the end: no per-pair division
     // and no nodeScale read per neighbour
     const double hiD = f.hinv[i];
-    double vmaxh = 0.0;
+    double vmaxh = 0.0, rho0 = 0.0;
+    if (DENS) {
+      R w, gw, graw;
+      kernel_wgw_c<R>(coef, tab, (R)0, hdet_iso<D, R>((R)hiD), w, gw, graw);   // self term W(|Hi ri - Hi ri|) = W(0)
+      rho0 = f.m[i]*(double)w;
+    }
+    NodeSum<L, sizeof(R) == sizeof(float)> rhos(rho0, sub);
     const size_t ld = (size_t)f.ld;
     const int nn = FILT ? f.ccnt[i] : f.cnt[i];
-    const double hiF = FILT ? f.hinv[i] : 0.0;
     int count = 0;
-    uint32_t chunk[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int k0 = 0; k0 < nn; k0 += G) {
-      int js[G], codes[G];
-      ell_group<G>(FILT ? f.cand : f.nbr, ld, k0, i, nn, js, codes);
-      double xj[G][D], vj[G][D], hj[G], mj[G];
-      bool acc[G];
+    for (int k0 = 0; k0 < nn; k0 += U*L) {
+      int js[U], codes[U];
+      bool acc[U];
+      lane_entries<U, L>(FILT ? f.cand : f.nbr, ld, k0, sub, i, nn, js, codes, acc);
+      double xj[U][D], rr[U][D], vj[U][D], hj[U], mj[U];
 #pragma unroll
-      for (int u = 0; u < G; ++u) {
-        const int j = js[u];
-        load_xh<D>(f.xh, j, xj[u], hj[u]);
-        if (!FILT) load_vm<D>(f.vmr, j, vj[u], mj[u]);
-        acc[u] = !FILT && k0 + u < nn;
+      for (int u = 0; u < U; ++u) {
+        load_xh<D>(f.xh, js[u], xj[u], hj[u]);
+        mj[u] = 0.0;
+        if (!FILT) load_vm<D>(f.vmr, js[u], vj[u], mj[u]);
       }
-      if (FILT) {
-        // the exact neighbour criterion (k_neighbor_filter) on the group's candidates first;
-        // velocities and masses are then read for the accepted ones only
+      // the candidates are tested first; velocities and masses are then read for the accepted
+      // ones only.  Accepted entries keep the candidates' order: a lane's place is the count so
+      // far plus the accepted lanes of its quad below it
 #pragma unroll
-        for (int u = 0; u < G; ++u) {
-          if (k0 + u >= nn) continue;
-          int code = codes[u];
+      for (int u = 0; u < U; ++u) {
+        if (FILT) {
+          acc[u] = acc[u] && neighbor_test<D>(g, ph.ext2, half, xi, hiD, xj[u], hj[u], js[u] == i, codes[u], rr[u]);
+          const unsigned q = (unsigned)(__ballot(acc[u]) >> (threadIdx.x & 63 & ~(L - 1))) & ((1u << L) - 1u);
+          const int place = count + __popc(q & ((1u << sub) - 1u));
+          if (acc[u] && place < f.cap)
+            f.nbr[ell_at(place, i, ld)] = (uint32_t)js[u] | ((uint32_t)codes[u] << kImgShift);
+          count += __popc(q);
+        } else if (acc[u]) {
+          if (codes[u]) image_pos<D>(g, codes[u], xj[u]);
 #pragma unroll
-          for (int a = 0; a < D; ++a) {
-            if ((g.permask >> a) & 1) {
-              const double half = 0.5*(g.xmax[a] - g.xmin[a]);
-              const double d = xj[u][a] - xi[a];
-              const int c = d > half ? 1 : (d < -half ? 2 : 0);
-              code = (code & ~(3 << (2*a))) | (c << (2*a));
-            }
-          }
-          codes[u] = code;
-          if (js[u] == i && code == 0) continue;
-          if (code) image_pos<D>(g, code, xj[u]);
-          double e2i = 0.0, e2j = 0.0;
-#pragma unroll
-          for (int a = 0; a < D; ++a) {
-            const double rr = dsub(xi[a], xj[u][a]);
-            const double ei = dmul(hiF, rr), ej = dmul(hj[u], rr);
-            e2i = a == 0 ? dmul(ei, ei) : dadd(e2i, dmul(ei, ei));
-            e2j = a == 0 ? dmul(ej, ej) : dadd(e2j, dmul(ej, ej));
-          }
-          if (!(e2i <= ph.ext2 || e2j <= ph.ext2)) continue;
-          acc[u] = true;
-          const uint32_t e = (uint32_t)js[u] | ((uint32_t)code << kImgShift);
-          const int sl = count & 7;
-#pragma unroll
-          for (int q = 0; q < 8; ++q) chunk[q] = sl == q ? e : chunk[q];
-          ++count;
-          if (sl == 7 && count <= f.cap) flush_chunk(f.nbr, count - 1, i, ld, chunk);
+          for (int a = 0; a < D; ++a) rr[u][a] = xi[a] - xj[u][a];
         }
+      }
+      if (!DENS && !DT) continue;
+      if (FILT) {
 #pragma unroll
-        for (int u = 0; u < G; ++u)
+        for (int u = 0; u < U; ++u)
           if (acc[u]) load_vm<D>(f.vmr, js[u], vj[u], mj[u]);
       }
 #pragma unroll
-      for (int u = 0; u < G; ++u) {
-        if (!acc[u]) continue;
-        const int code = codes[u];
-        if (DENS) {
-          if (!FILT && code) image_pos<D>(g, code, xj[u]);
-          R s = (R)0;
-          if (sizeof(R) == sizeof(double)) {
+      for (int u = 0; u < U; ++u) {
+        R w = (R)0;
+        if (acc[u]) {
+          if (DENS) {
+            R d[D], gw, graw;
 #pragma unroll
-            for (int a = 0; a < D; ++a) { const double d = hj[u]*xi[a] - hj[u]*xj[u][a]; s += (R)(d*d); }
-          } else {
-#pragma unroll
-            for (int a = 0; a < D; ++a) { const R d = (R)hj[u]*(R)(xi[a] - xj[u][a]); s += d*d; }
+            for (int a = 0; a < D; ++a) d[a] = (R)hj[u]*(R)rr[u][a];
+            // (in mixed precision the package-level sum starts most chains from the second axis:
+            // the last FP32 bit it has always had)
+            const R s = !FILT && sizeof(R) == sizeof(float) && !(D == 3 && sub == 0) ? norm2_second<D>(d) : norm2<D>(d);
+            kernel_wgw_c<R>(coef, tab, sqrt(s), hdet_iso<D, R>((R)hj[u]), w, gw, graw);
           }
-          R w, gw, graw;
-          kernel_wgw_c<R>(coef, tab, sqrt(s), hdet_iso<D, R>((R)hj[u]), w, gw, graw);
-          rho += mj[u]*(double)w;
-        }
-        if (DT) {
-          double s = 0.0;
+          if (DT) {
+            double d[D];
 #pragma unroll
-          for (int a = 0; a < D; ++a) { const double d = vi[a] - refl_sign<D>(g, code, a)*vj[u][a]; s += d*d; }
-          const double hm = fmax(hiD, hj[u]);
-          vmaxh = fmax(vmaxh, s*(hm*hm));
+            for (int a = 0; a < D; ++a)
+              d[a] = vi[a] - (codes[u] ? refl_sign<D>(g, codes[u], a)*vj[u][a] : vj[u][a]);
+            const double hm = fmax(hiD, hj[u]);
+            vmaxh = fmax(vmaxh, norm2<D>(d)*(hm*hm));
+          }
         }
+        if (DENS) rhos.add(mj[u], w);
       }
     }
-    if (FILT) {
-      if ((count & 7) && count <= f.cap) flush_chunk(f.nbr, count - 1, i, ld, chunk);
+    if (FILT && sub == 0) {
       f.cnt[i] = count;
       if (count > f.cap) atomicMax(overflow, count);
     }
-    if (DENS) f.rho[i] = rho; else rho = f.rho[i];
+    double rho = rhos.total();
     if (DT) {
-      const double tiny = 2.220446049250313e-16;
-      // min(ns_i, ns_j)/max(tiny, |v_ij|) minimised over the pairs
-      const double vmax2 = vmaxh*(ph.nperh*ph.nperh);
-      if (vmax2 > 0.0) dtmin = fmin(dtmin, 1.0/sqrt(vmax2));
-      dtmin = fmin(dtmin, nsi/(f.cs[i] + tiny));
-      const double csq = sqrt(f.maxQ[i]/rho);
-      dtmin = fmin(dtmin, nsi/(csq + tiny));
-      double tr = 0.0;
+      vmaxh = fmax(vmaxh, quad_swap<0xB1>(vmaxh));
+      vmaxh = fmax(vmaxh, quad_swap<0x4E>(vmaxh));
+    }
+    if (sub == 0 && (DENS || DT)) {
+      if (DENS) f.rho[i] = rho; else rho = f.rho[i];
+      if (DT) {
+        const double nsi = f.ns[i];
+        const double tiny = 2.220446049250313e-16;
+        // min(ns_i, ns_j)/max(tiny, |v_ij|) minimised over the pairs
+        const double vmax2 = vmaxh*(ph.nperh*ph.nperh);
+        if (vmax2 > 0.0) dtmin = fmin(dtmin, 1.0/sqrt(vmax2));
+        dtmin = fmin(dtmin, nsi/(f.cs[i] + tiny));
+        const double csq = sqrt(f.maxQ[i]/rho);
+        dtmin = fmin(dtmin, nsi/(csq + tiny));
+        double tr = 0.0;
 #pragma unroll
-      for (int a = 0; a < D; ++a) tr += f.DvDx[(a*D + a)*(size_t)f.ld + i];
-      dtmin = fmin(dtmin, 1.0/(fabs(tr) + tiny));
-      double v2 = 0.0, a2 = 0.0;
+        for (int a = 0; a < D; ++a) tr += f.DvDx[(a*D + a)*(size_t)f.ld + i];
+        dtmin = fmin(dtmin, 1.0/(fabs(tr) + tiny));
+        double ai[D];
 #pragma unroll
-      for (int a = 0; a < D; ++a) { v2 += vi[a]*vi[a]; a2 += f.DvDt[a][i]*f.DvDt[a][i]; }
-      const double vmag = sqrt(v2);
-      dtmin = fmin(dtmin, 0.1*fmax(nsi/(vmag + tiny), vmag/(sqrt(a2) + tiny)));
-      if (ph.useVmagDt) dtmin = fmin(dtmin, nsi/(vmag + 1.0e-10));
+        for (int a = 0; a < D; ++a) ai[a] = f.DvDt[a][i];
+        const double vmag = sqrt(norm2_second<D>(vi));
+        dtmin = fmin(dtmin, 0.1*fmax(nsi/(vmag + tiny), vmag/(sqrt(norm2_second<D>(ai)) + tiny)));
+        if (ph.useVmagDt) dtmin = fmin(dtmin, nsi/(vmag + 1.0e-10));
+      }
     }
   }
-  if (DT) run_min(sc, r, dtmin, valid);
+  if (DT) run_min(sc, r, dtmin, valid && sub == 0);
 }
 
-// The kernel is a thin wrapper around the node body: compiled this way the filtering pass on
-// Taylor-Green 128^3 runs in 1.28 ms (FP64) / 1.24 ms (mixed) per step instead of 1.43 / 1.40 ms
-// with the body written in the kernel itself (same arithmetic, different register allocation).
-template <int D, bool DENS, bool DT, typename R, int G, bool FILT = false>
+template <int D, bool DENS, bool DT, typename R, int U, bool FILT = false>
 __global__ void __launch_bounds__(kBlock) k_density_dt(Fields f, Geo g, Phys ph, DevTable tab, int n, Scalars* sc,
                                                        int* overflow, int ldsTable) {
   with_table<R>(tab, DENS ? ldsTable : 0, [&](auto coef) {
-    density_dt_node<D, DENS, DT, R, G, FILT>(f, g, ph, tab, coef, n, sc, overflow);
+    density_dt_node<D, DENS, DT, R, U, FILT>(f, g, ph, tab, coef, n, sc, overflow);
   });
 }
 
@@ -900,39 +870,47 @@ __global__ void __launch_bounds__(kBlock) k_eos(Fields f, Phys ph, int n) {
 // also writes node i's midpoint record for the SPH pass (write_mid_record).  runMask
 // (optional): only nodes of runs with a non-zero entry are updated.
 // ---------------------------------------------------------------------------
-template <int D, typename R, bool MID, int G, typename CP>
+// L lanes per node, U entries in flight per lane; the sums are in list order for either L, so the
+// choice by particle count (kOmegaWideNodes) changes no bit.
+template <int D, typename R, bool MID, int U, int L, typename CP>
 __device__ __forceinline__ void omega_node(const Fields& f, const Geo& g, const DevTable& tab, CP coef, int n,
                                            const double* xh, double* omega, const int* runMask) {
-  const int i = xcd_block()*blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  const int gl = xcd_block()*blockDim.x + threadIdx.x;
+  const int i = gl/L, sub = gl & (L - 1);
+  if (i >= n) return;                       // the lanes of a node leave together
   if (runMask && !runMask[f.run[i]]) return;
   double xi[D], hid;
   load_xh<D>(xh, i, xi, hid);
   const R hi = (R)hid;
   const R hdeti = hdet_iso<D, R>(hi);
-  double wsum = 0.0, gsum = 0.0;
+  NodeSum<L, true> ws(0.0, sub), gs(0.0, sub);
   const int nn = f.cnt[i];
-  for (int k0 = 0; k0 < nn; k0 += G) {
-    int js[G], codes[G];
-    ell_group<G>(f.nbr, (size_t)f.ld, k0, i, nn, js, codes);
-    double xj[G][D], hjunk[G];
+  for (int k0 = 0; k0 < nn; k0 += U*L) {
+    int js[U], codes[U];
+    bool in[U];
+    lane_entries<U, L>(f.nbr, (size_t)f.ld, k0, sub, i, nn, js, codes, in);
+    double xj[U][D], hjunk[U];
 #pragma unroll
-    for (int u = 0; u < G; ++u) load_xh<D>(xh, js[u], xj[u], hjunk[u]);
+    for (int u = 0; u < U; ++u) load_xh<D>(xh, js[u], xj[u], hjunk[u]);
 #pragma unroll
-    for (int u = 0; u < G; ++u) {
-      if (k0 + u < nn) {
+    for (int u = 0; u < U; ++u) {
+      R w = (R)0, t = (R)0;
+      if (in[u]) {
         if (codes[u]) image_pos<D>(g, codes[u], xj[u]);
-        R s = (R)0;
+        R d[D], gw, graw;
 #pragma unroll
-        for (int a = 0; a < D; ++a) { const R rr = hi*(R)(xi[a] - xj[u][a]); s += rr*rr; }
-        const R eta = sqrt(s);
-        R w, gw, graw;
+        for (int a = 0; a < D; ++a) d[a] = hi*(R)(xi[a] - xj[u][a]);
+        const R eta = sqrt(norm2<D>(d));
         kernel_wgw_c<R>(coef, tab, eta, hdeti, w, gw, graw);
-        wsum += (double)w;
-        gsum += (double)(eta*gw);
+        t = rounded_product(eta, gw);
       }
+      ws.add(w);
+      gs.add(t);
     }
   }
+  double wsum = ws.total();
+  const double gsum = gs.total();
+  if (sub) return;
   double om;
   if (nn == 0) {
     om = 1.0;
@@ -943,10 +921,11 @@ __device__ __forceinline__ void omega_node(const Fields& f, const Geo& g, const 
   omega[i] = om;
   if (MID) write_mid_record<D>(f, i, om);
 }
-template <int D, typename R, bool MID, int G = kGroup>
+template <int D, typename R, bool MID, int U, int L>
 __global__ void __launch_bounds__(kBlock) k_omega(Fields f, Geo g, DevTable tab, int n, const double* xh,
                                                   double* omega, const int* runMask, int ldsTable) {
-  with_table<R>(tab, ldsTable, [&](auto coef) { omega_node<D, R, MID, G>(f, g, tab, coef, n, xh, omega, runMask); });
+  with_table<R>(tab, ldsTable,
+                [&](auto coef) { omega_node<D, R, MID, U, L>(f, g, tab, coef, n, xh, omega, runMask); });
 }
 
 // SynchronousRK2 with TreeGravity as the only package (Integrator/SynchronousRK2.cc:40-135): the

@@ -446,9 +446,16 @@ __global__ void __launch_bounds__(kBlock, 3) k_sph(Fields f, Geo g, Phys ph, Dev
 // half-step velocity, DepsDt, m and the evaluation's position).  The pairwise acceleration is
 // re-formed as C*r with r computed from the evaluation's positions by the SPH pass's own
 // operations, so it is the same bits the SPH pass summed into DvDt.
+//
+// FP64 forms a pair's share from node i's own side: with q = (v_o - v_i)^{1/2} . (C r) it is
+// w (-m_o q), w = w_i/(w_i + w_o), w_x = max(eps, DepsDt_x sgn(-m q)).  q has the same bits from
+// both sides (both factors change sign exactly), so both sides take the same branch and the two
+// shares add up to the pair's work; one reciprocal instead of two divisions.  Mixed precision keeps
+// the canonical (a, b) form.  Every lane of the quad returns the node's rate.
 // ---------------------------------------------------------------------------
-template <int D, typename R, int G>
-__device__ __forceinline__ double compatible_rate(const Fields& f, const Geo& g, int i) {
+template <int D, typename R, int U>
+__device__ __forceinline__ double compatible_rate(const Fields& f, const Geo& g, int i, int sub) {
+  constexpr int L = kNodeLanes;
   const size_t ld = (size_t)f.ld;
   const R* pdd = (const R*)f.pdd;       // pair coefficients in the pair arithmetic; the partition is FP64
   const double ms = f.m[i];
@@ -465,15 +472,16 @@ __device__ __forceinline__ double compatible_rate(const Fields& f, const Geo& g,
   }
   const double de0s = f.DepsDt[i];
   const double epsm = 2.220446049250313e-16;
-  double du = 0.0;
+  NodeSum<L, sizeof(R) == sizeof(float)> du(0.0, sub);
   const int nn = f.cnt[i];
-  for (int k0 = 0; k0 < nn; k0 += G) {
-    int js[G], codes[G];
-    ell_group<G>(f.nbr, ld, k0, i, nn, js, codes);
-    double vo[G][D], xo[G][D], mo[G], deo[G];
-    R C[G];
+  for (int k0 = 0; k0 < nn; k0 += U*L) {
+    int js[U], codes[U];
+    bool in[U];
+    lane_entries<U, L>(f.nbr, ld, k0, sub, i, nn, js, codes, in);
+    double vo[U][D], xo[U][D], mo[U], deo[U];
+    R C[U];
 #pragma unroll
-    for (int u = 0; u < G; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int j = js[u];
       const double2 a = PV[4*(size_t)j], b = PV[4*(size_t)j + 1], c = PV[4*(size_t)j + 2], d = PV[4*(size_t)j + 3];
       vo[u][0] = a.x;
@@ -484,32 +492,50 @@ __device__ __forceinline__ double compatible_rate(const Fields& f, const Geo& g,
       xo[u][0] = c.y;
       if (D >= 2) xo[u][1 % D] = d.x;
       if (D >= 3) xo[u][2 % D] = d.y;
-      C[u] = pdd[(size_t)(k0 + u)*ld + i];
+      C[u] = pdd[(size_t)(in[u] ? k0 + u*L + sub : 0)*ld + i];
     }
 #pragma unroll
-    for (int u = 0; u < G; ++u) {
-      if (k0 + u >= nn) continue;
-      const int j = js[u], code = codes[u];
-      const bool aFirst = code != 0 || i < j;
-      if (code) image_pos<D>(g, code, xo[u]);
-      // canonical: pacc_ab = (-m_b) C r_ab ; du_ab = (v_b^{1/2} - v_a^{1/2}) . pacc_ab
-      const double mb = aFirst ? mo[u] : ms, ma = aFirst ? ms : mo[u];
-      double duab = 0.0;
+    for (int u = 0; u < U; ++u) {
+      double t = 0.0;
+      if (in[u]) {
+        const int j = js[u], code = codes[u];
+        if (code) {
+          image_pos<D>(g, code, xo[u]);
 #pragma unroll
-      for (int c = 0; c < D; ++c) {
-        const double dd = (double)(C[u]*(R)(xs[c] - xo[u][c]));     // the SPH pass's C*r, this lane's side
-        const double v12o = refl_sign<D>(g, code, c)*vo[u][c];
-        const double va = aFirst ? v12s[c] : v12o, vb = aFirst ? v12o : v12s[c];
-        const double ddc = aFirst ? dd : -dd;
-        duab += (vb - va)*((-mb)*ddc);
+          for (int c = 0; c < D; ++c) vo[u][c] *= refl_sign<D>(g, code, c);
+        }
+        if (sizeof(R) == sizeof(double)) {
+          double q = 0.0;
+#pragma unroll
+          for (int c = 0; c < D; ++c)
+            q += (vo[u][c] - v12s[c])*(double)(C[u]*(R)(xs[c] - xo[u][c]));     // the SPH pass's C*r
+          const double e = -mo[u]*q;
+          const double sgn = e < 0.0 ? -1.0 : 1.0;
+          const double wi = fmax(epsm, de0s*sgn), wo = fmax(epsm, deo[u]*sgn);
+          t = wi*fast_rcp(wi + wo)*e;
+        } else {
+          // canonical: pacc_ab = (-m_b) C r_ab ; du_ab = (v_b^{1/2} - v_a^{1/2}) . pacc_ab
+          const bool aFirst = code != 0 || i < j;
+          const double mb = aFirst ? mo[u] : ms, ma = aFirst ? ms : mo[u];
+          double duab = 0.0;
+#pragma unroll
+          for (int c = 0; c < D; ++c) {
+            const double dd = (double)(C[u]*(R)(xs[c] - xo[u][c]));     // the SPH pass's C*r, this lane's side
+            const double va = aFirst ? v12s[c] : vo[u][c], vb = aFirst ? vo[u][c] : v12s[c];
+            const double ddc = aFirst ? dd : -dd;
+            const double ac = (-mb)*ddc;
+            duab = c == 0 ? rounded_product(vb - va, ac) : fused(vb - va, ac, duab);
+          }
+          const double sgn = duab < 0.0 ? -1.0 : 1.0;
+          const double wa = fmax(epsm, (aFirst ? de0s : deo[u])*sgn), wb = fmax(epsm, (aFirst ? deo[u] : de0s)*sgn);
+          const double w = wa/(wa + wb);
+          t = aFirst ? w*duab : (1.0 - w)*duab*ma/mb;
+        }
       }
-      const double sgn = duab < 0.0 ? -1.0 : 1.0;
-      const double wa = fmax(epsm, (aFirst ? de0s : deo[u])*sgn), wb = fmax(epsm, (aFirst ? deo[u] : de0s)*sgn);
-      const double w = wa/(wa + wb);
-      du += aFirst ? w*duab : (1.0 - w)*duab*ma/mb;
+      du.add(t);
     }
   }
-  return du;
+  return du.total();
 }
 
 // ---------------------------------------------------------------------------
@@ -520,16 +546,18 @@ __device__ __forceinline__ double compatible_rate(const Fields& f, const Geo& g,
 // grown since the candidate list was built (see k_candidates).  ENERGY_ONLY: the
 // package-level policy call (eps only).
 // ---------------------------------------------------------------------------
-template <int D, bool ENERGY_ONLY, typename R, int G>
+template <int D, bool ENERGY_ONLY, typename R, int U>
 __global__ void __launch_bounds__(kBlock) k_full_update(Fields f, Geo g, Phys ph, Scalars* sc, double multiplier,
                                                         int n) {
-  const int i = xcd_block()*blockDim.x + threadIdx.x;
-  const bool valid = i < n;
+  const int gl = xcd_block()*blockDim.x + threadIdx.x;
+  const int i = gl/kNodeLanes, sub = gl & (kNodeLanes - 1);
+  const bool valid = i < n && sub == 0;
   int skr = 0;                       // candidate-list check (k_skin_check's measure, fused)
   double skd = 0.0, skg = 0.0;
+  double du = 0.0;
+  if (i < n) du = compatible_rate<D, R, U>(f, g, i, sub);
   if (valid) {
   const double dt = ENERGY_ONLY ? multiplier : sc[f.run[i]].dt;
-  const double du = compatible_rate<D, R, G>(f, g, i);
   const double eps1 = f.eps[i] + du*dt;
   f.eps[i] = eps1;
   if (ENERGY_ONLY) return;
@@ -557,9 +585,9 @@ __global__ void __launch_bounds__(kBlock) k_full_update(Fields f, Geo g, Phys ph
   for (int a = 0; a < D; ++a) {
     double d = x1[a] - f.xb[a][i];
     if ((g.permask >> a) & 1) {
-      const double L = g.xmax[a] - g.xmin[a];
+      const double box = g.xmax[a] - g.xmin[a];
       d = fabs(d);
-      d = fmin(d, fabs(L - d));
+      d = fmin(d, fabs(box - d));
     }
     d2 += d*d;
   }
@@ -580,12 +608,14 @@ __global__ void __launch_bounds__(kBlock) k_full_update(Fields f, Geo g, Phys ph
 // the full policies, not timeAdvanceOnly -- the compatible energy partition of the start-of-step
 // pair accelerations, the increments, H replaced by the ideal H (ReplaceBoundedState) and the
 // EOS -- written to the midpoint arrays and position record; the start-of-step state stays.
-template <int D, typename R, int G>
+template <int D, typename R, int U>
 __global__ void __launch_bounds__(kBlock) k_half_update(Fields f, Geo g, Phys ph, const Scalars* sc, int n) {
-  const int i = xcd_block()*blockDim.x + threadIdx.x;
+  const int gl = xcd_block()*blockDim.x + threadIdx.x;
+  const int i = gl/kNodeLanes, sub = gl & (kNodeLanes - 1);
   if (i >= n) return;
+  const double du = compatible_rate<D, R, U>(f, g, i, sub);
+  if (sub) return;
   const double hdt = sc[f.run[i]].hdt;
-  const double du = compatible_rate<D, R, G>(f, g, i);
   const double eps = f.eps[i] + du*hdt;
   double xm[3] = {0.0, 0.0, 0.0};
 #pragma unroll
