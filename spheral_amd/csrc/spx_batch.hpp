@@ -758,7 +758,7 @@ class Batch {
       for (int a = 0; a < 3; ++a) { gr.origin[a] = 0.0; gr.inv_cell[a] = 0.0; gr.nc[a] = 1; }
       gr.cellBase = (int)base;
       gr.hinvMin = 0.0;
-      gr.ext2c = 0.0;
+      gr.ext2c = gr.extc = 0.0;
       gr.support = 0.0;
       gr.levels = 1;
       if (runs[r].state != RUN_ACTIVE || !hbuild[r]) continue;
@@ -767,6 +767,7 @@ class Batch {
       gr.hinvMin = hinvMin;
       const double extc = cfg.neighbor_extent*(1.0 + runs[r].skin);
       gr.ext2c = extc*extc;
+      gr.extc = extc;
       const double support = extc/hinvMin*(1.0 + 1.0e-9);
       gr.support = support;
       // where h varies by 2x or more: with open boundaries, cell levels down to the smallest
@@ -1119,11 +1120,11 @@ class Batch {
         HIP_CHECK(hipMemsetAsync(tcnt, 0, nActive*sizeof(int), stream));
         launchD([&](auto d) {
           constexpr int DD = decltype(d)::value;
-          hipLaunchKernelGGL(k_candidates<DD>, dim3(xcd_grid(nBuild, kBlock)), dim3(kBlock), 0, stream, f, geo,
+          hipLaunchKernelGGL(k_candidates<DD>, dim3(xcd_grid(nBuild*kSearchLanes, kBlock)), dim3(kBlock), 0, stream, f, geo,
                              (const RunGrid*)dgrids, (const int2*)dseg, nseg, (int)nBuild, (const int*)cellStart,
                              (const int*)cellEnd, tlist, tcnt, tcap, dOverflow);
         });
-        hipLaunchKernelGGL(k_candidates_merge, dim3(nblocks(nBuild)), dim3(kBlock), 0, stream, f, (const int2*)dseg,
+        hipLaunchKernelGGL(k_candidates_merge, dim3(xcd_grid(nBuild*kMergeLanes, kBlock)), dim3(kBlock), 0, stream, f, (const int2*)dseg,
                            nseg, (int)nBuild, (const uint32_t*)tlist, (const int*)tcnt, tcap, dOverflow);
         HIP_CHECK(hipGetLastError());
         download(hOverflow, dOverflow, 2*sizeof(int));

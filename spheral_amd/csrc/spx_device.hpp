@@ -235,6 +235,7 @@ struct RunGrid {
   double inv_cell[3];  // of the finest level when levels > 1
   double hinvMin;      // smallest h^-1 of the run's nodes: bounds every node's support radius
   double ext2c;        // candidate-list criterion: ext^2 (1 + skin)^2
+  double extc;         // ext (1 + skin)
   double support;      // the largest widened support radius
   int nc[3];           // cells per axis (of the finest level when levels > 1)
   int cellBase;        // first cell of the run's table (of level 0 when levels > 1)

@@ -263,13 +263,6 @@ __device__ __forceinline__ void load_vm(const double* vm, int j, double* v, doub
   m = b.y;
 }
 
-// Store the 8-entry chunk holding entry k of slot i (two 16-byte stores).
-__device__ __forceinline__ void flush_chunk(uint32_t* nbr, int k, int i, size_t ld, const uint32_t* c) {
-  uint4* dst = reinterpret_cast<uint4*>(nbr + ell_at(k & ~7, i, ld));
-  dst[0] = make_uint4(c[0], c[1], c[2], c[3]);
-  dst[1] = make_uint4(c[4], c[5], c[6], c[7]);
-}
-
 // ---------------------------------------------------------------------------
 // ConnectivityMap::computeConnectivity (Neighbor/ConnectivityMap.cc:905-947): j is a
 // neighbour of i iff |Hi rij|^2 <= ext^2 or |Hj rij|^2 <= ext^2, i != j (an image of i
@@ -277,10 +270,8 @@ __device__ __forceinline__ void flush_chunk(uint32_t* nbr, int k, int i, size_t 
 // rounding (no contraction) so the sets match exactly.
 //
 // Two stages.  k_candidates builds, for the runs whose list is stale, a candidate list
-// with the criterion widened to ext (1 + skin): one lane per particle walks the 3^D cells
-// (of side >= the widened support) around its own; lanes of a wavefront mostly share a
-// cell, so candidate reads are wave-uniform.  It records the positions and h^-1 the list
-// was built from.  The filtering pass (k_density_dt) applies the exact criterion to the
+// with the criterion widened to ext (1 + skin): a few lanes per particle walk the cells its
+// widened support reaches.  It records the positions and h^-1 the list was built from.  The filtering pass (k_density_dt) applies the exact criterion to the
 // candidates every step.  The candidates stay complete while no pair can have closed in from beyond the
 // widened radius: with D = max |x - xb| hb/ext and G = max hb/h^-1 over the run's nodes,
 // |rij(now)| <= max(Si, Sj)(now) implies |rij(built)| <= max(Si, Sj)(built) (G + 2D), so a
@@ -338,183 +329,251 @@ __device__ __forceinline__ int build_pos(const int2* seg, int nseg, int k) {
 // Every node collects each j within its own widened support; where j's support does not reach
 // i, i hands j the mirrored entry (tlist, merged by k_candidates_merge).  Together each list
 // holds exactly the j with |Hi rij| or |Hj rij| within the widened extent.
+//
+// kSearchLanes lanes per node.  The stencil's cells are taken kSearchCells at a time, two consecutive
+// ones per lane; a scan of their particle counts lays their particles out as one list (in cell order,
+// then slot order, as one lane alone would meet them), which the lanes test kSearchLanes at a time,
+// each finding its particle's cell by bisection of the scan in LDS.  Accepted entries keep the list's
+// order by a ballot, so the candidate lists are the same for any lane count.  One lane per node left
+// small runs with a few blocks walking up to a thousand candidates in turn, and where h varies most
+// cells of a node's level hold no or few particles.  Per rebuild, one lane -> 16: KH 2-D 4096 245 ->
+// 32 us, 65536 253 -> 91, Sod 3-D 25k 1879 -> 256, Evrard 250k 3030 -> 1599; Taylor-Green 128^3 3003 ->
+// 3041 (instruction issue: 8 waves per SIMD and the test's ~80 instructions per candidate; at 79
+// VGPRs and 6 waves 3167).  8 lanes: Sod 451, Evrard 2494, Taylor-Green 4245.
+constexpr int kSearchLanes = 16, kSearchCells = 32;
 template <int D>
-__global__ void __launch_bounds__(kBlock) k_candidates(Fields f, Geo g, const RunGrid* grids, const int2* seg, int nseg,
+__global__ void __launch_bounds__(kBlock, 8) k_candidates(Fields f, Geo g, const RunGrid* grids, const int2* seg, int nseg,
                                                        int nBuild, const int* cstart, const int* cend, uint32_t* tlist,
                                                        int* tcnt, int tcap, int* overflow) {
-  const int k = xcd_block()*blockDim.x + threadIdx.x;
-  if (k >= nBuild) return;
+  constexpr int C = kSearchLanes, Q = kSearchCells/C;
+  __shared__ int sEnd[kBlock/C][kSearchCells];         // particles up to and including the cell
+  __shared__ uint32_t sFirst[kBlock/C][kSearchCells];  // the cell's first slot minus those before it, image code on top
+  const int gl = xcd_block()*blockDim.x + threadIdx.x;
+  const int k = gl/C, sub = gl & (C - 1), grp = threadIdx.x/C;
+  if (k >= nBuild) return;                             // a node's lanes leave together
   const int sg = seg_of(seg, nseg, k);
   const int i = seg[sg].x + (k - seg[sg].y);
-  const int r = f.run[i];
-  const RunGrid gr = grids[r];
+  const RunGrid& gr = grids[f.run[i]];
   double xi[D];
   int ci[3] = {0, 0, 0};
 #pragma unroll
   for (int a = 0; a < D; ++a) {
     xi[a] = f.x[a][i];
     ci[a] = cell_coord<D>(gr, a, xi[a]);
-    f.xb[a][i] = xi[a];
+    if (sub == 0) f.xb[a][i] = xi[a];
   }
   const double hi = f.hinv[i];
-  f.hb[i] = hi;
+  if (sub == 0) f.hb[i] = hi;
   const double ext2c = gr.ext2c;
-  const double reach = sqrt(ext2c)/hi;
+  const double reach = gr.extc*fast_rcp(hi);
   // FP32 distance pre-filter with a 1e-4 relative margin (far above its own rounding): only the
   // FP64 criterion decides membership
-  const float reach2 = (float)(ext2c/(hi*hi)*(1.0 + 1.0e-4));
+  const float reach2 = (float)(reach*reach*(1.0 + 1.0e-4));
   const size_t ld = (size_t)f.ld;
   const int cap = f.ccap;
-  int count = 0;
-  uint32_t chunk[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  auto visit = [&](int j, int code) {
-    if (j == i && code == 0) return;
-    double xj[D];
-#pragma unroll
-    for (int a = 0; a < D; ++a) xj[a] = f.x[a][j];
-    if (code) image_pos<D>(g, code, xj);
-    float r2 = 0.0f;
-#pragma unroll
-    for (int a = 0; a < D; ++a) { const float d = (float)(xi[a] - xj[a]); r2 += d*d; }
-    if (r2 > reach2) return;
-    const double hj = f.hinv[j];
-    double e2i = 0.0, e2j = 0.0;
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-      const double rr = dsub(xi[a], xj[a]);
-      const double ei = dmul(hi, rr), ej = dmul(hj, rr);
-      e2i = a == 0 ? dmul(ei, ei) : dadd(e2i, dmul(ei, ei));
-      e2j = a == 0 ? dmul(ej, ej) : dadd(e2j, dmul(ej, ej));
-    }
-    if (!(e2i <= ext2c)) return;
-    // write-combine 8 entries in registers, flush them as one 32-byte chunk
-    const uint32_t e = (uint32_t)j | ((uint32_t)code << kImgShift);
-    const int s = count & 7;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) chunk[u] = s == u ? e : chunk[u];
-    ++count;
-    if (s == 7 && count <= cap) flush_chunk(f.cand, count - 1, i, ld, chunk);
-    if (!(e2j <= ext2c)) {
-      // j's own support does not reach i: j receives the pair from here
-      const int slot = atomicAdd(&tcnt[j], 1);
-      if (slot < tcap) tlist[ell_at(slot, j, ld)] = (uint32_t)i | ((uint32_t)inverse_image(g, code) << kImgShift);
-    }
-  };
-  if (gr.levels > 1) {
-    // the node's level: the finest l with support/2^l >= its reach; those cells are at least
-    // support/2^(l+2) wide, a quarter of the reach or more, so it scans 3 to 9 cells per axis
-    int lv = 0;
+  // the stencil: the cells of the node's level that its own widened support reaches (with one grid,
+  // at least the 3^D cells around its own)
+  const bool levels = gr.levels > 1;
+  int lv = 0, cl[3] = {0, 0, 0}, ncl[3] = {1, 1, 1}, kw[3] = {0, 0, 0};
+  if (levels) {
+    // the finest l with support/2^l >= its reach; those cells are at least support/2^(l+2) wide, a
+    // quarter of the reach or more, so it scans 3 to 9 cells per axis
     double w = 0.5*gr.support;
     while (lv + 1 < gr.levels && w >= reach) { ++lv; w *= 0.5; }
     const int sh = gr.levels - 1 - lv;
-    int cl[3] = {0, 0, 0}, ncl[3] = {1, 1, 1}, kl[3] = {0, 0, 0};
     level_cells<D>(gr, lv, ncl);
 #pragma unroll
     for (int a = 0; a < D; ++a) {
       cl[a] = ci[a] >> sh;
-      kl[a] = max(1, (int)ceil(reach*gr.inv_cell[a]/(double)(1 << sh)*(1.0 + 1.0e-12)));
+      kw[a] = max(1, (int)ceil(reach*gr.inv_cell[a]/(double)(1 << sh)*(1.0 + 1.0e-12)));
     }
-    const int kz = D >= 3 ? kl[2] : 0, ky = D >= 2 ? kl[1] : 0;
-    for (int dz = -kz; dz <= kz; ++dz)
-      for (int dy = -ky; dy <= ky; ++dy)
-        for (int dx = -kl[0]; dx <= kl[0]; ++dx) {
-          const int off[3] = {dx, dy, dz};
-          int cc[3] = {0, 0, 0};
-          bool skip = false;
-#pragma unroll
-          for (int a = 0; a < D; ++a) {
-            cc[a] = cl[a] + off[a];
-            skip |= cc[a] < 0 || cc[a] >= ncl[a];
-          }
-          if (skip) continue;
-          const int cell = lin_level_cell<D>(gr, lv, ncl, cc);
-          const int q1 = cend[cell];
-          for (int j = cstart[cell]; j < q1; ++j) visit(j, 0);
-        }
   } else {
-    // stencil half-width per axis: the cells the node's own widened support reaches
-    int kw[3] = {0, 0, 0};
 #pragma unroll
-    for (int a = 0; a < D; ++a) kw[a] = max(1, (int)ceil(reach*gr.inv_cell[a]*(1.0 + 1.0e-12)));
-    const int kz = D >= 3 ? kw[2] : 0, ky = D >= 2 ? kw[1] : 0;
-    for (int dz = -kz; dz <= kz; ++dz)
-      for (int dy = -ky; dy <= ky; ++dy)
-        for (int dx = -kw[0]; dx <= kw[0]; ++dx) {
-          const int off[3] = {dx, dy, dz};
-          int cc[3] = {0, 0, 0};
-          int code = 0;
-          bool skip = false;
-#pragma unroll
-          for (int a = 0; a < D; ++a) {
-            int c = ci[a] + off[a];
-            const bool per = (g.permask >> a) & 1;
-            if (c < 0) {
-              if (per) { c += gr.nc[a]; code |= 1 << (2*a); }
-              else if ((g.reflmask >> (2*a)) & 1) { c = -c - 1; code |= 1 << (2*a); skip |= c >= gr.nc[a]; }
-              else skip = true;
-            } else if (c >= gr.nc[a]) {
-              if (per) { c -= gr.nc[a]; code |= 2 << (2*a); }
-              else if ((g.reflmask >> (2*a + 1)) & 1) { c = 2*gr.nc[a] - 1 - c; code |= 2 << (2*a); skip |= c < 0; }
-              else skip = true;
-            }
-            cc[a] = c;
-          }
-          if (skip) continue;
-          const int cell = lin_cell<D>(gr, cc);
-          const int q1 = cend[cell];
-          for (int j = cstart[cell]; j < q1; ++j) visit(j, code);
-        }
+    for (int a = 0; a < D; ++a) {
+      cl[a] = ci[a];
+      ncl[a] = gr.nc[a];
+      kw[a] = max(1, (int)ceil(reach*gr.inv_cell[a]*(1.0 + 1.0e-12)));
+    }
   }
-  if ((count & 7) && count <= cap) flush_chunk(f.cand, count - 1, i, ld, chunk);
-  f.ccnt[i] = count;
-  if (count > cap) atomicMax(overflow, count);
+  const int wx = 2*kw[0] + 1, wy = D >= 2 ? 2*kw[1] + 1 : 1, wz = D >= 3 ? 2*kw[2] + 1 : 1;
+  const int ncells = wx*wy*wz;
+  bool inside = true;                                  // no cell of the stencil leaves the grid
+#pragma unroll
+  for (int a = 0; a < D; ++a) inside &= cl[a] >= kw[a] && cl[a] + kw[a] < ncl[a];
+  // the particle range and image code of the cell at offset (dx, dy, dz); false: nothing there
+  auto cell_range = [&](const int* off, int& first, int& last, int& code) -> bool {
+    int cc[3] = {0, 0, 0};
+    code = 0;
+#pragma unroll
+    for (int a = 0; a < D; ++a) cc[a] = cl[a] + off[a];
+    if (!inside) {
+      bool skip = false;
+#pragma unroll
+      for (int a = 0; a < D; ++a) {
+        const bool per = !levels && ((g.permask >> a) & 1);
+        const int refl = levels ? 0 : (g.reflmask >> (2*a)) & 3;
+        int c = cc[a];
+        if (c < 0) {
+          if (per) { c += ncl[a]; code |= 1 << (2*a); }
+          else if (refl & 1) { c = -c - 1; code |= 1 << (2*a); skip |= c >= ncl[a]; }
+          else skip = true;
+        } else if (c >= ncl[a]) {
+          if (per) { c -= ncl[a]; code |= 2 << (2*a); }
+          else if (refl & 2) { c = 2*ncl[a] - 1 - c; code |= 2 << (2*a); skip |= c < 0; }
+          else skip = true;
+        }
+        cc[a] = c;
+      }
+      if (skip) return false;
+    }
+    const int cell = levels ? lin_level_cell<D>(gr, lv, ncl, cc) : lin_cell<D>(gr, cc);
+    first = cstart[cell];
+    last = cend[cell];
+    return last > first;
+  };
+  int count = 0;
+  for (int b0 = 0; b0 < ncells; b0 += kSearchCells) {
+    // this lane's Q consecutive cells
+    int len[Q], first[Q], codes[Q], sum = 0;
+    int c = b0 + Q*sub;
+    int off[3] = {c % wx, 0, 0};
+    { const int t = c/wx; off[1] = t % wy; off[2] = t/wy; }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      len[q] = 0;
+      first[q] = codes[q] = 0;
+      if (c + q < ncells) {
+        const int o[3] = {off[0] - kw[0], off[1] - kw[1], off[2] - kw[2]};
+        int last = 0;
+        if (cell_range(o, first[q], last, codes[q])) len[q] = last - first[q];
+      }
+      sum += len[q];
+      if (++off[0] == wx) { off[0] = 0; if (++off[1] == wy) { off[1] = 0; ++off[2]; } }
+    }
+    int before = sum;
+#pragma unroll
+    for (int d = 1; d < C; d <<= 1) {
+      const int o = __shfl_up(before, d, C);
+      if (sub >= d) before += o;
+    }
+    const int total = __shfl(before, C - 1, C);
+    before -= sum;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      sFirst[grp][Q*sub + q] = ((uint32_t)(first[q] - before) & kIdxMask) | ((uint32_t)codes[q] << kImgShift);
+      before += len[q];
+      sEnd[grp][Q*sub + q] = before;
+    }
+    // only this node's lanes, of one wavefront, read what they wrote
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (int t0 = 0; t0 < total; t0 += C) {
+      const int t = t0 + sub;
+      bool acc = t < total;
+      int j = i, code = 0;
+      if (acc) {
+        int m = 0;                                     // the first cell whose count exceeds t
+#pragma unroll
+        for (int s = kSearchCells/2; s > 0; s >>= 1) m += sEnd[grp][m + s - 1] <= t ? s : 0;
+        const uint32_t e = sFirst[grp][m];
+        j = (int)((e + (uint32_t)t) & kIdxMask);
+        code = (int)(e >> kImgShift);
+        acc = !(j == i && code == 0);
+      }
+      double rr[D];
+      if (acc) {
+        double xj[D];
+#pragma unroll
+        for (int a = 0; a < D; ++a) xj[a] = f.x[a][j];
+        if (code) image_pos<D>(g, code, xj);
+        float r2 = 0.0f;
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+          rr[a] = dsub(xi[a], xj[a]);
+          const float d = (float)rr[a];
+          r2 += d*d;
+        }
+        acc = r2 <= reach2;
+      }
+      if (acc) {
+        double e[D];
+#pragma unroll
+        for (int a = 0; a < D; ++a) e[a] = dmul(hi, rr[a]);
+        acc = norm2<D>(e) <= ext2c;
+        if (acc) {
+          const double hj = f.hinv[j];
+#pragma unroll
+          for (int a = 0; a < D; ++a) e[a] = dmul(hj, rr[a]);
+          if (!(norm2<D>(e) <= ext2c)) {
+            // j's own support does not reach i: j receives the pair from here
+            const int slot = atomicAdd(&tcnt[j], 1);
+            if (slot < tcap) tlist[ell_at(slot, j, ld)] = (uint32_t)i | ((uint32_t)inverse_image(g, code) << kImgShift);
+          }
+        }
+      }
+      const unsigned q = (unsigned)(__ballot(acc) >> (threadIdx.x & 63 & ~(C - 1))) & ((1u << C) - 1u);
+      const int place = count + __popc(q & ((1u << sub) - 1u));
+      if (acc && place < cap) f.cand[ell_at(place, i, ld)] = (uint32_t)j | ((uint32_t)code << kImgShift);
+      count += __popc(q);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  if (sub == 0) {
+    f.ccnt[i] = count;
+    if (count > cap) atomicMax(overflow, count);
+  }
+}
+
+// Number of the row's 16 lanes whose v is below e (row rotations by DPP).
+template <int S = 15>
+__device__ __forceinline__ int row_below(uint32_t v, uint32_t e) {
+  if constexpr (S == 0) {
+    return v < e ? 1 : 0;
+  } else {
+    const uint32_t o = (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x120 + S, 0xf, 0xf, false);   // row_ror:S
+    return (o < e ? 1 : 0) + row_below<S - 1>(v, e);
+  }
 }
 
 // Appends each rebuilding node's handed-over entries (tlist) to its candidate list, in
 // ascending entry order (the order they arrived in is not deterministic).  Over the rebuilding
-// runs' particles (seg, nBuild); each wavefront takes its 64 nodes in turn, only those that
-// received entries: lane l ranks entries l, l+64, ...
-// against all the node's entries, read 64 at a time and broadcast lane by lane
-// (v_readlane); entry k goes to c0 + (number of smaller entries), entries being distinct.
-// Batches whose h is uniform hand nothing over, so most waves only read their counts.
+// runs' particles (seg, nBuild), 16 lanes (a DPP row) per node: each lane ranks an entry against all
+// the node's entries, 16 at a time, and entry k goes to c0 + (number of smaller entries), entries
+// being distinct.  Batches whose h is uniform hand nothing over and only read their counts.
 // overflow[0]: the candidate capacity needed, overflow[1]: the handed-over capacity needed.
+// A wavefront per 64 nodes, one node after the other, was bound by the latency of each node's reads:
+// KH 2-D 58.7 us per rebuild, Sod 3-D 25k 135 us, Evrard 250k 865 us.
+constexpr int kMergeLanes = 16;
 __global__ void __launch_bounds__(kBlock) k_candidates_merge(Fields f, const int2* seg, int nseg, int nBuild,
                                                              const uint32_t* tlist, const int* tcnt, int tcap,
                                                              int* overflow) {
-  const int lane = threadIdx.x & 63;
-  const int k = blockIdx.x*blockDim.x + threadIdx.x;
-  const int me = k < nBuild ? build_pos(seg, nseg, k) : 0;
-  int t = 0, c0 = 0;
-  bool ok = false;
-  if (k < nBuild) {
-    t = tcnt[me];
-    if (t > tcap) {
-      atomicMax(&overflow[1], t);
-    } else if (t > 0) {
-      c0 = f.ccnt[me];
-      if (c0 + t > f.ccap) atomicMax(&overflow[0], c0 + t);
-      else ok = true;
-    }
+  const int gl = xcd_block()*blockDim.x + threadIdx.x;
+  const int k = gl/kMergeLanes, sub = gl & (kMergeLanes - 1);
+  if (k >= nBuild) return;                     // a node's lanes leave together
+  const int i = build_pos(seg, nseg, k);
+  const int t = tcnt[i];
+  if (t == 0) return;
+  if (t > tcap) {
+    if (sub == 0) atomicMax(&overflow[1], t);
+    return;
+  }
+  const int c0 = f.ccnt[i];
+  if (c0 + t > f.ccap) {
+    if (sub == 0) atomicMax(&overflow[0], c0 + t);
+    return;
   }
   const size_t ld = (size_t)f.ld;
-  unsigned long long todo = __ballot(ok);
-  while (todo) {
-    const int l = __ffsll((long long)todo) - 1;
-    todo &= todo - 1;
-    const int i = __shfl(me, l), ti = __shfl(t, l), ci = __shfl(c0, l);
-    for (int kb = 0; kb < ti; kb += 64) {
-      const int k = kb + lane;
-      const uint32_t e = k < ti ? tlist[ell_at(k, i, ld)] : 0u;
-      int rank = 0;
-      for (int cb = 0; cb < ti; cb += 64) {
-        const int v = cb + lane < ti ? (int)tlist[ell_at(cb + lane, i, ld)] : -1;
-        const int m = min(64, ti - cb);
-        for (int q = 0; q < m; ++q) rank += (uint32_t)__builtin_amdgcn_readlane(v, q) < e ? 1 : 0;
-      }
-      if (k < ti) f.cand[ell_at(ci + rank, i, ld)] = e;
+  for (int kb = 0; kb < t; kb += kMergeLanes) {
+    const uint32_t e = kb + sub < t ? tlist[ell_at(kb + sub, i, ld)] : ~0u;
+    int rank = 0;
+    for (int cb = 0; cb < t; cb += kMergeLanes) {
+      const uint32_t v = cb == kb ? e : (cb + sub < t ? tlist[ell_at(cb + sub, i, ld)] : ~0u);
+      rank += row_below(v, e);
     }
+    if (kb + sub < t) f.cand[ell_at(c0 + rank, i, ld)] = e;
   }
-  if (ok) f.ccnt[me] = c0 + t;
+  if (sub == 0) f.ccnt[i] = c0 + t;
 }
 
 // Per-run maximum of an order-preserving double key: a wavefront whose lanes share a run

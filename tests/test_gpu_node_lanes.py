@@ -54,3 +54,30 @@ def test_short_lists_match_oracle(gpu, oracle_mod, reach):
     for f in FIELDS:
         a, c = g.field(f), o.field(f)
         assert np.all(np.abs(a - c) <= 1e-9*max(np.abs(c).max(), 1e-300)), f
+
+
+@pytest.mark.parametrize("wide", [1, 15, 16, 17, 40, 70])
+@pytest.mark.parametrize("dim", [2, 3])
+def test_handed_over_entries_match_oracle(gpu, oracle_mod, dim, wide):
+    """`wide` nodes whose support covers a cluster of nodes with an eighth of it: every cluster node
+    receives `wide` entries its own support does not find, below, at and beyond the 16 that one
+    row of lanes ranks at a time."""
+    print(f"[case] {wide} wide nodes, {dim}-D", flush=True)
+    rng = np.random.default_rng(100*dim + wide)
+    n = 60
+    x = np.concatenate([0.05*rng.uniform(-1, 1, (n, dim)), 0.5 + 0.1*rng.uniform(-1, 1, (wide, dim))])
+    h = np.concatenate([np.full(n, 0.1), np.full(wide, 0.8)])
+    H = np.zeros((n + wide, dim, dim))
+    for a in range(dim):
+        H[:, a, a] = 1.0/h
+    st = dict(x=x, v=np.zeros_like(x), m=np.full(n + wide, 1.0/(n + wide)), rho=np.ones(n + wide), eps=np.ones(n + wide),
+              H=H)
+    cfg = abi.default_config(dim, nperh=2.01)
+    g = gpu.make_run(cfg, st)
+    g.initialize()
+    o = oracle_mod.OracleRun(cfg, n + wide)
+    o.set_state(**st)
+    o.initialize()
+    for a, c in zip(g.neighbors(), o.neighbors()):
+        assert np.array_equal(a, c)
+    assert g.neighbor_counts()[:n].min() >= wide
