@@ -341,18 +341,22 @@ class Batch {
   void uploadTable() {
     const size_t nint = table.W.N1 + 1;
     std::vector<double> coef(6*nint);
+    std::vector<double> coefG(table.gW.coef);
     std::vector<float> coef32(6*nint);
     for (size_t k = 0; k < nint; ++k)
       for (int c = 0; c < 3; ++c) { coef[6*k + c] = table.W.coef[3*k + c]; coef[6*k + 3 + c] = table.gW.coef[3*k + c]; }
     for (size_t k = 0; k < coef.size(); ++k) coef32[k] = (float)coef[k];
     double* dc = dalloc<double>(coef.size());
     float* dc32 = dalloc<float>(coef32.size());
+    double* dg = dalloc<double>(coefG.size());
     double* dh = dalloc<double>(table.nperh.vals.size());
     upload(dc, coef.data(), coef.size()*sizeof(double));
     upload(dc32, coef32.data(), coef32.size()*sizeof(float));
+    upload(dg, coefG.data(), coefG.size()*sizeof(double));
     upload(dh, table.nperh.vals.data(), table.nperh.vals.size()*sizeof(double));
     dtab.coef = dc;
     dtab.coef32 = dc32;
+    dtab.coefG = dg;
     dtab.herm = dh;
     dtab.n1 = (int)table.W.N1;
     dtab.inv_xstep = 1.0/table.W.xstep;
@@ -1379,12 +1383,13 @@ class Batch {
   // what Integrator::postStateUpdate left: tensor images with grad-h on (SPH asks for boundaries
   // after the Q's copy), zero with it off.  Package calls see boundaries applied.
   void sphPass(bool full, bool withV12 = false, bool stepMid = false) {
-    // lanes per node: the kernel's own choice, from dimension and precision
-    const int64_t lanes = sph_lanes(D, mixed);
+    // lanes per node: from dimension and precision alone
+    const int64_t lanes = mixed ? kSphLanesMixed : D == 1 ? kSphLanes64<1> : D == 2 ? kSphLanes64<2> : kSphLanes64<3>;
     const int nb = (int)xcd_grid(nActive*lanes, kBlock);
     Phys ph = this->ph;
     ph.qImages = stepMid ? (cfg.gradh_correction ? 1 : 0) : 1;
-    const size_t tabBytes = tableBytes();
+    // FP64 stages the gradient's coefficients alone, unless the outputs include kernel values
+    const size_t tabBytes = mixed || full ? tableBytes() : tableBytes()/2;
     const int useLds = tabBytes <= kLdsTableMax ? 1 : 0;
     const size_t shm = useLds ? tabBytes : 0;
     const Scalars* sc = withV12 ? (const Scalars*)dsc : nullptr;

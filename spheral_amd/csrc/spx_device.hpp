@@ -210,6 +210,7 @@ enum RunState { RUN_FREE = 0, RUN_ACTIVE = 1, RUN_DONE = 2, RUN_REMOVED = 3 };
 struct DevTable {
   const double* coef;
   const float* coef32;     // the same coefficients rounded to float (mixed-precision pair math)
+  const double* coefG;     // dW's three coefficients per interval alone
   const double* herm;
   int n1;
   int hn;
@@ -401,28 +402,13 @@ template <typename R> __device__ __forceinline__ const R* table_coef(const DevTa
 template <> __device__ __forceinline__ const double* table_coef<double>(const DevTable& t) { return t.coef; }
 template <> __device__ __forceinline__ const float* table_coef<float>(const DevTable& t) { return t.coef32; }
 
-// TableKernelView::kernelAndGradValue (Kernel/TableKernelViewInline.hh:84-99) in arithmetic R.
-template <typename R = double>
-__device__ __forceinline__ void kernel_wgw(const DevTable& t, R eta, R hdet, R& w, R& gw) {
-  if (eta < (R)t.extent) {
-    int b = (int)(eta*(R)t.inv_xstep);
-    b = b < t.n1 ? b : t.n1;
-    const R* c = table_coef<R>(t) + 6*b;
-    w = hdet*(c[0] + (c[1] + c[2]*eta)*eta);
-    gw = hdet*(c[3] + (c[4] + c[5]*eta)*eta);
-  } else {
-    w = (R)0;
-    gw = (R)0;
-  }
-}
-
 // A pointer into the block's LDS, typed as such (address space 3) so that loads through it are
 // LDS reads wherever the optimiser moves them.
 template <typename R>
 using lds_ptr = const R __attribute__((address_space(3)))*;
 
-// The same lookup on a given copy of the coefficients (a global pointer, or an lds_ptr to the
-// block's staged copy); graw is the gradient polynomial before the Hdet factor, so |graw| is
+// TableKernelView::kernelAndGradValue (Kernel/TableKernelViewInline.hh:84-99) in arithmetic R, on a
+// given copy of the coefficients (a global pointer, or an lds_ptr to the block's staged copy); graw is the gradient polynomial before the Hdet factor, so |graw| is
 // kernelValueSPH at the same eta.  Branch-free: the interval index is clamped to the last one (in
 // bounds for any eta >= 0, the float-to-int conversion saturates), and the values beyond the
 // extent are selected to zero.
@@ -439,18 +425,25 @@ __device__ __forceinline__ void kernel_wgw_c(CP coef, const DevTable& t, R eta, 
   gw = in ? hdet*gr : (R)0;
 }
 
-// The kernel table's coefficients for a pair pass, staged in the block's dynamic LDS (every
-// thread of the block must call this before any returns).  Pair passes call their node body
-// through with_table: once with this LDS pointer and once with the global table, never with a
-// generic pointer that may be either -- a load through such a pointer is a flat load, and waiting
-// for its result also waits for every global load issued before it (e.g. the next neighbour's
-// prefetched record).
+// dW/deta before the Hdet factor, from coefficients c0 c1 c2 at coef + STRIDE*interval.
+template <int STRIDE, typename R, typename CP>
+__device__ __forceinline__ R kernel_graw(CP coef, const DevTable& t, R eta) {
+  int b = (int)(eta*(R)t.inv_xstep);
+  b = b < t.n1 ? b : t.n1;
+  const CP c = coef + STRIDE*b;
+  const R gr = fused(fused(c[2], eta, c[1]), eta, c[0]);
+  return eta < (R)t.extent ? gr : (R)0;
+}
+
+// nc coefficients of the kernel table staged in the block's dynamic LDS (every thread of the block
+// must call this before any returns).  Pair passes call their node body through with_table: once
+// with this LDS pointer and once with the global table, never with a generic pointer that may be
+// either -- a load through such a pointer is a flat load, and waiting for its result also waits for
+// every global load issued before it (e.g. the next neighbour's prefetched record).
 template <typename R>
-__device__ __forceinline__ lds_ptr<R> stage_table_lds(const DevTable& tab) {
+__device__ __forceinline__ lds_ptr<R> stage_table_lds(const R* coef, int nc) {
   extern __shared__ __align__(16) unsigned char spx_lds[];
-  const R* coef = table_coef<R>(tab);
   R* t = reinterpret_cast<R*>(spx_lds);
-  const int nc = 6*(tab.n1 + 1);
   for (int k = threadIdx.x; k < nc; k += blockDim.x) t[k] = coef[k];
   __syncthreads();
   return (lds_ptr<R>)t;
@@ -460,20 +453,14 @@ __device__ __forceinline__ lds_ptr<R> stage_table_lds(const DevTable& tab) {
 // memory; body is a generic lambda, instantiated once per pointer type.
 template <typename R, typename F>
 __device__ __forceinline__ void with_table(const DevTable& tab, int lds, F&& body) {
-  if (lds) body(stage_table_lds<R>(tab));
+  if (lds) body(stage_table_lds<R>(table_coef<R>(tab), 6*(tab.n1 + 1)));
   else body(table_coef<R>(tab));
 }
-
-// kernelValueSPH: |dW/deta| at Hdet = 1 (Kernel/TableKernelViewInline.hh:112-120)
-template <typename R = double>
-__device__ __forceinline__ R kernel_wsph(const DevTable& t, R eta) {
-  if (eta < (R)t.extent) {
-    int b = (int)(eta*(R)t.inv_xstep);
-    b = b < t.n1 ? b : t.n1;
-    const R* c = table_coef<R>(t) + 6*b;
-    return fabs(c[3] + (c[4] + c[5]*eta)*eta);
-  }
-  return (R)0;
+// The same with dW's coefficients alone, three per interval.
+template <typename F>
+__device__ __forceinline__ void with_gradient_table(const DevTable& tab, int lds, F&& body) {
+  if (lds) body(stage_table_lds<double>(tab.coefG, 3*(tab.n1 + 1)));
+  else body(tab.coefG);
 }
 
 // equivalentNodesPerSmoothingScale: cubic Hermite lookup (CubicHermiteInterpolatorViewInline.hh:9-33,120-125)

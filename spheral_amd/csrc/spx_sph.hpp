@@ -1,4 +1,5 @@
-// spx_sph.hpp -- the SPH derivative pass and the compatible-energy full update (FP64 path).
+// spx_sph.hpp -- the SPH derivative pass (mixed precision and FP64) and the compatible-energy full
+// update.
 #pragma once
 
 #include "spx_kernels.hpp"
@@ -82,6 +83,45 @@ struct PairS {
   R C, Ws, Qs, workQs, vdg, etaMagS, wsphS;
 };
 
+// LimitedMonaghanGingoldViscosity's velocity jump dotted with r (LimitedMonaghanGingoldViscosity.cc:
+// 160-195): the jump at the pair's midpoint, extrapolated with the nodes' velocity gradients TS, TO
+// (row-major D x D, the partner's already image-transformed) scaled by the limiter.
+template <int D, typename R>
+__device__ __forceinline__ R limited_jump(const Phys& ph, const R* r, const double* vS, const double* vO, R etaS, R etaO,
+                                          const R* TS, const R* TO) {
+  // van Leer limiter on the ratio of the gradients' projections along the half separation,
+  // phased back toward the full Q when the pair is closer than etaCrit
+  R xij[D], gi = (R)0, gj = (R)0;
+#pragma unroll
+  for (int c = 0; c < D; ++c) xij[c] = (R)0.5*r[c];
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    R s1 = TS[a*D]*xij[0], s2 = TO[a*D]*xij[0];
+#pragma unroll
+    for (int b = 1; b < D; ++b) { s1 += TS[a*D + b]*xij[b]; s2 += TO[a*D + b]*xij[b]; }
+    gi = a == 0 ? s1*xij[0] : gi + s1*xij[a];
+    gj = a == 0 ? s2*xij[0] : gj + s2*xij[a];
+  }
+  const R tiny30 = sizeof(R) == sizeof(double) ? (R)1.0e-30 : (R)1.0e-30f;
+  const R ri = gi/((gj < (R)0 ? (R)-1 : (R)1)*fmax(tiny30, fabs(gj)));
+  const R rj = gj/((gi < (R)0 ? (R)-1 : (R)1)*fmax(tiny30, fabs(gi)));
+  const R rmin = fmin(ri, rj);
+  R phi = rmin > (R)0 ? (R)2/((R)1 + rmin)*(R)2*rmin/((R)1 + rmin) : (R)0;
+  const R etaij = fmin(etaS, etaO), ec = (R)ph.etaCrit;
+  if (etaij < ec) { const R q = (etaij - ec)/(R)ph.etaFold; phi *= exp(-(q*q)); }
+  // (phi*T).xij: the product with the scaled tensor, as the reference forms it
+  R vqr = (R)0;
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    R s1 = (phi*TS[a*D])*xij[0], s2 = (phi*TO[a*D])*xij[0];
+#pragma unroll
+    for (int b = 1; b < D; ++b) { s1 += (phi*TS[a*D + b])*xij[b]; s2 += (phi*TO[a*D + b])*xij[b]; }
+    const R vq = (R)((vS[a] - (double)s1) - (vO[a] + (double)s2));
+    vqr += vq*r[a];
+  }
+  return vqr;
+}
+
 // coef: the kernel table's coefficients in arithmetic R (global, or the block's LDS copy).
 // LQ: LimitedMonaghanGingoldViscosity::QPiij (LimitedMonaghanGingoldViscosity.cc:160-195) in
 // place of the plain Q; TS, TO are the two nodes' velocity gradients as the Q holds them
@@ -101,7 +141,7 @@ __device__ __forceinline__ void pair_eval(const DevTable& tab, CP coef, const Ph
     e.vso[c] = (R)(S.v[c] - O.v[c]);
   }
   // |eta| and safeInvVar(|eta|) = 1/max(1e-30, |eta|) from one reciprocal square root each
-  const R tiny = sizeof(R) == sizeof(double) ? (R)1.0e-30 : (R)1.0e-30f;
+  const R tiny = (R)1.0e-30f;
   const R is = e2s > tiny*tiny ? rsqrt(e2s) : (R)1/tiny, io = e2o > tiny*tiny ? rsqrt(e2o) : (R)1/tiny;
   e.etaMagS = e2s*is;
   const R etaMagO = e2o*io;
@@ -119,36 +159,7 @@ __device__ __forceinline__ void pair_eval(const DevTable& tab, CP coef, const Ph
   // velocity jump the Q sees: the plain difference, or the limited midpoint extrapolation
   R vqr = vsr;
   if (LQ) {
-    // van Leer limiter on the ratio of the gradients' projections along the half separation,
-    // phased back toward the full Q when the pair is closer than etaCrit
-    R xij[D], gi = (R)0, gj = (R)0;
-#pragma unroll
-    for (int c = 0; c < D; ++c) xij[c] = (R)0.5*e.r[c];
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-      R s1 = TS[a*D]*xij[0], s2 = TO[a*D]*xij[0];
-#pragma unroll
-      for (int b = 1; b < D; ++b) { s1 += TS[a*D + b]*xij[b]; s2 += TO[a*D + b]*xij[b]; }
-      gi = a == 0 ? s1*xij[0] : gi + s1*xij[a];
-      gj = a == 0 ? s2*xij[0] : gj + s2*xij[a];
-    }
-    const R tiny30 = sizeof(R) == sizeof(double) ? (R)1.0e-30 : (R)1.0e-30f;
-    const R ri = gi/((gj < (R)0 ? (R)-1 : (R)1)*fmax(tiny30, fabs(gj)));
-    const R rj = gj/((gi < (R)0 ? (R)-1 : (R)1)*fmax(tiny30, fabs(gi)));
-    const R rmin = fmin(ri, rj);
-    R phi = rmin > (R)0 ? (R)2/((R)1 + rmin)*(R)2*rmin/((R)1 + rmin) : (R)0;
-    const R etaij = fmin(e.etaMagS, etaMagO), ec = (R)ph.etaCrit;
-    if (etaij < ec) { const R q = (etaij - ec)/(R)ph.etaFold; phi *= exp(-(q*q)); }
-    // (phi*T).xij: the product with the scaled tensor, as the reference forms it
-    vqr = (R)0;
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-      R s1 = (phi*TS[a*D])*xij[0], s2 = (phi*TO[a*D])*xij[0];
-#pragma unroll
-      for (int b = 1; b < D; ++b) { s1 += (phi*TS[a*D + b])*xij[b]; s2 += (phi*TO[a*D + b])*xij[b]; }
-      const R vq = (R)((S.v[a] - (double)s1) - (O.v[a] + (double)s2));
-      vqr += vq*e.r[a];
-    }
+    vqr = limited_jump<D, R>(ph, e.r, S.v, O.v, e.etaMagS, etaMagO, TS, TO);
   }
   // mu = (vq . eta)/(eta^2 + eps^2) with eta = h^-1 r on each side
   const R mus = (S.h*vqr)/(e2s + (R)1.0e-2), muo = (O.h*vqr)/(e2o + (R)1.0e-2);
@@ -176,21 +187,6 @@ __device__ __forceinline__ void pair_eval(const DevTable& tab, CP coef, const Ph
 // pair loop makes three lookups per pair at scattered intervals).  sc != nullptr (the step):
 // the node's half-step velocity record for the compatible-energy update is written too (as
 // k_v12 would, with the run's dt/2).
-template <typename R>
-constexpr bool kSymM = sizeof(R) == sizeof(double);
-
-// Lanes per node of the SPH pass.  With two, the lanes of an adjacent (even, odd) pair take the
-// node's ELL entries k = 0, 2, 4, ... and 1, 3, 5, ... and add their partial sums at the end (a
-// DPP swap within the pair: both lanes form the same a + b), doubling the pass's parallelism
-// for the same registers per lane.  Measured on one MI355X (SPH pass time): KH 2-D 4096 mixed
-// 57.8 -> 32.6 us, KH 2-D 65536 mixed 75.0 -> 52.7 us, TG 3-D 16^3 FP64 65.6 -> 39.8 us,
-// TG 3-D 128^3 mixed 1.244 -> 1.209 ms, but TG 3-D 128^3 FP64 1.362 -> 1.384 ms and TG 3-D 48^3
-// FP64 unchanged.  The choice depends only on the configuration (dimension, precision), never on
-// the particle count, so a run gives the same bits in any batch.
-__host__ __device__ constexpr int sph_lanes(int D, bool mixed) { return (mixed || D <= 2) ? 2 : 1; }
-template <int D, typename R>
-constexpr int kSphLanes = sph_lanes(D, sizeof(R) == sizeof(float));
-
 __device__ __forceinline__ double lane_pair_swap(double v) {
   const int lo = __double2loint(v), hi = __double2hiint(v);
   // quad_perm [1, 0, 3, 2]: lane 2m reads lane 2m+1 and vice versa
@@ -199,12 +195,115 @@ __device__ __forceinline__ double lane_pair_swap(double v) {
   return __hiloint2double(hi2, lo2);
 }
 
-template <int D, bool FULL, typename R, bool LQ, typename CP>
+// A node's sums over its pairs.
+template <int D>
+struct SphSums {
+  double dvdt[D], dvdx[D*D], M[D*D], depsdt, maxq, m0;
+  double rhosum, nrm, effq, grho[D], m1[D];              // FULL
+};
+
+// The node's derivatives and ideal H from its sums (SPH.cc:480-551, SPHSmoothingScale.cc:228-245),
+// double precision, and its partition record.
+template <int D, bool FULL>
+__device__ __forceinline__ void sph_finalize(const Fields& f, const Phys& ph, const DevTable& tab, int i, int nn,
+                                             SphSums<D>& q, const Scalars* sc) {
+  const size_t ld = (size_t)f.ld;
+  const double Sm = f.m[i], Srho = f.rhom[i], Sh = f.hinvm[i];
+  const double hdet = hdet_iso<D>(Sh);
+  double det;
+  if (D == 1) det = q.M[0];
+  else if (D == 2) det = q.M[0]*q.M[3] - q.M[1]*q.M[2];
+  else det = (q.M[0]*q.M[4]*q.M[8] + q.M[1]*q.M[5]*q.M[6] + q.M[2]*q.M[3]*q.M[7] -
+              q.M[0]*q.M[5]*q.M[7] - q.M[1]*q.M[3]*q.M[8] - q.M[2]*q.M[4]*q.M[6]);
+  const double pow2d = D == 1 ? 2.0 : (D == 2 ? 4.0 : 8.0);
+  double G[D*D];
+  if (ph.correctVG && fabs(det) > 1.0e-10 && (double)nn > pow2d) {
+    double Mi[D*D];
+    if (D == 1) {
+      Mi[0] = 1.0/q.M[0];
+    } else if (D == 2) {
+      const double r = 1.0/det;
+      Mi[0] = q.M[3]*r; Mi[1] = -q.M[1]*r; Mi[2] = -q.M[2]*r; Mi[3] = q.M[0]*r;
+    } else {
+      const double r = 1.0/det;
+      const double xx = q.M[0], xy = q.M[1], xz = q.M[2], yx = q.M[3], yy = q.M[4], yz = q.M[5], zx = q.M[6], zy = q.M[7], zz = q.M[8];
+      Mi[0] = (yy*zz - yz*zy)*r; Mi[1] = (xz*zy - xy*zz)*r; Mi[2] = (xy*yz - xz*yy)*r;
+      Mi[3] = (yz*zx - yx*zz)*r; Mi[4] = (xx*zz - xz*zx)*r; Mi[5] = (xz*yx - xx*yz)*r;
+      Mi[6] = (yx*zy - yy*zx)*r; Mi[7] = (xy*zx - xx*zy)*r; Mi[8] = (xx*yy - xy*yx)*r;
+    }
+#pragma unroll
+    for (int a = 0; a < D; ++a)
+#pragma unroll
+      for (int b = 0; b < D; ++b) {
+        double s = 0.0;
+#pragma unroll
+        for (int k2 = 0; k2 < D; ++k2) s += q.dvdx[a*D + k2]*Mi[k2*D + b];
+        G[a*D + b] = s;
+      }
+    if (FULL) {
+#pragma unroll
+      for (int a = 0; a < D*D; ++a) q.M[a] = Mi[a];
+    }
+  } else {
+#pragma unroll
+    for (int a = 0; a < D*D; ++a) G[a] = rdiv<D>(q.dvdx[a], Srho);
+  }
+  double tr = 0.0;
+#pragma unroll
+  for (int a = 0; a < D; ++a) tr += G[a*D + a];
+#pragma unroll
+  for (int a = 0; a < D*D; ++a) f.DvDx[a*ld + i] = G[a];
+#pragma unroll
+  for (int a = 0; a < D; ++a) { f.DvDt[a][i] = q.dvdt[a]; f.DxDt[a][i] = f.vm[a][i]; }
+  f.DepsDt[i] = q.depsdt;
+  {
+    // the partition record: this evaluation's positions (the pair coefficients' r) always; the
+    // half-step velocities and DepsDt in the step (otherwise k_v12 writes them)
+    double2* PV = reinterpret_cast<double2*>(f.pkv) + 4*(size_t)i;
+    double xs[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int a = 0; a < D; ++a) xs[a] = f.xm[a][i];
+    if (sc) {
+      const double hdt = 0.5*sc[f.run[i]].dt;
+      double w[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+      for (int a = 0; a < D; ++a) w[a] = f.v[a][i] + q.dvdt[a]*hdt;
+      PV[0] = make_double2(w[0], w[1]);
+      PV[1] = make_double2(w[2], q.depsdt);
+    }
+    PV[2] = make_double2(Sm, xs[0]);
+    PV[3] = make_double2(xs[1], xs[2]);
+  }
+  f.DrhoDt[i] = -Srho*tr;
+  f.maxQ[i] = q.maxq;
+  // ---- SPHSmoothingScale finalize (SPHSmoothingScale.cc:228-245)
+  const double m0 = rootnu<D>(fmax(0.0, q.m0));
+  f.m0[i] = m0;
+  f.DHDt[i] = rdiv<D>(-Sh, double(D))*tr;
+  const double cur = (fabs(m0) <= 1.0e-15*fmax(1.0, fabs(m0))) ? 0.5*ph.nperh : nperh_lookup(tab, m0);
+  const double s = fmin(4.0, fmax(0.25, ph.nperh/(cur + 1.0e-30)));
+  const double aa = s < 1.0 ? 0.4*(1.0 + s*s) : 0.4*(1.0 + 1.0/(s*s*s));
+  const double hi0 = 1.0/Sh;
+  const double hi1 = fmin(ph.hmax, fmax(ph.hmin, hi0*(1.0 - aa + aa*s)));
+  f.Hideal[i] = 1.0/hi1;
+  if (FULL) {
+    f.rhoSum[i] = q.rhosum + Sm*tab.W0*hdet;
+    f.norm[i] = q.nrm + Sm/Srho*tab.W0*hdet;
+    f.effQ[i] = q.effq;
+#pragma unroll
+    for (int c = 0; c < D; ++c) { f.gradRho[c][i] = rdiv<D>(q.grho[c], Srho); f.m1[c][i] = q.m1[c]; }
+#pragma unroll
+    for (int a = 0; a < D*D; ++a) f.Mcorr[a*ld + i] = q.M[a];
+  }
+}
+
+template <int D, bool FULL, bool LQ, typename CP>
 __device__ __forceinline__ void sph_node(const Fields& f, const Geo& g, const Phys& ph, const DevTable& tab,
                                          CP coef, int n, const Scalars* sc) {
-  constexpr int L = kSphLanes<D, R>;
+  using R = float;
+  constexpr int L = 2;
   const int gl = xcd_block()*blockDim.x + threadIdx.x;
-  const int i = L == 1 ? gl : gl >> 1, sub = L == 1 ? 0 : (gl & 1);
+  const int i = gl >> 1, sub = gl & 1;
   // both lanes of a pair share i: they leave together
   if (i >= n) return;
   const size_t ld = (size_t)f.ld;
@@ -226,39 +325,18 @@ __device__ __forceinline__ void sph_node(const Fields& f, const Geo& g, const Ph
     for (int a = 0; a < D*D; ++a) TS[a] = (R)f.DvDxQ[a*ld + i];
   }
   const int nn = f.cnt[i];
-  // the next ELL entry and its neighbour's record are fetched one pair ahead (one lane: the
-  // entries come 8 at a time in the blocked list's 32-byte chunks)
-  uint4 c0 = make_uint4(0u, 0u, 0u, 0u), c1 = c0;
+  // the next ELL entry and its neighbour's record are fetched one pair ahead
   uint32_t en = 0;
   NbrRaw<D> rn;
   if (sub < nn) {
-    if (L == 1) {
-      const uint4* cp = reinterpret_cast<const uint4*>(f.nbr + ell_at(0, i, ld));
-      c0 = cp[0];
-      c1 = cp[1];
-      en = c0.x;
-    } else {
-      en = f.nbr[ell_at(sub, i, ld)];
-    }
+    en = f.nbr[ell_at(sub, i, ld)];
     load_raw<D>(f, (int)(en & kIdxMask), rn);
   }
   for (int k = sub; k < nn; k += L) {
     const uint32_t ent = en;
     const NbrRaw<D> rc = rn;
     if (k + L < nn) {
-      const int k1 = k + L;
-      if (L == 1) {
-        const int u = k1 & 7;
-        if (u == 0) {
-          const uint4* cp = reinterpret_cast<const uint4*>(f.nbr + ell_at(k1, i, ld));
-          c0 = cp[0];
-          c1 = cp[1];
-        }
-        en = u == 0 ? c0.x : u == 1 ? c0.y : u == 2 ? c0.z : u == 3 ? c0.w
-           : u == 4 ? c1.x : u == 5 ? c1.y : u == 6 ? c1.z : c1.w;
-      } else {
-        en = f.nbr[ell_at(k1, i, ld)];
-      }
+      en = f.nbr[ell_at(k + L, i, ld)];
       load_raw<D>(f, (int)(en & kIdxMask), rn);
     }
     const int j = (int)(ent & kIdxMask);
@@ -292,10 +370,8 @@ __device__ __forceinline__ void sph_node(const Fields& f, const Geo& g, const Ph
 #pragma unroll
       for (int d = 0; d < D; ++d) {
         dvdx[c*D + d] -= mv*(double)e.gs[d];
-        // with isotropic H the gradient is parallel to r, so M = sum m r (x) gradW is symmetric:
-        // in FP64 the upper triangle is accumulated and mirrored after the loop (the FP32 pair
-        // terms round r_c g_d and r_d g_c differently, so mixed precision keeps all nine)
-        if (!kSymM<R> || d >= c) Mc[c*D + d] -= mr*(double)e.gs[d];
+        // (the FP32 pair terms round r_c g_d and r_d g_c differently: all of M is accumulated)
+        Mc[c*D + d] -= mr*(double)e.gs[d];
       }
     }
     depsdt += mo*(double)(S.prho*e.vdg + e.workQs);
@@ -315,7 +391,7 @@ __device__ __forceinline__ void sph_node(const Fields& f, const Geo& g, const Ph
     }
   }
 
-  if (L == 2) {
+  {
     // the pair's partial sums: each lane forms (own + partner's), the same bits on both
 #pragma unroll
     for (int a = 0; a < D; ++a) dvdt[a] += lane_pair_swap(dvdt[a]);
@@ -324,7 +400,7 @@ __device__ __forceinline__ void sph_node(const Fields& f, const Geo& g, const Ph
 #pragma unroll
       for (int d = 0; d < D; ++d) {
         dvdx[c*D + d] += lane_pair_swap(dvdx[c*D + d]);
-        if (!kSymM<R> || d >= c) Mc[c*D + d] += lane_pair_swap(Mc[c*D + d]);
+        Mc[c*D + d] += lane_pair_swap(Mc[c*D + d]);
       }
     depsdt += lane_pair_swap(depsdt);
     m0 += lane_pair_swap(m0);
@@ -338,105 +414,247 @@ __device__ __forceinline__ void sph_node(const Fields& f, const Geo& g, const Ph
     }
     if (sub != 0) return;
   }
-  if (kSymM<R>) {
+  SphSums<D> q;
 #pragma unroll
-    for (int c = 1; c < D; ++c)
+  for (int a = 0; a < D; ++a) { q.dvdt[a] = dvdt[a]; q.grho[a] = grho[a]; q.m1[a] = m1[a]; }
 #pragma unroll
-      for (int d = 0; d < c; ++d) Mc[c*D + d] = Mc[d*D + c];
-  }
-  // ---- per-node finalize (SPH.cc:480-551), double precision
-  const double hdet = hdet_iso<D>(Sh);
-  double det;
-  if (D == 1) det = Mc[0];
-  else if (D == 2) det = Mc[0]*Mc[3] - Mc[1]*Mc[2];
-  else det = (Mc[0]*Mc[4]*Mc[8] + Mc[1]*Mc[5]*Mc[6] + Mc[2]*Mc[3]*Mc[7] -
-              Mc[0]*Mc[5]*Mc[7] - Mc[1]*Mc[3]*Mc[8] - Mc[2]*Mc[4]*Mc[6]);
-  const double pow2d = D == 1 ? 2.0 : (D == 2 ? 4.0 : 8.0);
-  double G[D*D];
-  if (ph.correctVG && fabs(det) > 1.0e-10 && (double)nn > pow2d) {
-    double Mi[D*D];
-    if (D == 1) {
-      Mi[0] = 1.0/Mc[0];
-    } else if (D == 2) {
-      const double r = 1.0/det;
-      Mi[0] = Mc[3]*r; Mi[1] = -Mc[1]*r; Mi[2] = -Mc[2]*r; Mi[3] = Mc[0]*r;
-    } else {
-      const double r = 1.0/det;
-      const double xx = Mc[0], xy = Mc[1], xz = Mc[2], yx = Mc[3], yy = Mc[4], yz = Mc[5], zx = Mc[6], zy = Mc[7], zz = Mc[8];
-      Mi[0] = (yy*zz - yz*zy)*r; Mi[1] = (xz*zy - xy*zz)*r; Mi[2] = (xy*yz - xz*yy)*r;
-      Mi[3] = (yz*zx - yx*zz)*r; Mi[4] = (xx*zz - xz*zx)*r; Mi[5] = (xz*yx - xx*yz)*r;
-      Mi[6] = (yx*zy - yy*zx)*r; Mi[7] = (xy*zx - xx*zy)*r; Mi[8] = (xx*yy - xy*yx)*r;
-    }
-#pragma unroll
-    for (int a = 0; a < D; ++a)
-#pragma unroll
-      for (int b = 0; b < D; ++b) {
-        double s = 0.0;
-#pragma unroll
-        for (int k2 = 0; k2 < D; ++k2) s += dvdx[a*D + k2]*Mi[k2*D + b];
-        G[a*D + b] = s;
-      }
-    if (FULL) {
-#pragma unroll
-      for (int a = 0; a < D*D; ++a) Mc[a] = Mi[a];
-    }
-  } else {
-#pragma unroll
-    for (int a = 0; a < D*D; ++a) G[a] = rdiv<D>(dvdx[a], Srho);
-  }
-  double tr = 0.0;
-#pragma unroll
-  for (int a = 0; a < D; ++a) tr += G[a*D + a];
-#pragma unroll
-  for (int a = 0; a < D*D; ++a) f.DvDx[a*ld + i] = G[a];
-#pragma unroll
-  for (int a = 0; a < D; ++a) { f.DvDt[a][i] = dvdt[a]; f.DxDt[a][i] = f.vm[a][i]; }
-  f.DepsDt[i] = depsdt;
-  {
-    // the partition record: this evaluation's positions (the pair coefficients' r) always; the
-    // half-step velocities and DepsDt in the step (otherwise k_v12 writes them)
-    double2* PV = reinterpret_cast<double2*>(f.pkv) + 4*(size_t)i;
-    double xs[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-    for (int a = 0; a < D; ++a) xs[a] = S.x[a];
-    if (sc) {
-      const double hdt = 0.5*sc[f.run[i]].dt;
-      double w[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-      for (int a = 0; a < D; ++a) w[a] = f.v[a][i] + dvdt[a]*hdt;
-      PV[0] = make_double2(w[0], w[1]);
-      PV[1] = make_double2(w[2], depsdt);
-    }
-    PV[2] = make_double2(Sm, xs[0]);
-    PV[3] = make_double2(xs[1], xs[2]);
-  }
-  f.DrhoDt[i] = -Srho*tr;
-  f.maxQ[i] = maxq;
-  // ---- SPHSmoothingScale finalize (SPHSmoothingScale.cc:228-245)
-  m0 = rootnu<D>(fmax(0.0, m0));
-  f.m0[i] = m0;
-  f.DHDt[i] = rdiv<D>(-Sh, double(D))*tr;
-  const double cur = (fabs(m0) <= 1.0e-15*fmax(1.0, fabs(m0))) ? 0.5*ph.nperh : nperh_lookup(tab, m0);
-  const double s = fmin(4.0, fmax(0.25, ph.nperh/(cur + 1.0e-30)));
-  const double aa = s < 1.0 ? 0.4*(1.0 + s*s) : 0.4*(1.0 + 1.0/(s*s*s));
-  const double hi0 = 1.0/Sh;
-  const double hi1 = fmin(ph.hmax, fmax(ph.hmin, hi0*(1.0 - aa + aa*s)));
-  f.Hideal[i] = 1.0/hi1;
-  if (FULL) {
-    f.rhoSum[i] = rhosum + Sm*tab.W0*hdet;
-    f.norm[i] = nrm + Sm/Srho*tab.W0*hdet;
-    f.effQ[i] = effq;
-#pragma unroll
-    for (int c = 0; c < D; ++c) { f.gradRho[c][i] = rdiv<D>(grho[c], Srho); f.m1[c][i] = m1[c]; }
-#pragma unroll
-    for (int a = 0; a < D*D; ++a) f.Mcorr[a*ld + i] = Mc[a];
-  }
+  for (int a = 0; a < D*D; ++a) { q.dvdx[a] = dvdx[a]; q.M[a] = Mc[a]; }
+  q.depsdt = depsdt; q.maxq = maxq; q.m0 = m0;
+  q.rhosum = rhosum; q.nrm = nrm; q.effq = effq;
+  sph_finalize<D, FULL>(f, ph, tab, i, nn, q, sc);
 }
 
+// ---------------------------------------------------------------------------
+// The FP64 pass: L lanes per node, each over the entries k = sub, sub + L, ...; the lanes' sums are
+// joined by DPP and left in LDS, and the block's first threads finalize its nodes.
+//
+// Everything both sides of a pair must agree on (C and what it is made of) is formed from r^2, the
+// two supports and the two records by operations that commute in the two nodes, each rounded as
+// written (no contraction the compiler could choose differently on the two sides): t_x = k_x (P_x +
+// Q_x/2), C = t_s + t_o has the same bits in both lanes, so C r is exactly antisymmetric without
+// selecting a canonical order.  An image partner's position is rounded on each side by itself, as
+// the reference's ghost is.
+// ---------------------------------------------------------------------------
+template <int D>
+__device__ __forceinline__ double h_power(double h) {   // h^(D + 1): k = dW/deta h^(D + 1) / |r|
+  if (D == 1) return rounded_product(h, h);
+  if (D == 2) return rounded_product(rounded_product(h, h), h);
+  const double h2 = rounded_product(h, h);
+  return rounded_product(h2, h2);
+}
+// A node's viscous term rho^-1 Q (before the division by rho^2's other half): Cq mu^2 - Cl cs mu.
+__device__ __forceinline__ double mg_term(const Phys& ph, double clcs, double mu) {
+  return rounded_product(mu, fused(ph.Cq, mu, -clcs));
+}
+
+// Sums of a node: DvDt, DvDx, M's upper triangle, DepsDt, the zeroth moment, the largest Q; with FULL
+// also the sum density, normalisation, effective Q, density gradient and first moment.
+constexpr int sph_sums(int D, bool full) { return D + D*D + D*(D + 1)/2 + 3 + (full ? 3 + 2*D : 0); }
+template <int D, bool FULL, bool LQ, int L, typename CP>
+__device__ __forceinline__ void sph_node64(const Fields& f, const Geo& g, const Phys& ph, const DevTable& tab, CP coef,
+                                           int n, const Scalars* sc, double (&sums)[sph_sums(D, FULL)][kBlock/L]) {
+  constexpr int NB = kBlock/L;
+  const int gl = xcd_block()*blockDim.x + threadIdx.x;
+  const int i = gl/L, sub = gl & (L - 1);
+  const size_t ld = (size_t)f.ld;
+  double* pdd = (double*)f.pdd;
+  double dvdt[D], dvdx[D*D], M[D*D], depsdt = 0.0, maxe = 0.0, m0 = 0.0;
+  double rhosum = 0.0, nrm = 0.0, effq = 0.0, grho[D], m1[D];
+#pragma unroll
+  for (int a = 0; a < D; ++a) { dvdt[a] = 0.0; grho[a] = 0.0; m1[a] = 0.0; }
+#pragma unroll
+  for (int a = 0; a < D*D; ++a) { dvdx[a] = 0.0; M[a] = 0.0; }
+  double Srho = 0.0;
+  if (i < n) {
+    NbrRaw<D> S;
+    load_raw<D>(f, i, S);
+    Srho = S.rho;
+    const double SA = h_power<D>(S.h), Sclcs = rounded_product(ph.Cl, S.cs);
+    double TS[LQ ? D*D : 1];
+    if (LQ) {
+#pragma unroll
+      for (int a = 0; a < D*D; ++a) TS[a] = f.DvDxQ[a*ld + i];
+    }
+    const int nn = f.cnt[i];
+    // the next entry and its neighbour's record are fetched one pair ahead
+    uint32_t en = 0;
+    NbrRaw<D> rn;
+    if (sub < nn) {
+      en = f.nbr[ell_at(sub, i, ld)];
+      load_raw<D>(f, (int)(en & kIdxMask), rn);
+    }
+    for (int k = sub; k < nn; k += L) {
+      const uint32_t ent = en;
+      NbrRaw<D> O = rn;
+      if (k + L < nn) {
+        en = f.nbr[ell_at(k + L, i, ld)];
+        load_raw<D>(f, (int)(en & kIdxMask), rn);
+      }
+      const int code = (int)(ent >> kImgShift);
+      if (code) {
+        image_pos<D>(g, code, O.x);
+#pragma unroll
+        for (int c = 0; c < D; ++c) O.v[c] *= refl_sign<D>(g, code, c);
+      }
+      double r[D], dv[D];
+#pragma unroll
+      for (int c = 0; c < D; ++c) { r[c] = S.x[c] - O.x[c]; dv[c] = S.v[c] - O.v[c]; }
+      const double r2 = norm2<D>(r);
+      const double rinv = r2 > 1.0e-290 ? fast_rsqrt(r2) : 0.0;
+      const double d = rounded_product(r2, rinv);
+      const double etas = rounded_product(S.h, d), etao = rounded_product(O.h, d);
+      double grs, gro, Ws = 0.0;
+      if (FULL) {
+        double gw;
+        kernel_wgw_c<double>(coef, tab, etas, hdet_iso<D, double>(S.h), Ws, gw, grs);
+        gro = kernel_graw<6, double>(coef + 3, tab, etao);
+      } else {
+        grs = kernel_graw<3, double>(coef, tab, etas);
+        gro = kernel_graw<3, double>(coef, tab, etao);
+      }
+      const double ks = rounded_product(rounded_product(grs, SA), rinv);             // gradW = k r
+      const double ko = rounded_product(rounded_product(gro, h_power<D>(O.h)), rinv);
+      double vsr = rounded_product(dv[0], r[0]);
+#pragma unroll
+      for (int c = 1; c < D; ++c) vsr = fused(dv[c], r[c], vsr);
+      double vqr = vsr;
+      if (LQ) {
+        // the limited velocity jump (pair_eval's, FP64)
+        const int j = (int)(ent & kIdxMask);
+        double TO[D*D];
+#pragma unroll
+        for (int a = 0; a < D; ++a)
+#pragma unroll
+          for (int b = 0; b < D; ++b) {
+            const double t = f.DvDxQ[(size_t)(a*D + b)*ld + j];
+            TO[a*D + b] = code ? (ph.qImages ? refl_sign<D>(g, code, a)*refl_sign<D>(g, code, b)*t : 0.0) : t;
+          }
+        vqr = limited_jump<D, double>(ph, r, S.v, O.v, etas, etao, TS, TO);
+      }
+      // mu = (vq . eta)/(eta^2 + eps^2) on each side, one reciprocal for both
+      const double ps = fused(etas, etas, 1.0e-2), po = fused(etao, etao, 1.0e-2);
+      const double inv = fast_rcp(rounded_product(ps, po));
+      const double mus = rounded_product(rounded_product(S.h, vqr), rounded_product(inv, po));
+      const double muo = rounded_product(rounded_product(O.h, vqr), rounded_product(inv, ps));
+      const double es = mg_term(ph, Sclcs, fmin(0.0, mus));
+      const double eo = mg_term(ph, rounded_product(ph.Cl, O.cs), fmin(0.0, muo));
+      const double us = fused(0.5, rounded_product(es, S.irho), S.prho);
+      const double uo = fused(0.5, rounded_product(eo, O.irho), O.prho);
+      const double C = rounded_product(ks, us) + rounded_product(ko, uo);
+      pdd[(size_t)k*ld + i] = C;
+      const double mC = O.m*C, w = O.m*ks;
+#pragma unroll
+      for (int c = 0; c < D; ++c) {
+        dvdt[c] -= mC*r[c];
+        const double wr = w*r[c];
+#pragma unroll
+        for (int b = 0; b < D; ++b) {
+          dvdx[b*D + c] -= dv[b]*wr;
+          // with isotropic H the gradient is parallel to r: M = sum m r (x) gradW is symmetric and
+          // only its upper triangle is summed
+          if (b <= c) M[b*D + c] -= r[b]*wr;
+        }
+      }
+      depsdt += w*vsr*us;
+      maxe = fmax(maxe, es);
+      m0 += fabs(grs);
+      if (FULL) {
+        rhosum += O.m*Ws;
+        nrm += S.m/S.rho*Ws;
+        effq += O.m*(S.rho*es)*Ws/O.rho;
+#pragma unroll
+        for (int c = 0; c < D; ++c) {
+          grho[c] += O.m*(O.rho - S.rho)*(ks*r[c]);
+          m1[c] -= fabs(grs)*(S.h*r[c]);
+        }
+      }
+    }
+  }
+  auto join = [&](double v) {
+    if (L >= 2) v += quad_swap<0xB1>(v);
+    if (L >= 4) v += quad_swap<0x4E>(v);
+    return v;
+  };
+  const int slot = threadIdx.x/L;
+  int q = 0;
+  auto put = [&](double v) {
+    v = join(v);
+    if (sub == 0) sums[q][slot] = v;
+    ++q;
+  };
+#pragma unroll
+  for (int a = 0; a < D; ++a) put(dvdt[a]);
+#pragma unroll
+  for (int a = 0; a < D*D; ++a) put(dvdx[a]);
+#pragma unroll
+  for (int a = 0; a < D; ++a)
+#pragma unroll
+    for (int b = a; b < D; ++b) put(M[a*D + b]);
+  put(depsdt);
+  put(m0);
+  {
+    double e = maxe;
+    if (L >= 2) e = fmax(e, quad_swap<0xB1>(e));
+    if (L >= 4) e = fmax(e, quad_swap<0x4E>(e));
+    if (sub == 0) sums[q][slot] = Srho*e;                // the largest rho^2 Q of the node
+    ++q;
+  }
+  if (FULL) {
+    put(rhosum);
+    put(nrm);
+    put(effq);
+#pragma unroll
+    for (int a = 0; a < D; ++a) { put(grho[a]); put(m1[a]); }
+  }
+  __syncthreads();
+  if ((int)threadIdx.x >= NB) return;
+  const int j = xcd_block()*NB + threadIdx.x;
+  if (j >= n) return;
+  SphSums<D> t;
+  q = 0;
+  auto get = [&] { return sums[q++][threadIdx.x]; };
+#pragma unroll
+  for (int a = 0; a < D; ++a) t.dvdt[a] = get();
+#pragma unroll
+  for (int a = 0; a < D*D; ++a) t.dvdx[a] = get();
+#pragma unroll
+  for (int a = 0; a < D; ++a)
+#pragma unroll
+    for (int b = a; b < D; ++b) t.M[a*D + b] = t.M[b*D + a] = get();
+  t.depsdt = get();
+  t.m0 = get();
+  t.maxq = get();
+  if (FULL) {
+    t.rhosum = get();
+    t.nrm = get();
+    t.effq = get();
+#pragma unroll
+    for (int a = 0; a < D; ++a) { t.grho[a] = get(); t.m1[a] = get(); }
+  }
+  sph_finalize<D, FULL>(f, ph, tab, j, f.cnt[j], t, sc);
+}
+
+// Lanes per node of the SPH pass.  The choice depends only on the configuration (dimension,
+// precision), never on the particle count, so a run gives the same bits in any batch.  FP64, us per
+// pass with 1 / 2 / 4 lanes: Sod 1-D 400 9.2 / 7.5 / 6.5, Noh 1-D 100 14.3 / 10.4 / 7.8, KH 2-D 65536
+// 71.9 / 46.7 / 41.5, Taylor-Green 37^3 56.4 / 39.8 / 41.8, 128^3 1451 / 1309 / 1385 (before, with two
+// sides' divisions, two reciprocal square roots and canonical-order selects per pair: 8.0, 10.6,
+// 53.8, 64 and 1406).  On large 3-D runs the pass is bound by the records' gathers: 96 bytes per
+// neighbour, 9 GB through the L1s of which most misses them.
+template <int D>
+constexpr int kSphLanes64 = D == 3 ? 2 : 4;
+constexpr int kSphLanesMixed = 2;
 template <int D, bool FULL, typename R, bool LQ = false>
 __global__ void __launch_bounds__(kBlock, 3) k_sph(Fields f, Geo g, Phys ph, DevTable tab, int n, int ldsTable,
                                                    const Scalars* sc) {
-  with_table<R>(tab, ldsTable, [&](auto coef) { sph_node<D, FULL, R, LQ>(f, g, ph, tab, coef, n, sc); });
+  if constexpr (sizeof(R) == sizeof(float)) {
+    with_table<float>(tab, ldsTable, [&](auto coef) { sph_node<D, FULL, LQ>(f, g, ph, tab, coef, n, sc); });
+  } else {
+    __shared__ double sums[sph_sums(D, FULL)][kBlock/kSphLanes64<D>];
+    auto body = [&](auto coef) { sph_node64<D, FULL, LQ, kSphLanes64<D>>(f, g, ph, tab, coef, n, sc, sums); };
+    if constexpr (FULL) with_table<double>(tab, ldsTable, body);
+    else with_gradient_table(tab, ldsTable, body);
+  }
 }
 
 // ---------------------------------------------------------------------------
