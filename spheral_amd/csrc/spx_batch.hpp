@@ -142,7 +142,8 @@ class Batch {
   uint32_t *vals = nullptr, *valsAlt = nullptr;
   void* sortTmp = nullptr;
   size_t sortTmpBytes = 0;
-  double* stage = nullptr;    // caller-order staging of one state component (updateState)
+  double* stage = nullptr;    // staging of Field records between the caller's layout and the arrays
+  int64_t stageCap = 0;       // its size in doubles
   int* cellStart = nullptr;
   int* cellEnd = nullptr;
   int64_t cellsAlloc = 0;
@@ -582,25 +583,95 @@ class Batch {
     }
   }
 
+  // ---------------------------------------------------------------- state transfer
+  // Room for up to `want` doubles of Field records, bounded: longer fields go in several pieces.
+  static constexpr int64_t kStageMax = (int64_t)1 << 21;
+  void ensureStage(int64_t want) {
+    want = std::min(want, kStageMax);
+    if (want <= stageCap) return;
+    HIP_CHECK(hipStreamSynchronize(stream));
+    dfree(stage);
+    stage = nullptr;
+    stageCap = 0;
+    stage = dalloc<double>((size_t)want);
+    stageCap = want;
+  }
+  static RecordSet records(std::initializer_list<double*> a) {
+    RecordSet s{};
+    for (double* p : a) s.a[s.nc++] = p;
+    return s;
+  }
+  RecordSet vectorRecords(double* const* v) const {
+    RecordSet s{};
+    for (int a = 0; a < D; ++a) s.a[s.nc++] = v[a];
+    return s;
+  }
+  // n records from the caller into the arrays' slots [slot0, slot0 + n): queued on the stream; the
+  // caller's memory is in use until the stream has been waited for.
+  void putRecords(const RecordSet& s, const double* src, const int64_t* oid, int64_t slot0, int64_t n) {
+    ensureStage(n*s.nc);
+    const int64_t per = std::max<int64_t>(1, stageCap/s.nc);
+    for (int64_t c0 = 0; c0 < n; c0 += per) {
+      const int64_t c1 = std::min(n, c0 + per);
+      HIP_CHECK(hipMemcpyAsync(stage, src + c0*s.nc, (size_t)((c1 - c0)*s.nc)*sizeof(double), hipMemcpyHostToDevice, stream));
+      hipLaunchKernelGGL(k_from_records, dim3(nblocks(n)), dim3(kBlock), 0, stream, s, (const double*)stage, oid, slot0, n,
+                         c0, c1);
+      HIP_CHECK(hipGetLastError());
+    }
+  }
+  void getRecords(const RecordSet& s, double* dst, int64_t slot0, int64_t n) {
+    ensureStage(n*s.nc);
+    const int64_t per = std::max<int64_t>(1, stageCap/s.nc);
+    for (int64_t c0 = 0; c0 < n; c0 += per) {
+      const int64_t c1 = std::min(n, c0 + per);
+      hipLaunchKernelGGL(k_to_records, dim3(nblocks(n)), dim3(kBlock), 0, stream, s, stage, (const int64_t*)f.oid, slot0, n,
+                         c0, c1);
+      HIP_CHECK(hipGetLastError());
+      download(dst + c0*s.nc, stage, (size_t)((c1 - c0)*s.nc)*sizeof(double));
+    }
+  }
+  // Position, velocity, mass, density, energy and h^-1 of n nodes; complete on return.
+  void putState(const double* x, const double* v, const double* m, const double* rho, const double* eps,
+                const double* hinv, const int64_t* oid, int64_t slot0, int64_t n) {
+    putRecords(vectorRecords(f.x), x, oid, slot0, n);
+    putRecords(vectorRecords(f.v), v, oid, slot0, n);
+    putRecords(records({f.m}), m, oid, slot0, n);
+    putRecords(records({f.rho}), rho, oid, slot0, n);
+    putRecords(records({f.eps}), eps, oid, slot0, n);
+    putRecords(records({f.hinv}), hinv, oid, slot0, n);
+    HIP_CHECK(hipStreamSynchronize(stream));
+  }
+  // The caller's state checked (H isotropic and positive, mass and density positive); returns h^-1.
+  std::vector<double> checkState(const double* m, const double* rho, const double* H, int64_t n) const {
+    std::vector<double> hinv((size_t)n);
+    bool ok = true;
+    for (int64_t i = 0; i < n; ++i) {
+      const double* Hi = H + i*D*D;
+      const double h = Hi[0];
+      bool iso = true;
+      for (int c = 0; c < D*D; ++c) iso &= Hi[c] == (c % (D + 1) == 0 ? h : 0.0);
+      ok &= iso & (h > 0.0) & (h <= 1.7976931348623157e308) & (m[i] > 0.0) & (rho[i] > 0.0);
+      hinv[i] = h;
+    }
+    if (ok) return hinv;
+    for (int64_t i = 0; i < n; ++i) {
+      const double* Hi = H + i*D*D;
+      for (int c = 0; c < D*D; ++c)
+        if (Hi[c] != (c % (D + 1) == 0 ? Hi[0] : 0.0))
+          raise(SPX_ERR_UNSUPPORTED, "H must be isotropic (h^-1 I); ASPH smoothing tensors are not implemented");
+      if (!(Hi[0] > 0.0) || !std::isfinite(Hi[0])) raise(SPX_ERR_ARG, "H must be positive definite");
+      if (!(m[i] > 0.0) || !(rho[i] > 0.0)) raise(SPX_ERR_ARG, "mass and mass density must be positive");
+    }
+    return hinv;
+  }
+
   // ---------------------------------------------------------------- run admission / retirement
   int addRun(const double* x, const double* v, const double* m, const double* rho, const double* eps, const double* H,
              int64_t n, double tEnd, int slot = -1) {
     if (!x || !v || !m || !rho || !eps || !H) raise(SPX_ERR_ARG, "null state pointer");
     if (n < 1) raise(SPX_ERR_ARG, "a run needs at least one node");
     if (!(tEnd >= 0.0)) raise(SPX_ERR_ARG, "end time must be >= 0");
-    // validate the whole input before touching the device
-    std::vector<double> hbuf((size_t)n);
-    for (int64_t i = 0; i < n; ++i) {
-      const double* Hi = H + i*D*D;
-      const double h = Hi[0];
-      for (int a = 0; a < D; ++a)
-        for (int b = 0; b < D; ++b)
-          if (Hi[a*D + b] != (a == b ? h : 0.0))
-            raise(SPX_ERR_UNSUPPORTED, "H must be isotropic (h^-1 I); ASPH smoothing tensors are not implemented");
-      if (!(h > 0.0) || !std::isfinite(h)) raise(SPX_ERR_ARG, "H must be positive definite");
-      if (!(m[i] > 0.0) || !(rho[i] > 0.0)) raise(SPX_ERR_ARG, "mass and mass density must be positive");
-      hbuf[i] = h;
-    }
+    std::vector<double> hbuf = checkState(m, rho, H, n);   // the whole input, before touching the device
     bool anyRemoved = false;
     for (auto& r : runs) anyRemoved |= r.state == RUN_REMOVED;
     if (slot < 0) {
@@ -618,32 +689,22 @@ class Batch {
     if (nTotal + n > cap) raise(SPX_ERR_CAPACITY, "particle capacity of the batch exceeded");
     HIP_CHECK(hipStreamSynchronize(stream));
     const int64_t o = nTotal;
-    std::vector<double> buf((size_t)n);
-    auto up = [&](double* dst, const double* src) { upload(dst + o, src, n*sizeof(double)); };
-    auto zero = [&](double* dst) { HIP_CHECK(hipMemsetAsync(dst + o, 0, n*sizeof(double), stream)); };
-    for (int a = 0; a < D; ++a) {
-      for (int64_t i = 0; i < n; ++i) buf[i] = x[i*D + a];
-      up(f.x[a], buf.data());
-      for (int64_t i = 0; i < n; ++i) buf[i] = v[i*D + a];
-      up(f.v[a], buf.data());
-      zero(f.DxDt[a]); zero(f.DvDt[a]); zero(f.DvDtG[a]);
-    }
-    up(f.hinv, hbuf.data());
-    up(f.m, m);
-    up(f.rho, rho);
-    up(f.eps, eps);
-    for (int64_t i = 0; i < n; ++i) buf[i] = 1.0;
-    up(f.omega, buf.data());
-    // derivatives start at zero (SPHBase::initializeProblemStartup)
-    for (double* p : {f.DepsDt, f.DrhoDt, f.DHDt, f.maxQ, f.pot, f.potS, f.P, f.cs}) zero(p);
-    for (int c = 0; c < D*D; ++c) HIP_CHECK(hipMemsetAsync(f.DvDx + (size_t)c*ld + o, 0, n*sizeof(double), stream));
+    const int nb = nblocks(n);
+    hipLaunchKernelGGL(k_new_ids, dim3(nb), dim3(kBlock), 0, stream, f.oid, f.run, o, n, slot);
+    // derivatives start at zero (SPHBase::initializeProblemStartup), Omega at one
+    FillSet z{};
+    for (int a = 0; a < D; ++a)
+      for (double* p : {f.DxDt[a], f.DvDt[a], f.DvDtG[a]}) z.a[z.count++] = p;
+    for (double* p : {f.DepsDt, f.DrhoDt, f.DHDt, f.maxQ, f.pot, f.potS, f.P, f.cs}) z.a[z.count++] = p;
+    for (int c = 0; c < D*D; ++c) z.a[z.count++] = f.DvDx + (size_t)c*ld;
     if (limitedQ())
-      for (int c = 0; c < D*D; ++c) HIP_CHECK(hipMemsetAsync(f.DvDxQ + (size_t)c*ld + o, 0, n*sizeof(double), stream));
-    std::vector<int64_t> ids(n);
-    std::vector<int32_t> rr(n, slot);
-    for (int64_t i = 0; i < n; ++i) ids[i] = ((int64_t)slot << 40) | i;
-    upload(f.oid + o, ids.data(), n*sizeof(int64_t));
-    upload(f.run + o, rr.data(), n*sizeof(int32_t));
+      for (int c = 0; c < D*D; ++c) z.a[z.count++] = f.DvDxQ + (size_t)c*ld;
+    hipLaunchKernelGGL(k_fill, dim3(nb), dim3(kBlock), 0, stream, z, o, n, 0.0);
+    FillSet one{};
+    one.a[one.count++] = f.omega;
+    hipLaunchKernelGGL(k_fill, dim3(nb), dim3(kBlock), 0, stream, one, o, n, 1.0);
+    HIP_CHECK(hipGetLastError());
+    putState(x, v, m, rho, eps, hbuf.data(), nullptr, o, n);
     RunInfo info;
     info.state = RUN_ACTIVE;
     info.n = n;
@@ -1961,36 +2022,8 @@ class Batch {
     if (!initialized) raise(SPX_ERR_STATE, "spx_run_initialize must be called first");
     if (!x || !v || !m || !rho || !eps || !H) raise(SPX_ERR_ARG, "null argument");
     const int64_t n = runs[0].n;
-    std::vector<double> hbuf((size_t)n);
-    for (int64_t i = 0; i < n; ++i) {
-      const double* Hi = H + i*D*D;
-      const double h = Hi[0];
-      for (int a = 0; a < D; ++a)
-        for (int b = 0; b < D; ++b)
-          if (Hi[a*D + b] != (a == b ? h : 0.0))
-            raise(SPX_ERR_UNSUPPORTED, "H must be isotropic (h^-1 I); ASPH smoothing tensors are not implemented");
-      if (!(h > 0.0) || !std::isfinite(h)) raise(SPX_ERR_ARG, "H must be positive definite");
-      if (!(m[i] > 0.0) || !(rho[i] > 0.0)) raise(SPX_ERR_ARG, "mass and mass density must be positive");
-      hbuf[i] = h;
-    }
-    if (!stage) stage = dalloc<double>(ld);
-    std::vector<double> buf((size_t)n);
-    auto put = [&](double* dst, const double* src) {
-      upload(stage, src, n*sizeof(double));
-      hipLaunchKernelGGL(k_from_local, dim3(nblocks(n)), dim3(kBlock), 0, stream, dst, (const double*)stage,
-                         (const int64_t*)f.oid, (int)n);
-      HIP_CHECK(hipGetLastError());
-    };
-    for (int a = 0; a < D; ++a) {
-      for (int64_t i = 0; i < n; ++i) buf[i] = x[i*D + a];
-      put(f.x[a], buf.data());
-      for (int64_t i = 0; i < n; ++i) buf[i] = v[i*D + a];
-      put(f.v[a], buf.data());
-    }
-    put(f.m, m);
-    put(f.rho, rho);
-    put(f.eps, eps);
-    put(f.hinv, hbuf.data());
+    const std::vector<double> hbuf = checkState(m, rho, H, n);
+    putState(x, v, m, rho, eps, hbuf.data(), f.oid, runs[0].offset, n);
     eos();
     HIP_CHECK(hipStreamSynchronize(stream));
     runs[0].candValid = false;
@@ -2115,41 +2148,24 @@ class Batch {
     auto needFull = [&] {
       if (!ri.fullOut) raise(SPX_ERR_STATE, "'" + name + "' is produced by spx_run_evaluate_derivatives only");
     };
-    std::vector<int64_t> local, slots;
-    runSlots(slot, local, slots);
     const int64_t n = ri.n;
-    // the run's segment of an array: tmp[k] is slot slots[k] = offset + k
-    std::vector<double> tmp(n);
-    auto dl = [&](const double* src) { if (n) download(tmp.data(), src + ri.offset, n*sizeof(double)); };
-    auto scalar = [&](const double* src) -> int64_t {
-      if (capacity < n) raise(SPX_ERR_ARG, "output capacity too small");
-      dl(src);
-      for (size_t k = 0; k < slots.size(); ++k) out[local[k]] = tmp[k];
-      return n;
+    auto read = [&](const RecordSet& q) -> int64_t {
+      if (capacity < n*q.nc) raise(SPX_ERR_ARG, "output capacity too small");
+      getRecords(q, out, ri.offset, n);
+      return n*q.nc;
     };
-    auto vec = [&](double* const* src) -> int64_t {
-      if (capacity < n*D) raise(SPX_ERR_ARG, "output capacity too small");
-      for (int a = 0; a < D; ++a) {
-        dl(src[a]);
-        for (size_t k = 0; k < slots.size(); ++k) out[local[k]*D + a] = tmp[k];
-      }
-      return n*D;
+    auto scalar = [&](double* src) { return read(records({src})); };
+    auto vec = [&](double* const* src) { return read(vectorRecords(src)); };
+    auto ten = [&](double* src) {
+      RecordSet q{};
+      for (int c = 0; c < D*D; ++c) q.a[q.nc++] = src + (size_t)c*ld;
+      return read(q);
     };
-    auto ten = [&](const double* src) -> int64_t {
-      if (capacity < n*D*D) raise(SPX_ERR_ARG, "output capacity too small");
-      for (int c = 0; c < D*D; ++c) {
-        dl(src + (size_t)c*ld);
-        for (size_t k = 0; k < slots.size(); ++k) out[local[k]*D*D + c] = tmp[k];
-      }
-      return n*D*D;
-    };
-    auto iso = [&](const double* src) -> int64_t {
-      if (capacity < n*D*D) raise(SPX_ERR_ARG, "output capacity too small");
-      dl(src);
-      for (size_t k = 0; k < slots.size(); ++k)
-        for (int a = 0; a < D; ++a)
-          for (int b = 0; b < D; ++b) out[local[k]*D*D + a*D + b] = a == b ? tmp[k] : 0.0;
-      return n*D*D;
+    auto iso = [&](double* src) {
+      RecordSet q = records({src});
+      q.nc = D*D;
+      q.iso = D;
+      return read(q);
     };
     if (name == "position") return vec(f.x);
     if (name == "velocity") return vec(f.v);

@@ -106,12 +106,59 @@ __global__ void __launch_bounds__(kBlock) k_gather(GatherSet s, const uint32_t* 
   const uint32_t q = perm[p];
   for (int k = 0; k < s.count; ++k) s.dst[k][p] = s.src[k][q];
 }
-// Values given in a run's own node order into the engine's current particle order: slot p
-// holds node (oid[p] & low 40 bits) of its run.
-__global__ void __launch_bounds__(kBlock) k_from_local(double* __restrict__ dst, const double* __restrict__ src,
-                                                       const int64_t* __restrict__ oid, int n) {
-  const int p = blockIdx.x*blockDim.x + threadIdx.x;
-  if (p < n) dst[p] = src[oid[p] & (((int64_t)1 << 40) - 1)];
+// State transfer between the engine's arrays (one per component, particle order) and the boundary's
+// Field records (NC doubles per node, the run's node order), through a staging buffer that holds the
+// records of nodes [c0, c1): one strided pass on the device and one copy per field instead of a copy
+// and a host loop per component.  Slot p holds node (oid[p] & low 40 bits); oid null: node p - slot0.
+struct RecordSet {
+  double* a[9];
+  int nc;          // components per record
+  int iso;         // > 0: the record is a[0] times the iso x iso identity (NC = iso^2)
+};
+__device__ __forceinline__ int64_t node_of(const int64_t* oid, int64_t slot0, int64_t k) {
+  return oid ? oid[slot0 + k] & (((int64_t)1 << 40) - 1) : k;
+}
+__global__ void __launch_bounds__(kBlock) k_to_records(RecordSet s, double* __restrict__ stage,
+                                                       const int64_t* __restrict__ oid, int64_t slot0, int64_t n,
+                                                       int64_t c0, int64_t c1) {
+  const int64_t k = (int64_t)blockIdx.x*blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const int64_t node = node_of(oid, slot0, k);
+  if (node < c0 || node >= c1) return;
+  double* out = stage + (node - c0)*s.nc;
+  if (s.iso) {
+    const double h = s.a[0][slot0 + k];
+    for (int c = 0; c < s.nc; ++c) out[c] = c % (s.iso + 1) == 0 ? h : 0.0;
+  } else {
+    for (int c = 0; c < s.nc; ++c) out[c] = s.a[c][slot0 + k];
+  }
+}
+__global__ void __launch_bounds__(kBlock) k_from_records(RecordSet s, const double* __restrict__ stage,
+                                                         const int64_t* __restrict__ oid, int64_t slot0, int64_t n,
+                                                         int64_t c0, int64_t c1) {
+  const int64_t k = (int64_t)blockIdx.x*blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const int64_t node = node_of(oid, slot0, k);
+  if (node < c0 || node >= c1) return;
+  const double* in = stage + (node - c0)*s.nc;
+  for (int c = 0; c < s.nc; ++c) s.a[c][slot0 + k] = in[c];
+}
+// Ids and run slots of a newly admitted run's nodes, at the slots from slot0.
+__global__ void __launch_bounds__(kBlock) k_new_ids(int64_t* oid, int32_t* run, int64_t slot0, int64_t n, int slot) {
+  const int64_t k = (int64_t)blockIdx.x*blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  oid[slot0 + k] = ((int64_t)slot << 40) | k;
+  run[slot0 + k] = slot;
+}
+// a[c][slot0 .. slot0 + n) = value for each of the set's arrays.
+struct FillSet {
+  double* a[40];
+  int count;
+};
+__global__ void __launch_bounds__(kBlock) k_fill(FillSet s, int64_t slot0, int64_t n, double value) {
+  const int64_t k = (int64_t)blockIdx.x*blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  for (int c = 0; c < s.count; ++c) s.a[c][slot0 + k] = value;
 }
 __global__ void __launch_bounds__(kBlock) k_gather_ids(const int64_t* src, int64_t* dst, const int32_t* rsrc, int32_t* rdst,
                                                        const uint32_t* perm, int n) {
