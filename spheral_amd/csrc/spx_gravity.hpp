@@ -187,77 +187,81 @@ __global__ void __launch_bounds__(kBlock) k_tree_gather(double* const* xs, const
   tp[2*(size_t)p + 1] = make_double2(z, mq);
 }
 
-// A cell as the walk reads it: one 64-byte record, (x, y), (z, M) of the centre of mass, the
-// opening radius^2 l^2/theta^2 + |xcm - centre|^2 for the walk's opening angle, and (first,
-// last, skip, level) -- one cache line per visited cell instead of one per array.
-struct alignas(64) TreeCell {
+// A cell as the walk reads it, in one record: the centre of mass, the mass, the opening radius^2
+// l^2/theta^2 + |xcm - centre|^2 for the walk's opening angle, the next cell behind its subtree,
+// and what a point too close for the monopole does with it: open it (kCellOpen), take its one
+// point (kCellPoint) or, at the deepest level, take its list of points (kCellList).
+enum : int { kCellOpen = 0, kCellPoint = 1, kCellList = 2 };
+struct alignas(16) TreeCell {
   double x, y, z, M;
-  double open, pad;
-  int first, last, skip, level;
+  double open;
+  int skip, kind;
 };
-static_assert(sizeof(TreeCell) == 64, "TreeCell is one 64-byte record");
+static_assert(sizeof(TreeCell) == 48, "TreeCell is read as three 16-byte words");
 
-__global__ void __launch_bounds__(kBlock) k_tree_pack(TreeView v, const double* cs2, double open2, TreeCell* cells) {
+__global__ void __launch_bounds__(kBlock) k_tree_pack(TreeView v, const double* cs2, double open2, double self2,
+                                                      TreeCell* cells) {
   const int c = blockIdx.x*blockDim.x + threadIdx.x;
-  if (c >= v.ncells) return;
-  const int lvl = v.level[c];
-  TreeCell t;
-  t.x = v.cx[0][c];
-  t.y = v.cx[1][c];
-  t.z = v.cx[2][c];
-  t.M = v.M[c];
-  t.open = cs2[lvl]/open2 + v.rc2[c];
-  t.pad = 0.0;
-  t.first = v.first[c];
-  t.last = v.last[c];
-  t.skip = v.skip[c];
-  t.level = lvl;
+  if (c > v.ncells) return;
+  TreeCell t{0.0, 0.0, 0.0, 0.0, INFINITY, v.ncells, kCellPoint};     // behind the last cell: nothing acts
+  if (c < v.ncells) {
+    const int lvl = v.level[c];
+    t.x = v.cx[0][c];
+    t.y = v.cx[1][c];
+    t.z = v.cx[2][c];
+    t.M = v.M[c];
+    t.open = cs2[lvl]/open2 + v.rc2[c];
+    t.skip = v.skip[c];
+    // A one-point cell acts through its monopole from its opening radius on and as its point down
+    // to the self screen, by the same formula: one radius.  (Below 1e-100 the formulas differ, and
+    // such a cell keeps both, the point in a list of one.)
+    const bool one = v.first[c] == v.last[c];
+    t.kind = one && t.open >= 1.0e-100 ? kCellPoint : one || lvl == kTreeBits ? kCellList : kCellOpen;
+    if (t.kind == kCellPoint) t.open = fmin(t.open, self2);
+  }
   cells[c] = t;
 }
 
-// Lanes that walk the tree together (64: the wavefront; 16, 8, 4: aligned lane groups).
-// Measured on the Evrard collapse (250k points) with the cells read as separate arrays: 64 ->
-// 5.0 ms per walk, 16 -> 4.15, 8 -> 3.99, 4 -> 4.69; with the packed cell records (gravity per
-// step over 60 steps from the start): 16 -> 2.16 ms, 8 -> 1.99, 4 -> 1.86, 2 -> 1.92, 1 -> 2.14;
-// with single-point leaves taken through the monopole path (one branch, no point-record read):
-// 8 -> 1.72 ms, 4 -> 1.59, 2 -> 1.60.  Same bits for every group size.
+// Neighbouring points that walk the tree together.  In a group of four a wavefront reads 16 records
+// per step instead of 64 but visits the cells that any of the four needs (21 to 42 % more steps
+// than a point by itself).  With many wavefronts per SIMD the reads count, with few the number of
+// dependent steps.  Evrard collapse, per walk with 1 / 2 / 4 together: 16k points 312 / 386 / 428 us,
+// 60k 371 / 476 / 550, 120k 665 / 620 / 665, 250k 1293 / 1055 / 928; uniform sphere of 33k with a
+// wide opening angle 69 / 102 / 115.  The line is at 1.5 wavefronts per SIMD.  Same bits either way.
 constexpr int kTreeGroup = 4;
+constexpr int kTreeAlone = 98304;
 
-// Device-library wavefront minimum (DPP lane exchanges, no LDS round trip).
-extern "C" __device__ int __ockl_wfred_min_i32(int);
-
-// Minimum over each aligned group of GROUP (4, 8 or 16) lanes by DPP lane exchanges; every
-// lane of the group ends with the group's minimum.  Quad permutes [1,0,3,2] and [2,3,0,1]
-// combine the lanes of a quad, the half-row mirror (lane l <-> 7 - l within 8) pairs the two
-// quads of a half-row, the row mirror (l <-> 15 - l within 16) the two halves of a row.
+// Minimum over a point by itself or over each quad of lanes (quad permutes [1,0,3,2], [2,3,0,1]).
 template <int GROUP>
 __device__ __forceinline__ int group_min(int v) {
-  v = min(v, __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, false));
-  v = min(v, __builtin_amdgcn_mov_dpp(v, 0x4E, 0xf, 0xf, false));
-  if (GROUP >= 8) v = min(v, __builtin_amdgcn_mov_dpp(v, 0x141, 0xf, 0xf, false));
-  if (GROUP >= 16) v = min(v, __builtin_amdgcn_mov_dpp(v, 0x140, 0xf, 0xf, false));
+  static_assert(GROUP == 1 || GROUP == 4);
+  if (GROUP == 4) {
+    v = min(v, __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true));
+    v = min(v, __builtin_amdgcn_mov_dpp(v, 0x4E, 0xf, 0xf, true));
+  }
   return v;
 }
 
 // applyTreeForces for the point in tree slot p; results scattered to its hydro slot.
-// The wavefront walks the pre-order cells together: each lane keeps the next cell its own
-// walk would visit, the wavefront visits the smallest of them, and only the lanes waiting
-// on that cell act on it.  Every lane therefore takes exactly the decisions, in exactly the
-// order, of an independent stackless walk (same bits).  The visited cell is wavefront-
-// uniform (readfirstlane), so its data and its leaf points are read through the scalar
-// cache; the tree arrays come as separate restrict-qualified arguments, which tells the
-// compiler they are not written here.  GROUP 16: each row of 16 lanes walks together instead
-// of the whole wavefront (the walks of 16 neighbouring points differ less than those of 64, so
-// fewer cells are visited), with per-group cell reads (64/GROUP addresses per instruction);
-// 8 and 4 likewise.  COUNT (a measurement variant, never in a step): also counts each point's
+// GROUP neighbouring points walk the pre-order cells together: each lane keeps the next cell its
+// own walk would visit, the group visits the smallest of them, and only the lanes waiting on that
+// cell act on it.  Every lane therefore takes exactly the decisions, in exactly the order, of an
+// independent stackless walk (same bits).  A wavefront walks 64/GROUP groups side by side.
+//
+// Bound by the vector instructions of a step (58 per visited cell) while wavefronts are plenty and
+// by a step's chain -- read a record, compare, choose the next -- where they are not.  So the next
+// record is requested before the force of the present one is formed, the record is 48 bytes, and
+// the decision is one comparison: the self screen's division became a radius, and a one-point
+// cell's two radii one (k_tree_pack).  250k Evrard 1591 -> 928 us per walk, 33k sphere 202 -> 69
+// (with the point by itself).  COUNT (a measurement variant, never in a step): counts each point's
 // monopole (accepted cell) and point-point interactions into counts[2p], counts[2p+1].
 template <int GROUP, bool COUNT = false, int DIM = 3>
 __global__ void __launch_bounds__(kBlock) k_tree_walk(
     const double* __restrict__ tx0, const double* __restrict__ tx1, const double* __restrict__ tx2,
-    const double2* __restrict__ tp, const TreeCell* __restrict__ cells, int ncells, int npts,
-    const uint32_t* __restrict__ perm, double soft2, double soft, double G, double* __restrict__ acc0,
-    double* __restrict__ acc1, double* __restrict__ acc2, double* __restrict__ pot, double* __restrict__ blockMin,
-    unsigned long long* __restrict__ counts = nullptr) {
+    const double2* __restrict__ tp, const TreeCell* __restrict__ cells, const int* __restrict__ first,
+    const int* __restrict__ last, int ncells, int npts, const uint32_t* __restrict__ perm, double soft2, double self2,
+    double soft, double G, double* __restrict__ acc0, double* __restrict__ acc1, double* __restrict__ acc2,
+    double* __restrict__ pot, double* __restrict__ blockMin, unsigned long long* __restrict__ counts = nullptr) {
   const int p = blockIdx.x*blockDim.x + threadIdx.x;
   unsigned long long nCell = 0, nPoint = 0;
   const bool valid = p < npts;
@@ -266,73 +270,71 @@ __global__ void __launch_bounds__(kBlock) k_tree_walk(
   if (valid) { xi = tx0[p]; yi = tx1[p]; zi = tx2[p]; }
   double ax = 0.0, ay = 0.0, az = 0.0, phi = 0.0;
   int next = valid ? 1 : ncells;
+  int c = group_min<GROUP>(next);
+  const double2* cr = reinterpret_cast<const double2*>(cells + c);
+  double2 c01 = cr[0], c23 = cr[1], c45 = cr[2];
   // every iteration moves the group's smallest pending cell strictly forward, so a walk
   // ends within ncells iterations; the bound only guards the loop
   for (int guard = 0; guard <= ncells; ++guard) {
-    int c;
-    if (GROUP == 64) {
-      c = __builtin_amdgcn_readfirstlane(__ockl_wfred_min_i32(next));
-      if (c >= ncells) break;                     // every lane of the wavefront is done
-    } else {
-      c = group_min<GROUP>(next);
-      if (__all(c >= ncells)) break;              // every group is done
-      if (c >= ncells) continue;                  // this group is done
-    }
-    // the cell's record, read at one address per group
-    const double2* cr = reinterpret_cast<const double2*>(cells + c);
-    const double2 c01 = cr[0], c23 = cr[1], co = cr[2];
-    const int4 ci = *reinterpret_cast<const int4*>(cr + 3);
-    const double ccx = c01.x, ccy = c01.y, ccz = c23.x, Mc = c23.y, open = co.x;
-    const int q0 = ci.x, q1 = ci.y, sk = ci.z, lvl = ci.w;
-    if (next != c) continue;
-    const double dx = ccx - xi, dy = ccy - yi, dz = ccz - zi;
-    const double r2 = dx*dx + dy*dy + dz*dz;
-    // An accepted cell acts through its monopole.  A single-point leaf acts as its point, and
-    // its record already holds that point: the monopole pass copies a one-point cell's x and m
-    // unchanged (no m*x/m round trip), so (ccx, ccy, ccz, Mc) are the point's own values and
-    // the point-point term below is the monopole formula with the point's softening guard.
-    // One code path for both: no second, dependent read of the point record, and lanes of a
-    // wavefront at accepted cells and at single-point leaves no longer run two branches (gravity
-    // 1.86 -> 1.59 ms per step on the 250k Evrard collapse; results move at roundoff, 7e-15 in
-    // density after 65 steps, as the compiler contracts the merged arithmetic differently).
-    const bool mono = r2 > open;
-    const bool single = !mono && q0 == q1;
-    if (mono || (single && r2/soft2 > 1.0e-10)) {
+    const double Mc = c23.y;
+    const int sk = __double2loint(c45.y), kind = __double2hiint(c45.y);
+    const double dx = c01.x - xi, dy = c01.y - yi, dz = c23.x - zi;
+    const double r2 = fused(dz, dz, fused(dy, dy, rounded_product(dx, dx)));
+    const bool mine = next == c;
+    const bool acts = mine && r2 > c45.x;
+    const bool list = mine && !acts && kind == kCellList;
+    const int own = c;
+    if (mine) next = acts || kind != kCellOpen ? sk : c + 1;
+    // The next cell's record is on its way while this one's force is formed.  A group that is
+    // done stays at the record behind the last cell, on which nothing acts.
+    c = group_min<GROUP>(next);
+    cr = reinterpret_cast<const double2*>(cells + c);
+    c01 = cr[0];
+    c23 = cr[1];
+    c45 = cr[2];
+    if (acts) {
       // 1/|r| and 1/sqrt(r^2 + s^2) from reciprocal square roots (the force is M/(r^2 + s^2) along
-      // r/|r|, the potential -M/sqrt(r^2 + s^2)): 11 % faster than two square roots and three
-      // divisions on the 250k Evrard walk, results within 2e-16 (L1 of density after 65 steps)
-      const bool far = single || r2 > 1.0e-100;
-      const double inv = far ? rsqrt(r2) : 0.0;
-      const double nx = far ? dx*inv : 1.0, ny = dy*inv, nz = dz*inv;
+      // r/|r|, the potential -M/sqrt(r^2 + s^2)).
       const double rs = r2 + soft2;
-      const double ri = rsqrt(rs);
+      double inv = fast_rsqrt(r2), ri = fast_rsqrt(rs);
+      double nx = dx*inv, ny = dy*inv, nz = dz*inv;
+      if (!(r2 > 1.0e-100 && rs < 1.0e300)) {      // coincident with the cell, or out of the estimate's range
+        const bool far = kind == kCellPoint || r2 > 1.0e-100;
+        inv = far ? rsqrt(r2) : 0.0;
+        ri = rsqrt(rs);
+        nx = far ? dx*inv : 1.0;
+        ny = dy*inv;
+        nz = dz*inv;
+      }
       const double f = DIM == 3 ? Mc*(ri*ri) : Mc*ri;
-      ax += f*nx; ay += f*ny; az += f*nz;
-      phi -= DIM == 3 ? Mc*ri : Mc*(0.5*log(rs));
-      if (COUNT) { if (mono) ++nCell; else ++nPoint; }
+      ax = fused(f, nx, ax);
+      ay = fused(f, ny, ay);
+      az = fused(f, nz, az);
+      phi = DIM == 3 ? fused(-Mc, ri, phi) : phi - Mc*(0.5*log(rs));
+      if (COUNT) ++nCell;
     }
-    if (mono || single) {
-      next = sk;
-    } else if (lvl == kTreeBits) {
-      for (int q = q0; q <= q1; ++q) {
+    if (COUNT && mine && !acts && kind == kCellPoint && r2 > self2) ++nPoint;
+    if (list) {
+      const int q1 = last[own];
+      for (int q = first[own]; q <= q1; ++q) {
         const double2 pa = tp[2*(size_t)q], pb = tp[2*(size_t)q + 1];
         const double ex = pa.x - xi, ey = pa.y - yi, ez = pb.x - zi;
-        const double q2 = ex*ex + ey*ey + ez*ez;
-        if (q2/soft2 > 1.0e-10) {
+        const double q2 = fused(ez, ez, fused(ex, ex, rounded_product(ey, ey)));
+        if (q2 > self2) {
           const double inv = rsqrt(q2);
           const double rs = q2 + soft2;
           const double mq = pb.y;
           const double ri = rsqrt(rs);
           const double f = DIM == 3 ? mq*(ri*ri) : mq*ri;
-          ax += f*(ex*inv); ay += f*(ey*inv); az += f*(ez*inv);
-          phi -= DIM == 3 ? mq*ri : mq*(0.5*log(rs));
+          ax = fused(f, ex*inv, ax);
+          ay = fused(f, ey*inv, ay);
+          az = fused(f, ez*inv, az);
+          phi = DIM == 3 ? fused(-mq, ri, phi) : phi - mq*(0.5*log(rs));
           if (COUNT) ++nPoint;
         }
       }
-      next = sk;
-    } else {
-      next = c + 1;
     }
+    if (__all(c >= ncells)) break;               // every group is done
   }
   if (valid) {
     const double amag = sqrt(ax*ax + ay*ay + az*az);
@@ -383,7 +385,8 @@ class GravityTree {
   double *tx[3] = {nullptr, nullptr, nullptr}, *tm = nullptr;
   double2* tp = nullptr;            // tree-order (x, y), (z, m) records of the walk's leaves
   TreeCell* cells = nullptr;        // the walk's cell records
-  double packedOpen2 = -1.0;        // opening^2 the cell records were packed for (< 0: stale)
+  // opening^2 (< 0: stale) and self-screen radius^2 that the cell records were packed for
+  double packedOpen2 = -1.0, packedSelf2 = 0.0;
   int *nheads = nullptr, *cstart = nullptr;
   unsigned char* lstart = nullptr;
   void* tmp = nullptr;
@@ -499,7 +502,7 @@ class GravityTree {
     HIP_CHECK(hipMemcpyAsync(&total, cstart + nn, sizeof(int), hipMemcpyDeviceToHost, stream));
     HIP_CHECK(hipStreamSynchronize(stream));
     ncells = total;
-    ensureCells(total);
+    ensureCells((int64_t)total + 1);                // and the record behind the last cell
     hipLaunchKernelGGL(k_tree_cells, dim3(nb), dim3(kBlock), 0, stream, codesSorted, nn, cstart, nheads, lstart, total,
                        first, last, skip, level);
     HIP_CHECK(hipGetLastError());
@@ -523,24 +526,39 @@ class GravityTree {
     HIP_CHECK(hipStreamSynchronize(stream));
   }
 
+  // The largest r^2 that the softening's self screen r^2/soft^2 > 1e-10 excludes: the quotient is
+  // monotone in r^2, so the walk compares r^2 with it instead of dividing at every visited leaf.
+  static double selfRadius2(double soft2) {
+    auto counts = [soft2](double r2) { return r2/soft2 > 1.0e-10; };
+    if (!(soft2 < INFINITY)) return INFINITY;       // nothing counts
+    double r = 1.0e-10*soft2;
+    while (r > 0.0 && counts(r)) r = std::nextafter(r, 0.0);
+    while (!counts(std::nextafter(r, INFINITY))) r = std::nextafter(r, INFINITY);
+    return r;
+  }
+
   // The walk's cell records for this opening angle (once per tree and angle).
-  void pack(double opening) {
+  void pack(double opening, double self2) {
     const double open2 = opening*opening;
-    if (packedOpen2 == open2) return;
-    const int cb = (int)((view.ncells + kBlock - 1)/kBlock);
-    hipLaunchKernelGGL(k_tree_pack, dim3(std::max(cb, 1)), dim3(kBlock), 0, stream, view, (const double*)cs2, open2, cells);
+    if (packedOpen2 == open2 && packedSelf2 == self2) return;
+    const int cb = view.ncells/kBlock + 1;          // one record more than there are cells
+    hipLaunchKernelGGL(k_tree_pack, dim3(cb), dim3(kBlock), 0, stream, view, (const double*)cs2, open2, self2, cells);
     HIP_CHECK(hipGetLastError());
     packedOpen2 = open2;
+    packedSelf2 = self2;
   }
 
   void evaluate(double* const* acc, double* pot, int nn, double G, double soft, double opening, Scalars* sc,
                 double ftimestep) {
     const int nb = (int)((nn + kBlock - 1)/kBlock);
     double* az = D == 3 ? acc[2] : sink;
-    pack(opening);
-    auto walk = D == 3 ? k_tree_walk<kTreeGroup, false, 3> : k_tree_walk<kTreeGroup, false, 2>;
+    const double self2 = selfRadius2(soft*soft);
+    pack(opening, self2);
+    auto walk = nn <= kTreeAlone ? (D == 3 ? k_tree_walk<1, false, 3> : k_tree_walk<1, false, 2>)
+                                 : (D == 3 ? k_tree_walk<kTreeGroup, false, 3> : k_tree_walk<kTreeGroup, false, 2>);
     hipLaunchKernelGGL(walk, dim3(nb), dim3(kBlock), 0, stream, view.tx[0], view.tx[1], view.tx[2], (const double2*)tp,
-                       (const TreeCell*)cells, view.ncells, view.n, (const uint32_t*)perm, soft*soft, soft, G,
+                       (const TreeCell*)cells, view.first, view.last, view.ncells, view.n, (const uint32_t*)perm, soft*soft,
+                       self2, soft, G,
                        acc[0], acc[1], az, pot, part, (unsigned long long*)nullptr);
     hipLaunchKernelGGL(k_tree_dt, dim3(1), dim3(kBlock), 0, stream, part, nb, sc, G, ftimestep);
     HIP_CHECK(hipGetLastError());
@@ -558,10 +576,11 @@ class GravityTree {
     HIP_CHECK(hipMalloc(&scratch, (size_t)(4*(size_t)std::max(nn, 1) + nb)*sizeof(double)));
     HIP_CHECK(hipMalloc(&counts, 2*(size_t)std::max(nn, 1)*sizeof(unsigned long long)));
     double* a = scratch;
-    pack(opening);
+    pack(opening, INFINITY);          // one-point cells keep their opening radius: told apart from points
     auto walk = D == 3 ? k_tree_walk<kTreeGroup, true, 3> : k_tree_walk<kTreeGroup, true, 2>;
     hipLaunchKernelGGL(walk, dim3(nb), dim3(kBlock), 0, stream, view.tx[0], view.tx[1], view.tx[2], (const double2*)tp,
-                       (const TreeCell*)cells, view.ncells, view.n, (const uint32_t*)perm, soft*soft, soft, 1.0, a, a + nn,
+                       (const TreeCell*)cells, view.first, view.last, view.ncells, view.n, (const uint32_t*)perm, soft*soft,
+                       selfRadius2(soft*soft), soft, 1.0, a, a + nn,
                        a + 2*(size_t)nn, a + 3*(size_t)nn, a + 4*(size_t)nn, counts);
     const hipError_t e = hipGetLastError();
     std::vector<unsigned long long> h(2*(size_t)nn);
