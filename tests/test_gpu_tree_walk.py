@@ -13,13 +13,14 @@ ALONE = 98304          # largest count whose points walk by themselves
 SOFT = 0.01
 
 
-def evaluate(gpu, x, m, opening):
+def evaluate(gpu, x, m, opening, hinv=None):
     n, dim = x.shape
+    hinv = hinv or n**(1.0/dim)
     cfg = abi.default_config(dim, nperh=2.01)
     cfg.integrator = abi.SPX_INTEGRATOR_SYNCHRONOUS_RK2
     cfg.gravity = cfg.gravity_only = 1
     cfg.G, cfg.softening, cfg.opening, cfg.ftimestep = 1.0, SOFT, opening, 0.1
-    H = np.broadcast_to(np.eye(dim)*n**(1.0/dim), (n, dim, dim)).copy()
+    H = np.broadcast_to(np.eye(dim)*hinv, (n, dim, dim)).copy()
     r = gpu.make_run(cfg, dict(x=x, v=np.zeros((n, dim)), m=m, rho=np.ones(n), eps=np.zeros(n), H=H))
     r.initialize()
     r.evaluate_derivatives()
@@ -69,3 +70,62 @@ def test_opened_walk_is_the_direct_sum(gpu, dim, n):
         size, psize = f.sum(1).cpu().numpy(), pot.abs().sum(1).cpu().numpy()
         assert np.all(np.abs(a[i0:i0 + 1024] - acc) <= eps*size[:, None])
         assert np.all(np.abs(p[i0:i0 + 1024] - pot.sum(1).cpu().numpy()) <= eps*psize)
+
+
+def sampled(n):
+    """The points that the build's sort samples."""
+    ns = min(n, 4096)
+    j = np.arange(ns, dtype=np.uint64)
+    i0, i1 = j*np.uint64(n)//np.uint64(ns), (j + np.uint64(1))*np.uint64(n)//np.uint64(ns)
+    return (i0 + (((j*np.uint64(2654435769)) & np.uint64(0xffffffff))*(i1 - i0) >> np.uint64(32))).astype(np.int64)
+
+
+@pytest.mark.parametrize("case", ["chunk - 1", "chunk", "chunk + 1", "two chunks", "lattice", "clump", "chains", "one place"])
+def test_tree_build_edges(gpu, oracle_mod, case):
+    """Builds at the edges of the sort and of the cells' chunks (512 points) against the oracle's tree."""
+    print(f"[case] {case}", flush=True)
+    if case == "lattice":                      # 16 points a row: the sampling stride is a row's
+        n = 65536
+        k = np.arange(n)
+        x = np.stack([k % 16, k//16 % 64, k//1024], 1)/16.0 + 0.01
+    elif case == "clump":                      # one bucket with all but the sampled points: sorted in memory
+        n = 20000
+        x = 0.25 + 0.05*ball(n, 3)
+        around = ball(8192, 3)
+        x[sampled(n)] = around[((around - 0.25)**2).sum(1) > 0.01][:4096]
+    elif case == "chains":                     # pairs at 1e-5: up to 16 single-daughter cells above each
+        n = 3000
+        x = ball(n, 3)
+        x[1::2] = x[::2] + 1.0e-5
+    elif case == "one place":                  # lists of coincident points over several chunks, in two places
+        n = 2600
+        x = np.where(np.arange(n)[:, None] % 2 == 0, 0.25, -0.5)*np.ones((n, 3))
+    else:
+        n = {"chunk - 1": 511, "chunk": 512, "chunk + 1": 513, "two chunks": 1024}[case]
+        x = ball(n, 3)
+    m = np.linspace(1.0, 2.0, n)/n
+    hinv = 200.0 if case == "clump" else n**(1.0/3.0)
+    a, p = evaluate(gpu, x, m, 0.7, hinv)
+    cfg = abi.default_config(3, nperh=2.01)
+    cfg.integrator = abi.SPX_INTEGRATOR_SYNCHRONOUS_RK2
+    cfg.gravity = cfg.gravity_only = 1
+    cfg.G, cfg.softening, cfg.opening, cfg.ftimestep = 1.0, SOFT, 0.7, 0.1
+    H = np.broadcast_to(np.eye(3)*hinv, (n, 3, 3)).copy()
+    o = oracle_mod.OracleRun(cfg, n)
+    o.set_state(x=x, v=np.zeros((n, 3)), m=m, rho=np.ones(n), eps=np.zeros(n), H=H)
+    o.initialize()
+    o.evaluate_derivatives()
+    ao, po = o.field("delta velocity"), o.field("gravitational potential")
+    assert np.all(np.abs(a - ao) <= 1e-10*np.abs(ao).max())
+    assert np.all(np.abs(p - po) <= 1e-10*np.abs(po).max())
+
+
+def test_the_two_sorts_give_the_same_bits(gpu):
+    """2^19 points are sorted by the sample sort, more by the library's radix sort."""
+    n = 1 << 19
+    print(f"[case] {n} + 1 points", flush=True)
+    x, m = ball(n, 3), np.full(n, 1.0/n)
+    x[0], x[1] = -1.0, 1.0
+    a, p = evaluate(gpu, x, m, 1.0)
+    a1, p1 = evaluate(gpu, np.concatenate([x, [[-0.9, 0.9, 0.9]]]), np.append(m, 1.0e-200), 1.0)
+    assert np.array_equal(a, a1[:-1]) and np.array_equal(p, p1[:-1])
