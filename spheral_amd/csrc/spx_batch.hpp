@@ -224,7 +224,7 @@ class Batch {
   bool timing = false;
   // TreeGravity's own stream and its fork / join events (gravity runs only)
   hipStream_t gstream = nullptr;
-  hipEvent_t evFork = nullptr, evJoin = nullptr;
+  hipEvent_t evFork = nullptr, evTree = nullptr, evJoin = nullptr;
   bool gravPending = false;
   std::vector<std::string> tnames;
   std::vector<double> tms;
@@ -252,6 +252,7 @@ class Batch {
       // the midpoint grad-h and SPH passes, which neither read nor write what they use
       HIP_CHECK(hipStreamCreateWithFlags(&gstream, hipStreamNonBlocking));
       HIP_CHECK(hipEventCreateWithFlags(&evFork, hipEventDisableTiming));
+      HIP_CHECK(hipEventCreateWithFlags(&evTree, hipEventDisableTiming));
       HIP_CHECK(hipEventCreateWithFlags(&evJoin, hipEventDisableTiming));
     }
   }
@@ -268,6 +269,7 @@ class Batch {
     if (gstream) (void)hipStreamSynchronize(gstream);
     grav.release();
     if (evFork) (void)hipEventDestroy(evFork);
+    if (evTree) (void)hipEventDestroy(evTree);
     if (evJoin) (void)hipEventDestroy(evJoin);
     if (gstream) (void)hipStreamDestroy(gstream);
     if (stream) (void)hipStreamDestroy(stream);
@@ -1487,6 +1489,10 @@ class Batch {
     double* xs[3] = {mid ? f.xm[0] : f.x[0], mid ? f.xm[1] : f.x[1], mid ? f.xm[2] : f.x[2]};
     grav.build(xs, f.m, (int)nActive);
     if (!forked) mark("tree_build");
+    if (forked) {
+      grav.prepareWalk(cfg.opening, cfg.softening);
+      HIP_CHECK(hipEventRecord(evTree, gstream));
+    }
     grav.evaluate(f.DvDtG, f.pot, (int)nActive, cfg.G, cfg.softening, cfg.opening, dsc, cfg.ftimestep);
     if (toState)
       HIP_CHECK(hipMemcpyAsync(f.potS, f.pot, nActive*sizeof(double), hipMemcpyDeviceToDevice, grav.stream));
@@ -1710,9 +1716,14 @@ class Batch {
     // its launches queued after the SPH pass's so the host's waits inside the tree build do not
     // hold them back, joined before the update)
     const bool overlap = cfg.gravity && !timing;
+    const bool early = overlap && grav.buildsWithoutWait((int)nActive);
     if (overlap) forkGravity();
     omegaPass(true);
     mark("omega");
+    if (early) {
+      gravityPass(true, false, true);
+      HIP_CHECK(hipStreamWaitEvent(stream, evTree, 0));
+    }
     // derivatives at the midpoint
     if (cfg.gravity && !overlap) { gravityPass(true); mark("gravity"); }
     // the Limited Q reads its gradient (the previous evaluation's DvDx, ArtificialViscosityHandle::
@@ -1720,7 +1731,7 @@ class Batch {
     // copies the new DvDx into it, as the reference's state holds it after the step
     sphPass(false, true, true);
     copyQVelocityGradient();
-    if (overlap) gravityPass(true, false, true);
+    if (overlap && !early) gravityPass(true, false, true);
     mark("sph");
     joinGravity();
     fullStep();

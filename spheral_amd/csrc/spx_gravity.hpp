@@ -39,13 +39,14 @@ struct TreeBox { double lo[3], box; };       // cube of the tree: lower corner, 
 // Points up to which the keys are sorted by the sample sort below, and cells are allocated for the
 // worst case (kTreeBits per point: 1.1 KB): building then takes no wait on the host.  Beyond, the
 // library's radix sort and a download of the cell count; the walk outweighs both there.
-constexpr int kTreeOwnSort = 1 << 19;
-constexpr int kTreeSample = 4096;       // keys sampled, sorted in one block
-constexpr int kTreeBuckets = 1024;      // every fourth of them starts a bucket
-constexpr int kTreeBucketLds = 2048;    // bucket size up to which it is sorted in LDS
+constexpr int kTreeOwnSort = 1 << 18;
+constexpr int kTreeBuckets = 1024;      // of the sort, half as many up to kTreeFewer points: as many
+constexpr int kTreeFewer = 1 << 16;     // points are sampled, and one block sorts them
+constexpr int kTreeBucketRoom = 16;     // mean bucket sizes up to which a bucket is sorted in LDS
 constexpr int kTreeBoxBlocks = 256;
 constexpr int kTreeChunk = 512;         // points per block of the cells' kernel
 constexpr int kTreeCellsLds = 1280;     // cells of a chunk whose moments are kept in LDS
+constexpr int kTreeTopUnits = 48;       // lists of 21 levels per block of k_tree_top
 
 __device__ __forceinline__ int lcp_levels(uint64_t a, uint64_t b) {
   const uint64_t x = a ^ b;
@@ -149,23 +150,51 @@ __device__ __forceinline__ void tree_bitonic(uint64_t* key, uint32_t* id, int cn
   }
 }
 
-// One block: the cube from the blocks' extents; and, for the sample sort, kTreeBuckets splitters
-// (key, index) out of kTreeSample sampled points.  Clears the counters of the build.
-__global__ void __launch_bounds__(1024) k_tree_split(TreePoints xs, int n, const double* part, int nparts, bool sample,
-                                                     TreeBox* out, uint64_t* splitKey, uint32_t* splitId, int* count,
-                                                     int* topCount) {
-  __shared__ double ext[6];
-  __shared__ uint64_t key[kTreeSample];
-  __shared__ uint32_t id[kTreeSample];
+// One entry per thread, in order over the block's first `size` threads (a power of two; the other
+// entries end anywhere behind them): a bitonic network, by lane exchanges within wavefronts and
+// through LDS across them.
+__device__ __forceinline__ void tree_bitonic_lanes(uint64_t& key, uint32_t& id, int size, uint64_t* skey, uint32_t* sid) {
   const int t = threadIdx.x;
+  for (int k = 2; k <= size; k <<= 1)
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      uint64_t ok;
+      uint32_t oi;
+      if (j >= 64) {
+        skey[t] = key;
+        sid[t] = id;
+        __syncthreads();
+        ok = skey[t ^ j];
+        oi = sid[t ^ j];
+        __syncthreads();
+      } else {
+        ok = __shfl_xor((unsigned long long)key, j);
+        oi = __shfl_xor(id, j);
+      }
+      const bool low = ((t & j) == 0) == ((t & k) == 0);      // this thread keeps the smaller
+      if (tree_less(ok, oi, key, id) == low) {
+        key = ok;
+        id = oi;
+      }
+    }
+}
+
+// One block: the cube from the blocks' extents; and, for the sample sort, its splitters
+// (key, index), sampled points in order.  Clears the counters of the build.
+template <int BUCKETS>
+__global__ void __launch_bounds__(BUCKETS) k_tree_split(TreePoints xs, int n, const double* part, int nparts, bool sample,
+                                                     TreeBox* out, uint64_t* splitKey, uint32_t* splitId, int* count) {
+  __shared__ double ext[6];
+  __shared__ uint64_t skey[BUCKETS];
+  __shared__ uint32_t sid[BUCKETS];
+  const int t = threadIdx.x;
+  static_assert(BUCKETS >= 6*64);
   if (t/64 < 6) {
     double v = 1.7976931348623157e308;
     for (int b = t % 64; b < nparts; b += 64) v = fmin(v, part[(size_t)b*6 + t/64]);
     for (int s = 32; s > 0; s >>= 1) v = fmin(v, __shfl_xor(v, s));
     if (t % 64 == 0) ext[t/64] = v;
   }
-  if (t <= kTreeBits) topCount[t] = 0;
-  for (int b = t; b < kTreeBuckets; b += 1024) count[b] = 0;
+  count[t] = 0;
   __syncthreads();
   const double lo[3] = {ext[0], ext[2], ext[4]};
   double box = 0.0;
@@ -173,21 +202,19 @@ __global__ void __launch_bounds__(1024) k_tree_split(TreePoints xs, int n, const
   for (int a = 0; a < 3; ++a) box = fmax(box, fabs(-ext[2*a + 1] - lo[a]));
   if (t == 0) *out = TreeBox{{lo[0], lo[1], lo[2]}, box};
   if (!sample) return;
-  const int ns = n < kTreeSample ? n : kTreeSample;
-  for (int j = t; j < ns; j += 1024) {
+  const int ns = n < BUCKETS ? n : BUCKETS;
+  uint64_t key = ~0ull;
+  uint32_t id = ~0u;
+  if (t < ns) {
     // one out of each of ns equal stretches, at a scrambled place: no period of the particles' order
-    const int64_t i0 = (int64_t)j*n/ns, i1 = (int64_t)(j + 1)*n/ns;
-    const int i = (int)(i0 + (int64_t)(((uint64_t)((uint32_t)j*2654435769u)*(uint64_t)(i1 - i0)) >> 32));
-    key[j] = tree_key(xs, i, lo, box);
-    id[j] = (uint32_t)i;
+    const int64_t i0 = (int64_t)t*n/ns, i1 = (int64_t)(t + 1)*n/ns;
+    const int i = (int)(i0 + (int64_t)(((uint64_t)((uint32_t)t*2654435769u)*(uint64_t)(i1 - i0)) >> 32));
+    key = tree_key(xs, i, lo, box);
+    id = (uint32_t)i;
   }
-  __syncthreads();
-  tree_bitonic(key, id, ns);
-  for (int b = t; b < kTreeBuckets; b += 1024) {
-    const int j = (int)((int64_t)b*ns/kTreeBuckets);
-    splitKey[b] = key[j];
-    splitId[b] = id[j];
-  }
+  tree_bitonic_lanes(key, id, BUCKETS, skey, sid);
+  splitKey[t] = key;
+  splitId[t] = id;
 }
 
 // Keys alone, in particle order (for the library's sort).
@@ -201,12 +228,13 @@ __global__ void __launch_bounds__(kBlock) k_tree_codes(TreePoints xs, int n, con
 
 // Keys, and each point's bucket and place in it (any order: the bucket is sorted afterwards).  The
 // block counts its points per bucket in LDS and reserves their places with one atomic each.
+template <int BUCKETS>
 __global__ void __launch_bounds__(kBlock) k_tree_rank(TreePoints xs, int n, const TreeBox* bx, const uint64_t* splitKey,
                                                       const uint32_t* splitId, int* count, uint64_t* codes, int2* slot) {
-  __shared__ uint64_t sk[kTreeBuckets];
-  __shared__ uint32_t si[kTreeBuckets];
-  __shared__ int cnt[kTreeBuckets];
-  for (int b = threadIdx.x; b < kTreeBuckets; b += kBlock) {
+  __shared__ uint64_t sk[BUCKETS];
+  __shared__ uint32_t si[BUCKETS];
+  __shared__ int cnt[BUCKETS];
+  for (int b = threadIdx.x; b < BUCKETS; b += kBlock) {
     sk[b] = splitKey[b];
     si[b] = splitId[b];
     cnt[b] = 0;
@@ -217,22 +245,23 @@ __global__ void __launch_bounds__(kBlock) k_tree_rank(TreePoints xs, int n, cons
   if (i < n) {
     const uint64_t key = tree_key(xs, i, bx->lo, bx->box);
     codes[i] = key;
-    for (int step = kTreeBuckets/2; step > 0; step >>= 1)
+    for (int step = BUCKETS/2; step > 0; step >>= 1)
       if (!tree_less(key, (uint32_t)i, sk[b + step], si[b + step])) b += step;
     r = atomicAdd(&cnt[b], 1);
   }
   __syncthreads();
-  for (int c = threadIdx.x; c < kTreeBuckets; c += kBlock)
+  for (int c = threadIdx.x; c < BUCKETS; c += kBlock)
     if (cnt[c] > 0) cnt[c] = atomicAdd(&count[c], cnt[c]);
   __syncthreads();
   if (i < n) slot[i] = make_int2(b, cnt[b] + r);
 }
 
 // Points into their buckets' places.
+template <int BUCKETS>
 __global__ void __launch_bounds__(kBlock) k_tree_scatter(int n, const int* count, const uint64_t* codes, const int2* slot,
                                                          uint64_t* keys, uint32_t* idx) {
-  constexpr int per = kTreeBuckets/kBlock;
-  __shared__ int start[kTreeBuckets];
+  constexpr int per = BUCKETS/kBlock;
+  __shared__ int start[BUCKETS];
   __shared__ int wsum[kBlock/64];
   const int t = threadIdx.x;
   int own[per], sum = 0;
@@ -274,33 +303,49 @@ __global__ void __launch_bounds__(kBlock) k_tree_gather(TreePoints xs, const dou
   if (p < n) tree_place(xs, m, perm[p], p, o);
 }
 
-// One block per bucket sorts it, in LDS or, where more points than expected fell between two
-// splitters, in place in memory; then the points go into tree order.
-__global__ void __launch_bounds__(kBlock) k_tree_sort(const int* count, uint64_t* keys, uint32_t* idx, TreePoints xs,
-                                                      const double* m, uint64_t* codes, uint32_t* perm, TreeOrder o) {
-  __shared__ uint64_t key[kTreeBucketLds];
-  __shared__ uint32_t id[kTreeBucketLds];
-  __shared__ int wsum[kBlock/64];
+// One block per bucket sorts it: in registers, in LDS or, where far more points than expected fell
+// between two splitters, in place in memory; then the points go into tree order.
+template <int BLOCK>
+__global__ void __launch_bounds__(BLOCK) k_tree_sort(const int* count, int room, uint64_t* keys, uint32_t* idx, TreePoints xs,
+                                                     const double* m, uint64_t* codes, uint32_t* perm, TreeOrder o) {
+  extern __shared__ char shared[];
+  uint64_t* key = reinterpret_cast<uint64_t*>(shared);
+  uint32_t* id = reinterpret_cast<uint32_t*>(key + room);
+  __shared__ int wsum[BLOCK/64];
   const int t = threadIdx.x, cnt = count[blockIdx.x];
   if (cnt == 0) return;
   int before = 0;
-  for (int b = t; b < (int)blockIdx.x; b += kBlock) before += count[b];
+  for (int b = t; b < (int)blockIdx.x; b += BLOCK) before += count[b];
   for (int s = 32; s > 0; s >>= 1) before += __shfl_xor(before, s);
   if (t % 64 == 0) wsum[t/64] = before;
   __syncthreads();
   before = 0;
-  for (int w = 0; w < kBlock/64; ++w) before += wsum[w];
+  for (int w = 0; w < BLOCK/64; ++w) before += wsum[w];
   uint64_t* gk = keys + before;
   uint32_t* gi = idx + before;
-  const bool inLds = cnt <= kTreeBucketLds;
+  if (cnt <= BLOCK) {
+    uint64_t k = ~0ull;
+    uint32_t q = ~0u;
+    if (t < cnt) { k = gk[t]; q = gi[t]; }
+    int size = 1;
+    while (size < cnt) size <<= 1;
+    tree_bitonic_lanes(k, q, size, key, id);
+    if (t < cnt) {
+      codes[before + t] = k;
+      perm[before + t] = q;
+      tree_place(xs, m, q, before + t, o);
+    }
+    return;
+  }
+  const bool inLds = cnt <= room;
   if (inLds) {
-    for (int j = t; j < cnt; j += kBlock) { key[j] = gk[j]; id[j] = gi[j]; }
+    for (int j = t; j < cnt; j += BLOCK) { key[j] = gk[j]; id[j] = gi[j]; }
     __syncthreads();
     tree_bitonic(key, id, cnt);
   } else {
     tree_bitonic(gk, gi, cnt);
   }
-  for (int j = t; j < cnt; j += kBlock) {
+  for (int j = t; j < cnt; j += BLOCK) {
     const uint32_t q = inLds ? id[j] : gi[j];
     codes[before + j] = inLds ? key[j] : gk[j];
     perm[before + j] = q;
@@ -364,16 +409,21 @@ struct TreeShape {
   int *first, *last;            // point range of the cells of kind kCellList
 };
 
-// The record of cell c at level l that holds points p..end-1.
-__device__ __forceinline__ void tree_store(const TreeShape& f, int c, int l, uint64_t key, int p, int end, int skip,
+// Cell coordinates of a key at the deepest level.
+struct TreeCoord { uint32_t i[3]; };
+__device__ __forceinline__ TreeCoord tree_coord(uint64_t key) {
+  return TreeCoord{{(uint32_t)third_bits(key), (uint32_t)third_bits(key >> 1), (uint32_t)third_bits(key >> 2)}};
+}
+
+// The record of cell c at level l that holds points p..end-1 (only lists need the exact end).
+__device__ __forceinline__ void tree_store(const TreeShape& f, int c, int l, const TreeCoord& at, int p, int end, int skip,
                                            double m, double x, double y, double z) {
   const double cs = ldexp(f.bx->box, -l), xc[3] = {x, y, z};
   double r2 = 0.0;
 #pragma unroll
   for (int a = 0; a < 3; ++a)
     if (a < f.dim) {
-      const uint64_t ia = third_bits(key >> (3*(kTreeBits - l) + a));
-      const double d = xc[a] - fused(cs, (double)ia + 0.5, f.bx->lo[a]);
+      const double d = xc[a] - fused(cs, (double)(at.i[a] >> (kTreeBits - l)) + 0.5, f.bx->lo[a]);
       r2 = fused(d, d, r2);
     }
   TreeCell t{x, y, z, m, ldexp(rounded_product(f.bx->box, f.bx->box), -2*l)/f.open2 + r2, skip, kCellOpen};
@@ -398,11 +448,15 @@ struct alignas(16) TreeTop {
   int child[8];                 // per octant: its first point, then its cell; -1: empty
 };
 
-// First point in [p, n) whose key is at least v.
+// First point in [p, n) whose key is at least v: four ways per step, as a step is one read's latency.
 __device__ __forceinline__ int tree_bound(const uint64_t* code, int p, int n, uint64_t v) {
   while (p < n) {
-    const int mid = (p + n) >> 1;
-    if (code[mid] < v) p = mid + 1; else n = mid;
+    const int len = n - p, a = p + len/4, b = p + len/2, c = p + (int)(3*(int64_t)len/4);
+    const uint64_t ka = code[a], kb = code[b], kc = code[c];
+    if (kc < v) p = c + 1;
+    else if (kb < v) { p = b + 1; n = c; }
+    else if (ka < v) { p = a + 1; n = b; }
+    else n = a;
   }
   return p;
 }
@@ -414,15 +468,17 @@ __device__ __forceinline__ int tree_bound(const uint64_t* code, int p, int n, ui
 // listed with their daughters for k_tree_top.  One launch instead of one per level: see build().
 __global__ void __launch_bounds__(kTreeChunk) k_tree_cells(TreeShape f, const uint64_t* code, TreeOrder o,
                                                            const int* total, const int* before, int* cstart, int* ncells,
-                                                           int* topCount, TreeTop* top) {
+                                                           TreeTop* top) {
   __shared__ uint64_t key[kTreeChunk];
-  __shared__ int at[kTreeChunk + 1], skips[kTreeCellsLds];
+  __shared__ int at[kTreeChunk + 1], skips[kTreeCellsLds + 1];
   __shared__ double lm[kTreeCellsLds], lx[kTreeCellsLds], ly[kTreeCellsLds], lz[kTreeCellsLds];
   __shared__ int wsum[kTreeChunk/64], topHead[kTreeBits + 1];
+  __shared__ unsigned levels;
   const int t = threadIdx.x, n = f.n, s = blockIdx.x*kTreeChunk, nloc = min(kTreeChunk, n - s), p = s + t;
   const uint64_t kk = t < nloc ? code[p] : 0;
   key[t] = kk;
   if (t <= kTreeBits) topHead[t] = -1;
+  if (t == 0) levels = 0;
   TreeHead h{1, 0, -1};
   if (t < nloc) h = tree_head(code, p, n, kk);
   const int nh = h.count();
@@ -452,24 +508,40 @@ __global__ void __launch_bounds__(kTreeChunk) k_tree_cells(TreeShape f, const ui
   const bool inLds = nc <= kTreeCellsLds;
   __syncthreads();
   const bool single = h.after < h.leaf;         // the leaf holds this point alone
+  // Levels at which this thread's cell has its moments formed from daughters (or a list): those
+  // within the chunk.  skips: the next cell behind the subtree, and the cell's level below it.
+  const int fine = h.leaf - (single ? 1 : 0), coarse = max(h.start, out + 1);
+  const unsigned mine = nh > 0 && fine >= coarse ? (2u << fine) - (1u << coarse) : 0u;
+  if (mine) atomicOr(&levels, mine);
+  const TreeCoord coord = tree_coord(kk);
+  if (inLds) {
+    for (int k = 0; k < nh; ++k) skips[j0 + k] = h.start + k;
+    if (t == 0) skips[nc] = 0;                  // ends any subtree
+  }
   if (nh > 0 && single) {
     const int j = j0 + nh - 1;
     const double m = o.m[p], x = o.x[0][p], y = o.x[1][p], z = o.x[2][p];
-    if (inLds) { lm[j] = m; lx[j] = x; ly[j] = y; lz[j] = z; skips[j] = j + 1; }
-    tree_store(f, base + j, h.leaf, kk, p, p + 1, base + j + 1, m, x, y, z);
+    if (inLds) { lm[j] = m; lx[j] = x; ly[j] = y; lz[j] = z; skips[j] |= (j + 1) << 5; }
+    tree_store(f, base + j, h.leaf, coord, p, p + 1, base + j + 1, m, x, y, z);
   }
+  __syncthreads();
   int lo = t;                                   // the last point found so far, of the finer level
-  for (int l = kTreeBits; l >= 0; --l) {
-    const bool has = nh > 0 && l >= h.start && l <= h.leaf && l > out && !(l == h.leaf && single);
-    if (!__syncthreads_or(has)) continue;
-    if (!has) continue;
-    const int sh = 3*(kTreeBits - l);
-    int hi = nloc - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (key[mid] >> sh == kk >> sh) lo = mid; else hi = mid - 1;
+  for (unsigned todo = levels; todo;) {
+    const int l = 31 - __clz(todo);
+    todo ^= 1u << l;
+    __syncthreads();
+    if (!(mine >> l & 1)) continue;
+    const int j = j0 + l - h.start;
+    int je = j + 1;
+    if (l == kTreeBits || !inLds) {
+      const int sh = 3*(kTreeBits - l);
+      int hi = nloc - 1;
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (key[mid] >> sh == kk >> sh) lo = mid; else hi = mid - 1;
+      }
+      je = at[lo + 1];
     }
-    const int j = j0 + l - h.start, je = at[lo + 1];
     double m = 0.0, x = 0.0, y = 0.0, z = 0.0;
     if (l == kTreeBits) {
       for (int q = p; q <= s + lo; ++q) {
@@ -480,12 +552,16 @@ __global__ void __launch_bounds__(kTreeChunk) k_tree_cells(TreeShape f, const ui
         z = fused(mq, o.x[2][q], z);
       }
     } else if (inLds) {
-      for (int d = j + 1; d < je; d = skips[d]) {
-        const double md = lm[d];
+      // the daughters' subtrees end where a cell of level <= l starts
+      for (int sk = skips[je]; (sk & 31) > l;) {
+        const int to = sk >> 5;
+        sk = skips[to];
+        const double md = lm[je];
         m += md;
-        x = fused(md, lx[d], x);
-        y = fused(md, ly[d], y);
-        z = fused(md, lz[d], z);
+        x = fused(md, lx[je], x);
+        y = fused(md, ly[je], y);
+        z = fused(md, lz[je], z);
+        je = to;
       }
     } else {
       for (int d = base + j + 1; d < base + je;) {
@@ -500,17 +576,18 @@ __global__ void __launch_bounds__(kTreeChunk) k_tree_cells(TreeShape f, const ui
     x /= m;
     y /= m;
     z /= m;
-    if (inLds) { lm[j] = m; lx[j] = x; ly[j] = y; lz[j] = z; skips[j] = je; }
-    tree_store(f, base + j, l, kk, p, s + lo + 1, base + je, m, x, y, z);
+    if (inLds) { lm[j] = m; lx[j] = x; ly[j] = y; lz[j] = z; skips[j] = je << 5 | l; }
+    tree_store(f, base + j, l, coord, p, l == kTreeBits ? s + lo + 1 : p + 2, base + je, m, x, y, z);
   }
   // Rows of 16 lanes: one level's listed cell each, a lane per octant and one for the end.
   const int l = t/16, r = t % 16;
-  if (l > kTreeBits || topHead[l] < 0) return;
+  if (l > kTreeBits) return;
+  TreeTop* w = top + (size_t)blockIdx.x*(kTreeBits + 1) + l;
   const int q = topHead[l], sh = 3*(kTreeBits - l);
-  int pos = 0;
-  if (r == 0) pos = atomicAdd(&topCount[l], 1);
-  pos = __shfl(pos, 0, 16);
-  TreeTop* w = top + (size_t)l*gridDim.x + pos;
+  if (q < 0) {
+    if (r == 9) w->c = -1;
+    return;
+  }
   const uint64_t pre = key[q] >> sh;
   if (r < 8) {
     int c = -1;
@@ -528,63 +605,68 @@ __global__ void __launch_bounds__(kTreeChunk) k_tree_cells(TreeShape f, const ui
   }
 }
 
-// The listed cells, one block: cells of their daughters and behind them first, then the moments
-// level by level.
-__global__ void __launch_bounds__(1024) k_tree_top(TreeShape f, const uint64_t* code, TreeOrder o, int nchunk,
-                                                   const int* cstart, const int* ncells, int* topCount, TreeTop* top) {
-  __shared__ int cnt[kTreeBits + 1];
-  const int t = threadIdx.x;
-  if (t <= kTreeBits) cnt[t] = topCount[t];
-  __syncthreads();
-  int all = 0;
-  for (int l = 0; l <= kTreeBits; ++l) all += cnt[l];
-  for (int i = t; i < all; i += 1024) {
-    int l = 0, k = i;
-    while (k >= cnt[l]) k -= cnt[l++];
-    TreeTop* w = top + (size_t)l*nchunk + k;
-    const int p = w->p;
-    w->skip = w->end < f.n ? cstart[w->end] : *ncells;
-    for (int a = 0; a < 8; ++a) {
-      const int q = w->child[a];
-      if (q >= 0) w->child[a] = q == p ? w->c + 1 : cstart[q];
-    }
+// The listed cells of kTreeTopUnits units (chunks at first), `span` points each, that end within
+// them: moments level by level, a thread per cell.  Cells that reach on are listed for the next
+// launch, in which these units are one (again at most one cell per level).  first: the daughters
+// are still points.
+__global__ void __launch_bounds__(1024) k_tree_top(TreeShape f, const uint64_t* code, TreeOrder o, int units, int64_t span,
+                                                   bool first, const int* cstart, const int* ncells, const TreeTop* top,
+                                                   TreeTop* up) {
+  __shared__ unsigned levels;
+  // by level, so that a level's cells are in one or two wavefronts
+  const int t = threadIdx.x, l = t/kTreeTopUnits, u = blockIdx.x*kTreeTopUnits + t % kTreeTopUnits;
+  const bool slot = l <= kTreeBits && u < units;
+  TreeTop w{-1};
+  if (slot) w = top[(size_t)u*(kTreeBits + 1) + l];
+  if (t == 0) levels = 0;
+  if (t <= kTreeBits) up[(size_t)blockIdx.x*(kTreeBits + 1) + t].c = -1;
+  if (first && w.c >= 0) {
+    int child[8];
+#pragma unroll
+    for (int a = 0; a < 8; ++a) child[a] = cstart[max(w.child[a], 0)];
+    w.skip = w.end < f.n ? cstart[w.end] : *ncells;
+#pragma unroll
+    for (int a = 0; a < 8; ++a)
+      if (w.child[a] >= 0) w.child[a] = w.child[a] == w.p ? w.c + 1 : child[a];
   }
-  for (int l = kTreeBits; l >= 0; --l) {
-    if (cnt[l] == 0) continue;
+  const bool here = w.c >= 0 && (blockIdx.x + 1 == gridDim.x || w.end <= (blockIdx.x + 1)*kTreeTopUnits*span);
+  __syncthreads();
+  if (w.c >= 0 && !here) up[(size_t)blockIdx.x*(kTreeBits + 1) + l] = w;
+  if (here) atomicOr(&levels, 1u << l);
+  __syncthreads();
+  for (unsigned todo = levels; todo;) {
+    const int lvl = 31 - __clz(todo);
+    todo ^= 1u << lvl;
     __syncthreads();
-    for (int k = t; k < cnt[l]; k += 1024) {
-      const TreeTop w = top[(size_t)l*nchunk + k];
-      double m = 0.0, x = 0.0, y = 0.0, z = 0.0;
-      if (l == kTreeBits) {
-        for (int q = w.p; q < w.end; ++q) {
-          const double mq = o.m[q];
-          m += mq;
-          x = fused(mq, o.x[0][q], x);
-          y = fused(mq, o.x[1][q], y);
-          z = fused(mq, o.x[2][q], z);
-        }
-      } else {
-        double2 xy[8], zm[8];
-#pragma unroll
-        for (int a = 0; a < 8; ++a) {
-          const double2* d = reinterpret_cast<const double2*>(f.cells + max(w.child[a], 0));
-          xy[a] = d[0];
-          zm[a] = d[1];
-        }
-#pragma unroll
-        for (int a = 0; a < 8; ++a)
-          if (w.child[a] >= 0) {
-            m += zm[a].y;
-            x = fused(zm[a].y, xy[a].x, x);
-            y = fused(zm[a].y, xy[a].y, y);
-            z = fused(zm[a].y, zm[a].x, z);
-          }
+    if (!here || l != lvl) continue;
+    double m = 0.0, x = 0.0, y = 0.0, z = 0.0;
+    if (l == kTreeBits) {
+      for (int q = w.p; q < w.end; ++q) {
+        const double mq = o.m[q];
+        m += mq;
+        x = fused(mq, o.x[0][q], x);
+        y = fused(mq, o.x[1][q], y);
+        z = fused(mq, o.x[2][q], z);
       }
-      tree_store(f, w.c, l, code[w.p], w.p, w.end, w.skip, m, x/m, y/m, z/m);
+    } else {
+      double2 xy[8], zm[8];
+#pragma unroll
+      for (int a = 0; a < 8; ++a) {
+        const double2* d = reinterpret_cast<const double2*>(f.cells + max(w.child[a], 0));
+        xy[a] = d[0];
+        zm[a] = d[1];
+      }
+#pragma unroll
+      for (int a = 0; a < 8; ++a)
+        if (w.child[a] >= 0) {
+          m += zm[a].y;
+          x = fused(zm[a].y, xy[a].x, x);
+          y = fused(zm[a].y, xy[a].y, y);
+          z = fused(zm[a].y, zm[a].x, z);
+        }
     }
+    tree_store(f, w.c, l, tree_coord(code[w.p]), w.p, w.end, w.skip, m, x/m, y/m, z/m);
   }
-  __syncthreads();
-  if (t <= kTreeBits) topCount[t] = 0;
 }
 
 // Neighbouring points that walk the tree together.  In a group of four a wavefront reads 16 records
@@ -751,8 +833,8 @@ class GravityTree {
   int2* slot = nullptr;
   uint64_t* splitKey = nullptr;
   uint32_t* splitId = nullptr;
-  int *count = nullptr, *topCount = nullptr, *chunkTotal = nullptr, *chunkBefore = nullptr, *ncells = nullptr;
-  TreeTop* top = nullptr;
+  int *count = nullptr, *chunkTotal = nullptr, *chunkBefore = nullptr, *ncells = nullptr;
+  TreeTop *top = nullptr, *topNext = nullptr;
   TreeOrder order{};                // points in tree order
   TreeBox* box = nullptr;
   int* cstart = nullptr;
@@ -802,11 +884,11 @@ class GravityTree {
     splitKey = alloc<uint64_t>(kTreeBuckets);
     splitId = alloc<uint32_t>(kTreeBuckets);
     count = alloc<int>(kTreeBuckets);
-    topCount = alloc<int>(kTreeBits + 1);
     chunkTotal = alloc<int>(nchunk + 1);
     chunkBefore = alloc<int>(nchunk + 1);
     ncells = alloc<int>(1);
     top = alloc<TreeTop>((size_t)(kTreeBits + 1)*nchunk);
+    topNext = alloc<TreeTop>((size_t)(kTreeBits + 1)*((nchunk + kTreeTopUnits - 1)/kTreeTopUnits));
     for (int a = 0; a < 3; ++a) order.x[a] = alloc<double>(n);
     order.m = alloc<double>(n);
     order.tp = alloc<double2>(2*(size_t)n);
@@ -840,23 +922,32 @@ class GravityTree {
   }
 
   // The points in tree order and the number of cells per chunk.  Up to kTreeOwnSort points a build
-  // is eight launches and no wait: extent, splitters, buckets, scatter, bucket sorts, counts, and
-  // the cells' two (formCells).  The merge sort of the library, one moments launch per level, and
-  // three waits on the host took 0.50 ms of a 33k build and 0.87 ms of a 250k one.
+  // is nine or ten launches and no wait: extent, splitters, buckets, scatter, bucket sorts, counts,
+  // and the cells' (formCells).  Bound by the launches' latencies: 33k points 87 us, 250k 230 beside
+  // the grad-h pass (extent 5, splitters 11 / 16, sort 15 / 40, cells 21 / 35, cells above 21 / 31).
+  // The library's merge sort, one moments launch per level and three waits on the host took 500
+  // and 870 us.  512 buckets instead of 1024 take 5 us off the splitters, and a bucket still fits a
+  // block's registers up to kTreeFewer points.
   void build(double* const* xs, const double* m, int nn) {
     const int nb = (int)((nn + kBlock - 1)/kBlock), nbox = std::min(nb, kTreeBoxBlocks);
     const int nchunk = (nn + kTreeChunk - 1)/kTreeChunk;
     const bool own = nn <= kTreeOwnSort;
     const TreePoints pts{{xs[0], xs[1], D == 3 ? xs[2] : zero}};
     hipLaunchKernelGGL(k_tree_bbox, dim3(nbox), dim3(kBlock), 0, stream, pts, nn, part);
-    hipLaunchKernelGGL(k_tree_split, dim3(1), dim3(1024), 0, stream, pts, nn, (const double*)part, nbox, own, box, splitKey,
-                       splitId, count, topCount);
+    const bool fewer = nn <= kTreeFewer;
+    hipLaunchKernelGGL(fewer ? k_tree_split<kTreeBuckets/2> : k_tree_split<kTreeBuckets>, dim3(1),
+                       dim3(fewer ? kTreeBuckets/2 : kTreeBuckets), 0, stream, pts, nn, (const double*)part, nbox, own, box,
+                       splitKey, splitId, count);
     if (own) {
-      hipLaunchKernelGGL(k_tree_rank, dim3(nb), dim3(kBlock), 0, stream, pts, nn, (const TreeBox*)box,
-                         (const uint64_t*)splitKey, (const uint32_t*)splitId, count, codes, slot);
-      hipLaunchKernelGGL(k_tree_scatter, dim3(nb), dim3(kBlock), 0, stream, nn, (const int*)count, (const uint64_t*)codes,
-                         (const int2*)slot, keys, idx);
-      hipLaunchKernelGGL(k_tree_sort, dim3(kTreeBuckets), dim3(kBlock), 0, stream, (const int*)count, keys, idx, pts, m,
+      const int buckets = fewer ? kTreeBuckets/2 : kTreeBuckets, block = fewer ? kBlock : 2*kBlock;
+      const int room = std::max(kTreeBucketRoom*((nn + buckets - 1)/buckets), 2*kBlock);
+      hipLaunchKernelGGL(fewer ? k_tree_rank<kTreeBuckets/2> : k_tree_rank<kTreeBuckets>, dim3(nb), dim3(kBlock), 0, stream,
+                         pts, nn, (const TreeBox*)box, (const uint64_t*)splitKey, (const uint32_t*)splitId, count, codes,
+                         slot);
+      hipLaunchKernelGGL(fewer ? k_tree_scatter<kTreeBuckets/2> : k_tree_scatter<kTreeBuckets>, dim3(nb), dim3(kBlock), 0,
+                         stream, nn, (const int*)count, (const uint64_t*)codes, (const int2*)slot, keys, idx);
+      hipLaunchKernelGGL(fewer ? k_tree_sort<kBlock> : k_tree_sort<2*kBlock>, dim3(buckets), dim3(block),
+                         room*(sizeof(uint64_t) + sizeof(uint32_t)), stream, (const int*)count, room, keys, idx, pts, m,
                          codesSorted, perm, order);
     } else {
       hipLaunchKernelGGL(k_tree_codes, dim3(nb), dim3(kBlock), 0, stream, pts, nn, (const TreeBox*)box, codes, idx);
@@ -900,18 +991,27 @@ class GravityTree {
     const TreeShape shape{box, open2, self2, D, npts, cells, first, last};
     hipLaunchKernelGGL(k_tree_cells, dim3(nchunk), dim3(kTreeChunk), 0, stream, shape, (const uint64_t*)codesSorted, order,
                        (const int*)chunkTotal, npts <= kTreeOwnSort ? (const int*)nullptr : (const int*)chunkBefore, cstart,
-                       ncells, topCount, top);
-    if (nchunk > 1)
-      hipLaunchKernelGGL(k_tree_top, dim3(1), dim3(1024), 0, stream, shape, (const uint64_t*)codesSorted, order, nchunk,
-                         (const int*)cstart, (const int*)ncells, topCount, top);
+                       ncells, top);
+    TreeTop *from = top, *to = topNext;
+    int64_t span = kTreeChunk;
+    for (int units = nchunk; units > 1; span *= kTreeTopUnits) {
+      const int groups = (units + kTreeTopUnits - 1)/kTreeTopUnits;
+      hipLaunchKernelGGL(k_tree_top, dim3(groups), dim3(1024), 0, stream, shape, (const uint64_t*)codesSorted, order, units,
+                         span, units == nchunk, (const int*)cstart, (const int*)ncells, (const TreeTop*)from, to);
+      std::swap(from, to);
+      units = groups;
+    }
     HIP_CHECK(hipGetLastError());
     cellsOpen2 = open2;
     cellsSelf2 = self2;
   }
 
+  bool buildsWithoutWait(int nn) const { return nn <= kTreeOwnSort; }
+  void prepareWalk(double opening, double soft) { formCells(opening, selfRadius2(soft*soft)); }
+
   void evaluate(double* const* acc, double* pot, int nn, double G, double soft, double opening, Scalars* sc,
                 double ftimestep) {
-    const int nb = (int)((nn + kBlock - 1)/kBlock);
+    const int nb = (nn + kBlock - 1)/kBlock;
     double* az = D == 3 ? acc[2] : sink;
     const double self2 = selfRadius2(soft*soft);
     formCells(opening, self2);

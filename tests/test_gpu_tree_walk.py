@@ -74,7 +74,7 @@ def test_opened_walk_is_the_direct_sum(gpu, dim, n):
 
 def sampled(n):
     """The points that the build's sort samples."""
-    ns = min(n, 4096)
+    ns = min(n, 512 if n <= 65536 else 1024)
     j = np.arange(ns, dtype=np.uint64)
     i0, i1 = j*np.uint64(n)//np.uint64(ns), (j + np.uint64(1))*np.uint64(n)//np.uint64(ns)
     return (i0 + (((j*np.uint64(2654435769)) & np.uint64(0xffffffff))*(i1 - i0) >> np.uint64(32))).astype(np.int64)
@@ -84,15 +84,15 @@ def sampled(n):
 def test_tree_build_edges(gpu, oracle_mod, case):
     """Builds at the edges of the sort and of the cells' chunks (512 points) against the oracle's tree."""
     print(f"[case] {case}", flush=True)
-    if case == "lattice":                      # 16 points a row: the sampling stride is a row's
+    if case == "lattice":                      # 64 points a row: the sampling stride is a row's
         n = 65536
         k = np.arange(n)
-        x = np.stack([k % 16, k//16 % 64, k//1024], 1)/16.0 + 0.01
+        x = np.stack([k % 64, k//64 % 32, k//2048], 1)/32.0 + 0.01
     elif case == "clump":                      # one bucket with all but the sampled points: sorted in memory
         n = 20000
         x = 0.25 + 0.05*ball(n, 3)
         around = ball(8192, 3)
-        x[sampled(n)] = around[((around - 0.25)**2).sum(1) > 0.01][:4096]
+        x[sampled(n)] = around[((around - 0.25)**2).sum(1) > 0.01][:512]
     elif case == "chains":                     # pairs at 1e-5: up to 16 single-daughter cells above each
         n = 3000
         x = ball(n, 3)
@@ -121,8 +121,8 @@ def test_tree_build_edges(gpu, oracle_mod, case):
 
 
 def test_the_two_sorts_give_the_same_bits(gpu):
-    """2^19 points are sorted by the sample sort, more by the library's radix sort."""
-    n = 1 << 19
+    """2^18 points are sorted by the sample sort, more by the library's radix sort."""
+    n = 1 << 18
     print(f"[case] {n} + 1 points", flush=True)
     x, m = ball(n, 3), np.full(n, 1.0/n)
     x[0], x[1] = -1.0, 1.0
