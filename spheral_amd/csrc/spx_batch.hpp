@@ -219,7 +219,8 @@ class Batch {
   int seenNext = 0;
   bool useGraphs = true;
   int64_t graphCaptures = 0, graphReplays = 0, eagerSteps = 0;
-  int* dOverflowG = nullptr;  // the filter's overflow flag in graph-replayed steps
+  int* dflags = nullptr;      // kFlags
+  int* hOverflowG = nullptr;  // the overflow flag of the last step
   // per-class kernel time (ms) summed over the steps since timing was enabled
   bool timing = false;
   // TreeGravity's own stream and its fork / join events (gravity runs only)
@@ -492,7 +493,9 @@ class Batch {
     upload(dorder, horder, sizeof(int)*maxRuns);
     dinit = dalloc<int>(maxRuns);
     dOverflow = dalloc<int>(2);
-    dOverflowG = dalloc<int>(1);
+    dflags = dalloc<int>(kFlags);
+    HIP_CHECK(hipMemsetAsync(dflags, 0, kFlags*sizeof(int), stream));
+    hOverflowG = halloc<int>(1);
     dbuild = dalloc<int>(maxRuns);
     dsub = dalloc<int>(3*(size_t)maxRuns);
     skeys = dalloc<uint64_t>(ld);
@@ -963,7 +966,7 @@ class Batch {
     launchD([&](auto d) {
       constexpr int DD = decltype(d)::value;
       hipLaunchKernelGGL(k_keys<DD>, dim3(nb), dim3(kBlock), 0, stream, f, geo, (const RunGrid*)dgrids, (const int*)dstate,
-                         (const int*)dorder, (const int*)dbuild, (int)nTotal, wrapPending ? 1 : 0, 1, mortonBits, runBits, keys, vals);
+                         (const int*)dorder, (const int*)dbuild, (int)nTotal, wrapPending ? 1 : 0, 1, mortonBits, runBits, keys, vals, dflags);
     });
     HIP_CHECK(hipGetLastError());
     wrapPending = false;
@@ -1047,7 +1050,7 @@ class Batch {
       constexpr int DD = decltype(d)::value;
       hipLaunchKernelGGL(k_keys<DD>, dim3(nblocks(nTotal)), dim3(kBlock), 0, stream, f, geo, (const RunGrid*)dgrids,
                          (const int*)dstate, (const int*)dorder, (const int*)dbuild, (int)nTotal, wrapPending ? 1 : 0, 1,
-                         mortonBits, runBits, keys, vals);
+                         mortonBits, runBits, keys, vals, dflags);
     });
     HIP_CHECK(hipGetLastError());
     wrapPending = false;
@@ -1129,7 +1132,8 @@ class Batch {
   // The part of the connectivity pass that decides and does candidate-list builds: boundary
   // enforcement, the reorders, the candidate search (with its own capacity checks, which may
   // resize buffers).  Leaves connValid false.
-  void connectivityPrep(bool force) {
+  // deferBoundaries: a step that builds no lists leaves pending boundaries to k_prepare.
+  void connectivityPrep(bool force, bool deferBoundaries = false) {
     if (nTotal == 0) raise(SPX_ERR_STATE, "no state uploaded");
     ensureOmega();                   // a CheapSynchronousRK2 step drops it first (it never reads it)
     npairsCache = -1;                // every pass re-derives the neighbour lists
@@ -1158,7 +1162,7 @@ class Batch {
       else sortRebuildingRuns(bits);
       orderDirty = false;
       mark("reorder");
-    } else {
+    } else if (!deferBoundaries) {
       applyPendingBoundaries();
     }
     connValid = false;
@@ -1258,7 +1262,7 @@ class Batch {
       constexpr int DD = decltype(d)::value;
       hipLaunchKernelGGL(k_keys<DD>, dim3(nblocks(nTotal)), dim3(kBlock), 0, stream, f, geo, (const RunGrid*)nullptr,
                          (const int*)nullptr, (const int*)nullptr, (const int*)nullptr, (int)nTotal, 1, 0, 0, 0, keys,
-                         vals);
+                         vals, dflags);
     });
     HIP_CHECK(hipGetLastError());
     wrapPending = false;
@@ -1651,8 +1655,7 @@ class Batch {
     if (nActive == 0) return;
     const int nb = (int)xcd_grid(nActive, kBlock);
     hipLaunchKernelGGL(k_reset_dt, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns);
-    hipLaunchKernelGGL(k_select_dt, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns, ph, cfg.dt_min,
-                       cfg.dt_max, cfg.dt_growth, 1);
+    hipLaunchKernelGGL(k_select_dt, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns, ph, dtLimits(), 1);
     HIP_CHECK(hipGetLastError());
     mark("select_dt");
     gravityPass(false, true);
@@ -1671,9 +1674,10 @@ class Batch {
     });
     HIP_CHECK(hipGetLastError());
     mark("update");
-    hipLaunchKernelGGL(k_advance_time, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns);
+    hipLaunchKernelGGL(k_advance_time, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns, hsc, dflags,
+                       hOverflowG);
     HIP_CHECK(hipGetLastError());
-    download(hsc, dsc, sizeof(Scalars)*maxRuns);
+    HIP_CHECK(hipStreamSynchronize(stream));        // k_advance_time wrote the runs' scalars to hsc
     collectTimes();
   }
 
@@ -1697,24 +1701,31 @@ class Batch {
     if (nActive == 0) return;
     mark("connectivity");
     if (fresh) finishNewRuns();
-    const int nb = (int)xcd_grid(nActive, kBlock);
-    // Integrator::selectDt; TreeGravity's vote is the previous evaluation's
-    hipLaunchKernelGGL(k_select_dt, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns, ph, cfg.dt_min,
-                       cfg.dt_max, cfg.dt_growth, cfg.gravity);
-    HIP_CHECK(hipGetLastError());
-    mark("select_dt");
-    // half step with the previous derivatives
+    selectAndMidstep();
+    mark("update");
+    midpointDerivatives();
+    fullStep();
+  }
+  DtLimits dtLimits() const { return DtLimits{cfg.dt_min, cfg.dt_max, cfg.dt_growth}; }
+  // Integrator::selectDt (TreeGravity's vote is the previous evaluation's) and the half step with
+  // the previous derivatives.
+  void selectAndMidstep() {
     launchD([&](auto d) {
       constexpr int DD = decltype(d)::value;
-      hipLaunchKernelGGL(k_midstep<DD>, dim3(nb), dim3(kBlock), 0, stream, f, ph, (const Scalars*)dsc, (int)nActive);
+      hipLaunchKernelGGL(k_midstep<DD>, dim3(nblocks(std::max<int64_t>(nActive, maxRuns))), dim3(kBlock), 0, stream, f, ph,
+                         dsc, maxRuns, dtLimits(), (int)nActive);
     });
     HIP_CHECK(hipGetLastError());
-    mark("update");
-    // TreeGravity at the midpoint reads the midpoint positions and the masses and writes the
-    // gravity acceleration, potential and dt vote, which only the full update reads: outside
-    // per-class timing it runs on its own stream beside the grad-h and SPH passes (forked here,
-    // its launches queued after the SPH pass's so the host's waits inside the tree build do not
-    // hold them back, joined before the update)
+  }
+  // Grad-h, gravity and the derivatives at the midpoint.  TreeGravity at the midpoint reads the
+  // midpoint positions and the masses and writes the gravity acceleration, potential and dt vote,
+  // which only the full update reads: outside per-class timing it runs on its own stream, joined
+  // before the update.  A tree that is built without waits on the host is built beside the grad-h
+  // pass; the SPH pass then waits for the tree and runs beside the walk (beside the build it slows
+  // the build's small kernels by more than it gains: Evrard 250k 2236 -> 2145 us per step).  A
+  // larger tree's launches are queued after the SPH pass's, so the host's waits inside its build do
+  // not hold them back.
+  void midpointDerivatives() {
     const bool overlap = cfg.gravity && !timing;
     const bool early = overlap && grav.buildsWithoutWait((int)nActive);
     if (overlap) forkGravity();
@@ -1724,7 +1735,6 @@ class Batch {
       gravityPass(true, false, true);
       HIP_CHECK(hipStreamWaitEvent(stream, evTree, 0));
     }
-    // derivatives at the midpoint
     if (cfg.gravity && !overlap) { gravityPass(true); mark("gravity"); }
     // the Limited Q reads its gradient (the previous evaluation's DvDx, ArtificialViscosityHandle::
     // postStateUpdate) while this evaluation writes DvDx; the end-of-step postStateUpdate then
@@ -1734,7 +1744,6 @@ class Batch {
     if (overlap && !early) gravityPass(true, false, true);
     mark("sph");
     joinGravity();
-    fullStep();
   }
 
   // Integrator::step with SynchronousRK2::step and the SPH package (Integrator/SynchronousRK2.cc:
@@ -1754,8 +1763,7 @@ class Batch {
     mark("connectivity");
     if (fresh) finishNewRuns();
     const int nb = (int)xcd_grid(nActive, kBlock);
-    hipLaunchKernelGGL(k_select_dt, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns, ph, cfg.dt_min,
-                       cfg.dt_max, cfg.dt_growth, cfg.gravity);
+    hipLaunchKernelGGL(k_select_dt, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns, ph, dtLimits(), cfg.gravity);
     HIP_CHECK(hipGetLastError());
     mark("select_dt");
     // derivatives at the start of the step (boundaries applied: the Q sees its gradient's images)
@@ -1793,7 +1801,7 @@ class Batch {
     fullStepLaunches();
     omegaStale = cfg.gradh_correction != 0;
     if (eagerOmega) ensureOmega();
-    download(hsc, dsc, sizeof(Scalars)*maxRuns);
+    HIP_CHECK(hipStreamSynchronize(stream));        // k_advance_time wrote the runs' scalars to hsc
     collectTimes();
     finishTuningStep();
     tunerStepDone();
@@ -1824,7 +1832,8 @@ class Batch {
     }
     mark("energy_update");
     wrapPending = true;
-    hipLaunchKernelGGL(k_advance_time, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns);
+    hipLaunchKernelGGL(k_advance_time, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns, hsc, dflags,
+                       hOverflowG);
     HIP_CHECK(hipGetLastError());
   }
   // Host bookkeeping once the step's run scalars are downloaded.
@@ -1849,19 +1858,21 @@ class Batch {
   // ---------------------------------------------------------------- graph-replayed steps
   // After the connectivity pass's build decisions (candidate-list builds and reorders, which
   // may resize buffers and wait on the device, run eagerly), the rest of a CheapSynchronousRK2
-  // step -- connectivity records, the filtering sum-density + dt pass, dt selection, half step,
-  // midpoint grad-h, derivatives, full step -- launches the same kernels with the same arguments
-  // as the step two before it whenever no buffer was reallocated and the active particle count
-  // is unchanged (the velocity arrays alternate between two buffers).  That part is captured as
-  // a HIP graph per buffer parity and replayed: one launch instead of about fifteen, which is
-  // most of a small run's step time.  The graph holds no memset and no host synchronisation: the
-  // overflow flag is cleared by a kernel, and with the neighbour lists sized to the candidate
-  // lists' capacity the filter cannot overflow (a node's neighbours are a subset of its
-  // candidates).  Results are the eager step's bit for bit.  Steps with newly admitted runs,
-  // TreeGravity (host-side tree sizing), the Limited Q (its gradient copy), SynchronousRK2,
-  // timing or a group-size measurement run eagerly.
+  // step -- boundaries and connectivity records, the filtering sum-density + dt pass, dt selection
+  // and half step, midpoint grad-h, gravity, derivatives, full step -- launches the same kernels
+  // with the same arguments as the step two before it whenever no buffer was reallocated and the
+  // active particle count is unchanged (the velocity arrays alternate between two buffers).  That
+  // part is captured as a HIP graph per buffer parity and replayed: one launch instead of seven
+  // (seventeen with gravity), and the end of the step reaches the host's memory from its last
+  // kernel.  A small run's step is these launches: 1-D Limited-Q Noh of 100 nodes 172 -> 102 us per
+  // step, 1-D Sod of 400 137 -> 107.  The graph holds no memset, no copy and no host
+  // synchronisation, and with the neighbour lists sized to the candidate lists' capacity the filter
+  // cannot overflow (a node's neighbours are a subset of its candidates).  Results are the eager
+  // step's bit for bit.  Steps with newly admitted runs, trees whose build waits on the host,
+  // SynchronousRK2, timing or a group-size measurement run eagerly.
   bool graphsAllowed() const {
-    if (!useGraphs || timing || tuner.phase >= 0 || cfg.gravity || limitedQ()) return false;
+    if (!useGraphs || timing || tuner.phase >= 0) return false;
+    if (cfg.gravity && !grav.buildsWithoutWait((int)nActive)) return false;
     for (int r = 0; r < maxRuns; ++r)
       if (runs[r].state == RUN_ACTIVE && runs[r].needInit) return false;
     return true;
@@ -1879,7 +1890,7 @@ class Batch {
     put(&ph, sizeof(ph));
     put(&geo, sizeof(geo));
     put(&dtab, sizeof(dtab));
-    const void* bufs[] = {keys, vals, dsc, dOverflowG};
+    const void* bufs[] = {keys, vals, dsc, dflags, hsc, hOverflowG};
     put(bufs, sizeof(bufs));
     return k;
   }
@@ -1893,30 +1904,25 @@ class Batch {
     }
     for (auto& k : seenKeys) k.clear();
   }
-  // The eager step's launches after the connectivity build decisions (connectivity records,
-  // filter + sum density + dt vote, dt selection, half step, midpoint grad-h, derivatives, full
-  // step), with the overflow flag cleared by a kernel.
+  // The eager step's launches after the connectivity build decisions (boundaries, connectivity
+  // records, filter + sum density + dt vote, dt selection and half step, midpoint grad-h,
+  // derivatives, full step).
   void launchSteadyStep() {
-    pack();
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, stream, dOverflowG, 1, 0);
-    hipLaunchKernelGGL(k_reset_dt, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns);
-    launchFilter(dOverflowG);
-    const int nb = (int)xcd_grid(nActive, kBlock);
-    hipLaunchKernelGGL(k_select_dt, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns, ph, cfg.dt_min,
-                       cfg.dt_max, cfg.dt_growth, cfg.gravity);
-    HIP_CHECK(hipGetLastError());
+    ensureOmega();
     launchD([&](auto d) {
       constexpr int DD = decltype(d)::value;
-      hipLaunchKernelGGL(k_midstep<DD>, dim3(nb), dim3(kBlock), 0, stream, f, ph, (const Scalars*)dsc, (int)nActive);
+      hipLaunchKernelGGL(k_prepare<DD>, dim3(nblocks(std::max<int64_t>(nTotal, maxRuns))), dim3(kBlock), 0, stream, f, geo, ph,
+                         (int)nTotal, (int)nActive, dsc, maxRuns, dflags);
     });
     HIP_CHECK(hipGetLastError());
-    omegaPass(true);
-    sphPass(false, true, true);
+    launchFilter(dflags + kFlagOverflow);
+    selectAndMidstep();
+    midpointDerivatives();
     fullStepLaunches();
   }
   void graphStep() {
-    connectivityPrep(false);
-    if (nActive == 0) return;
+    connectivityPrep(false, true);
+    if (nActive == 0) { applyPendingBoundaries(); return; }
     ensureNbrCapacity(f.ccap);          // every candidate fits: the filter cannot overflow
     const Fields f0 = f;
     std::vector<unsigned char> key = graphKey();
@@ -1938,9 +1944,8 @@ class Batch {
       connValid = true;
       npairsCache = -1;
       wrapPending = true;
-      HIP_CHECK(hipMemcpyAsync(hOverflow, dOverflowG, sizeof(int), hipMemcpyDeviceToHost, stream));
-      download(hsc, dsc, sizeof(Scalars)*maxRuns);
-      if (*hOverflow != 0) raise(SPX_ERR_STATE, "neighbour list overflow in a steady step");
+      HIP_CHECK(hipStreamSynchronize(stream));
+      if (*hOverflowG != 0) raise(SPX_ERR_STATE, "neighbour list overflow in a steady step");
       tunerStepDone();
       endOfStep();
       return;
@@ -1971,6 +1976,7 @@ class Batch {
     }
     f = f0;
     HIP_CHECK(hipGraphLaunch(g->exec, stream));
+    if (cfg.gravity) grav.rebuilt((int)nActive, cfg.opening, cfg.softening);
     for (int a = 0; a < D; ++a) std::swap(f.v[a], f.v1[a]);
     omegaStale = cfg.gradh_correction != 0;
     if (eagerOmega) ensureOmega();
@@ -1978,9 +1984,8 @@ class Batch {
     connValid = true;
     npairsCache = -1;
     wrapPending = true;
-    HIP_CHECK(hipMemcpyAsync(hOverflow, dOverflowG, sizeof(int), hipMemcpyDeviceToHost, stream));
-    download(hsc, dsc, sizeof(Scalars)*maxRuns);
-    if (*hOverflow != 0) raise(SPX_ERR_STATE, "neighbour list overflow in a replayed step");
+    HIP_CHECK(hipStreamSynchronize(stream));
+    if (*hOverflowG != 0) raise(SPX_ERR_STATE, "neighbour list overflow in a replayed step");
     tunerStepDone();
     endOfStep();
   }
@@ -2002,9 +2007,9 @@ class Batch {
   // Limited Q's gradient becomes a copy of the hydro's DvDx of the last evaluation.
   void copyQVelocityGradient() {
     if (!limitedQ() || nTotal == 0) return;
-    for (int c = 0; c < D*D; ++c)
-      HIP_CHECK(hipMemcpyAsync(f.DvDxQ + (size_t)c*ld, f.DvDx + (size_t)c*ld, nTotal*sizeof(double),
-                               hipMemcpyDeviceToDevice, stream));
+    hipLaunchKernelGGL(k_copy_rows, dim3(nblocks(nTotal)), dim3(kBlock), 0, stream, (const double*)f.DvDx, f.DvDxQ, nTotal,
+                       (int64_t)ld, D*D);
+    HIP_CHECK(hipGetLastError());
   }
 
   // ---------------------------------------------------------------- single-run package calls
@@ -2049,8 +2054,8 @@ class Batch {
     requireConn();
     pack();
     densityDt(false, true);
-    hipLaunchKernelGGL(k_select_dt, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns, ph, 0.0,
-                       1.7976931348623157e308, 1.7976931348623157e308, cfg.gravity);
+    hipLaunchKernelGGL(k_select_dt, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns, ph,
+                       DtLimits{0.0, 1.7976931348623157e308, 1.7976931348623157e308}, cfg.gravity);
     HIP_CHECK(hipGetLastError());
     download(hsc, dsc, sizeof(Scalars)*maxRuns);
     *hydro = hsc[slot].hydroDt;

@@ -322,6 +322,10 @@ struct Scalars {
   int nonfinite, pad;
 };
 
+// A batch's device flags: the filter's overflow in steady steps, and whether the last step's
+// positions still await the boundaries.
+enum : int { kFlagOverflow = 0, kFlagWrap = 1, kFlags = 2 };
+
 // Order-preserving map between doubles and unsigned 64-bit integers (for atomic min/max).
 __device__ __forceinline__ unsigned long long ord_bits(double d) {
   const unsigned long long b = (unsigned long long)__double_as_longlong(d);

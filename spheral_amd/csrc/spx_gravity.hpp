@@ -1006,6 +1006,12 @@ class GravityTree {
     cellsSelf2 = self2;
   }
 
+  // The tree now held was built and its cells formed by launches that were recorded earlier.
+  void rebuilt(int nn, double opening, double soft) {
+    npts = nn;
+    cellsOpen2 = opening*opening;
+    cellsSelf2 = selfRadius2(soft*soft);
+  }
   bool buildsWithoutWait(int nn) const { return nn <= kTreeOwnSort; }
   void prepareWalk(double opening, double soft) { formCells(opening, selfRadius2(soft*soft)); }
 

@@ -52,11 +52,34 @@ __device__ __forceinline__ int cell_coord(const RunGrid& gr, int a, double x) {
 // that keep their candidate list (build[run] == 0) get no Morton bits: the sort is
 // stable, so they keep their order.
 // ---------------------------------------------------------------------------
+// Node i's coordinate xa along axis a with the boundaries enforced (periodic: moved back into the
+// box; reflecting: mirrored, the velocity too).
+template <int D>
+__device__ __forceinline__ double enforce_axis(const Fields& f, const Geo& g, int a, int i, double xa) {
+  for (int side = 1; side <= 2; ++side) {
+    const int bc = side == 1 ? (((g.permask >> a) & 1) ? BC_PERIODIC : (((g.reflmask >> (2*a)) & 1) ? BC_REFLECTING : BC_NONE))
+                             : (((g.permask >> a) & 1) ? BC_PERIODIC : (((g.reflmask >> (2*a + 1)) & 1) ? BC_REFLECTING : BC_NONE));
+    if (bc == BC_NONE) continue;
+    const double thpt = side == 1 ? (xa - g.xmin[a]) : -(xa - g.xmax[a]);
+    const bool fuzzy0 = fabs(thpt) <= 1.0e-15*fmax(1.0, fabs(thpt));
+    if (!fuzzy0 && thpt < 0.0) {
+      if (bc == BC_PERIODIC) {
+        xa = image_coord<D>(bc, side == 1 ? 2 : 1, xa, g.xmin[a], g.xmax[a]);
+      } else {
+        xa = image_coord<D>(bc, side, xa, g.xmin[a], g.xmax[a]);
+        f.v[a][i] = -f.v[a][i];
+      }
+    }
+  }
+  return xa;
+}
+
 template <int D>
 __global__ void __launch_bounds__(kBlock) k_keys(Fields f, Geo g, const RunGrid* grids, const int* rstate,
                                                  const int* rorder, const int* build, int n, int enforce, int withKeys,
-                                                 int mortonBits, int runBits, uint64_t* keys, uint32_t* vals) {
+                                                 int mortonBits, int runBits, uint64_t* keys, uint32_t* vals, int* flags) {
   const int i = blockIdx.x*blockDim.x + threadIdx.x;
+  if (enforce && i == 0) flags[kFlagWrap] = 0;
   if (i >= n) return;
   const int r = f.run[i];
   uint64_t key = 0;
@@ -64,21 +87,7 @@ __global__ void __launch_bounds__(kBlock) k_keys(Fields f, Geo g, const RunGrid*
   for (int a = 0; a < D; ++a) {
     double xa = f.x[a][i];
     if (enforce) {
-      for (int side = 1; side <= 2; ++side) {
-        const int bc = side == 1 ? (((g.permask >> a) & 1) ? BC_PERIODIC : (((g.reflmask >> (2*a)) & 1) ? BC_REFLECTING : BC_NONE))
-                                 : (((g.permask >> a) & 1) ? BC_PERIODIC : (((g.reflmask >> (2*a + 1)) & 1) ? BC_REFLECTING : BC_NONE));
-        if (bc == BC_NONE) continue;
-        const double thpt = side == 1 ? (xa - g.xmin[a]) : -(xa - g.xmax[a]);
-        const bool fuzzy0 = fabs(thpt) <= 1.0e-15*fmax(1.0, fabs(thpt));
-        if (!fuzzy0 && thpt < 0.0) {
-          if (bc == BC_PERIODIC) {
-            xa = image_coord<D>(bc, side == 1 ? 2 : 1, xa, g.xmin[a], g.xmax[a]);
-          } else {
-            xa = image_coord<D>(bc, side, xa, g.xmin[a], g.xmax[a]);
-            f.v[a][i] = -f.v[a][i];
-          }
-        }
-      }
+      xa = enforce_axis<D>(f, g, a, i, xa);
       f.x[a][i] = xa;
     }
     if (withKeys && build[r]) key |= spread_bits((uint64_t)cell_coord<D>(grids[r], a, xa), D) << a;
@@ -276,9 +285,7 @@ __device__ __forceinline__ void run_min(Scalars* sc, int r, double v, bool valid
 // Packed neighbour records (Fields::xh, Fields::vmr) of the current state, and nodeScale =
 // 1/(lambda_max(H) nPerh) of each node (GenericHydro::dt, Physics/GenericHydro.cc:142-150).
 template <int D>
-__global__ void __launch_bounds__(kBlock) k_pack(Fields f, Phys ph, int n) {
-  const int i = blockIdx.x*blockDim.x + threadIdx.x;
-  if (i >= n) return;
+__device__ __forceinline__ void pack_node(const Fields& f, const Phys& ph, int i) {
   const double h = f.hinv[i];
   double2* P = reinterpret_cast<double2*>(f.xh) + 2*(size_t)i;
   P[0] = make_double2(f.x[0][i], D >= 2 ? f.x[1 % D][i] : 0.0);
@@ -287,6 +294,26 @@ __global__ void __launch_bounds__(kBlock) k_pack(Fields f, Phys ph, int n) {
   V[0] = make_double2(f.v[0][i], D >= 2 ? f.v[1 % D][i] : 0.0);
   V[1] = make_double2(D >= 3 ? f.v[2 % D][i] : 0.0, f.m[i]);
   f.ns[i] = 1.0/max_eigen_iso<D>(h)/ph.nperh;
+}
+template <int D>
+__global__ void __launch_bounds__(kBlock) k_pack(Fields f, Phys ph, int n) {
+  const int i = blockIdx.x*blockDim.x + threadIdx.x;
+  if (i < n) pack_node<D>(f, ph, i);
+}
+constexpr unsigned long long kNoVote = 0xfff0000000000000ull;   // ord_bits(+inf)
+// The start of a steady step in one launch: boundaries enforced where the last step left that
+// pending, records packed, the dt votes and the filter's overflow flag cleared.
+template <int D>
+__global__ void __launch_bounds__(kBlock) k_prepare(Fields f, Geo g, Phys ph, int nTotal, int n, Scalars* sc, int nruns,
+                                                    int* flags) {
+  const int i = blockIdx.x*blockDim.x + threadIdx.x;
+  if (i < nruns) sc[i].dtBits = kNoVote;
+  if (i == 0) flags[kFlagOverflow] = 0;
+  if (i >= nTotal) return;
+  if (flags[kFlagWrap])
+#pragma unroll
+    for (int a = 0; a < D; ++a) f.x[a][i] = enforce_axis<D>(f, g, a, i, f.x[a][i]);
+  if (i < n) pack_node<D>(f, ph, i);
 }
 
 // Position and h^-1 of node j from a 4-double (x, h^-1) record array.
@@ -861,43 +888,55 @@ __global__ void __launch_bounds__(kBlock) k_density_dt(Fields f, Geo g, Phys ph,
 }
 
 // Integrator::selectDt (Integrator/Integrator.cc:116-169), one thread per run.
-__global__ void k_select_dt(Scalars* sc, int nruns, Phys ph, double dtMin, double dtMax, double dtGrowth, int useGravity) {
-  const int r = blockIdx.x*blockDim.x + threadIdx.x;
-  if (r >= nruns) return;
-  Scalars& s = sc[r];
-  s.skinD = 0ull;
-  s.skinG = 0ull;
-  if (!s.active) { s.dt = 0.0; s.hdt = 0.0; return; }
-  const double vote = ord_value(s.dtBits);
-  const double hydro = vote*ph.cfl;
-  s.hydroDt = hydro;
-  const double lo = fmin(dtMin, s.tEnd - s.t), hi = fmin(dtMax, s.tEnd - s.t);
+struct DtLimits { double lo, hi, growth; };
+// Integrator::selectDt from the run's votes.
+__device__ __forceinline__ double choose_dt(const Scalars& s, double hydro, const DtLimits& lim, int useGravity) {
+  const double lo = fmin(lim.lo, s.tEnd - s.t), hi = fmin(lim.hi, s.tEnd - s.t);
   double dt = hi;
   if (hydro > 0.0 && hydro < dt) dt = hydro;
   if (useGravity) {
     const double gd = s.gravDt;
     if (gd > 0.0 && gd < dt) dt = gd;
   }
-  dt = fmin(dt, dtGrowth*s.lastDt);
-  dt = fmin(hi, fmax(lo, dt));
+  dt = fmin(dt, lim.growth*s.lastDt);
+  return fmin(hi, fmax(lo, dt));
+}
+__device__ __forceinline__ void store_dt(Scalars& s, const Phys& ph, const DtLimits& lim, int useGravity) {
+  s.skinD = 0ull;
+  s.skinG = 0ull;
+  if (!s.active) { s.dt = 0.0; s.hdt = 0.0; return; }
+  const double hydro = ord_value(s.dtBits)*ph.cfl;
+  const double dt = choose_dt(s, hydro, lim, useGravity);
+  s.hydroDt = hydro;
   s.dt = dt;
   s.hdt = 0.5*dt;
 }
-
+__global__ void k_select_dt(Scalars* sc, int nruns, Phys ph, DtLimits lim, int useGravity) {
+  const int r = blockIdx.x*blockDim.x + threadIdx.x;
+  if (r < nruns) store_dt(sc[r], ph, lim, useGravity);
+}
 __global__ void k_reset_dt(Scalars* sc, int nruns) {
   const int r = blockIdx.x*blockDim.x + threadIdx.x;
-  if (r < nruns) sc[r].dtBits = 0xfff0000000000000ull;   // ord_bits(+inf)
+  if (r < nruns) sc[r].dtBits = kNoVote;
 }
 
 // Time bookkeeping after a step; a run is done when it reaches its end time.
-__global__ void k_advance_time(Scalars* sc, int nruns) {
+// End of the step: time advance, and the runs' scalars and the overflow flag into the host's memory
+// (the host waits for the stream and reads them: no copies behind the step).
+__global__ void k_advance_time(Scalars* sc, int nruns, Scalars* host, int* flags, int* hostOverflow) {
   const int r = blockIdx.x*blockDim.x + threadIdx.x;
+  if (r == 0) {
+    flags[kFlagWrap] = 1;
+    *hostOverflow = flags[kFlagOverflow];
+  }
   if (r >= nruns) return;
   Scalars& s = sc[r];
-  if (!s.active) return;
-  s.t = s.t + s.dt;
-  s.lastDt = s.dt;
-  s.cycle = s.cycle + 1;
+  if (s.active) {
+    s.t = s.t + s.dt;
+    s.lastDt = s.dt;
+    s.cycle = s.cycle + 1;
+  }
+  host[r] = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -907,10 +946,14 @@ __global__ void k_advance_time(Scalars* sc, int nruns) {
 // IncrementBoundedStateInline.hh; ReplaceBoundedState::updateAsIncrement; GammaLawGas).
 // ---------------------------------------------------------------------------
 template <int D>
-__global__ void __launch_bounds__(kBlock) k_midstep(Fields f, Phys ph, const Scalars* sc, int n) {
+__global__ void __launch_bounds__(kBlock) k_midstep(Fields f, Phys ph, Scalars* sc, int nruns, DtLimits lim, int n) {
   const int i = blockIdx.x*blockDim.x + threadIdx.x;
+  // dt selection: thread r stores run r's, and each node forms its run's from the fields that no
+  // thread stores (one launch instead of two, 5 us of a small run's step)
+  if (i < nruns) store_dt(sc[i], ph, lim, ph.gravity);
   if (i >= n) return;
-  const double hdt = sc[f.run[i]].hdt;
+  const Scalars& s = sc[f.run[i]];
+  const double hdt = 0.5*choose_dt(s, ord_value(s.dtBits)*ph.cfl, lim, ph.gravity);
 #pragma unroll
   for (int a = 0; a < D; ++a) {
     f.xm[a][i] = f.x[a][i] + hdt*f.DxDt[a][i];
@@ -1174,12 +1217,13 @@ __global__ void __launch_bounds__(kBlock) k_finite(Fields f, int n, Scalars* sc)
   if (!ok) atomicOr(&sc[f.run[i]].nonfinite, 1);
 }
 
-// dst[0..n) = value.  Clears flags inside captured step graphs, which hold no memset nodes.
-__global__ void k_fill_int(int* dst, int n, int value) {
-  const int i = blockIdx.x*blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = value;
+// `rows` arrays of n doubles, ld apart (a kernel: a captured graph holds no copies).
+__global__ void __launch_bounds__(kBlock) k_copy_rows(const double* __restrict__ src, double* __restrict__ dst, int64_t n,
+                                                      int64_t ld, int rows) {
+  const int64_t i = (int64_t)blockIdx.x*kBlock + threadIdx.x;
+  if (i < n)
+    for (int c = 0; c < rows; ++c) dst[c*ld + i] = src[c*ld + i];
 }
-
 // dst[0..n) = src[0..n) (doubles): the velocities of the finished runs behind the active ones,
 // which the update does not write, carried into the other velocity buffer.
 __global__ void __launch_bounds__(kBlock) k_copy_doubles(const double* __restrict__ src, double* __restrict__ dst,
