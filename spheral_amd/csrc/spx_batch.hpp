@@ -219,6 +219,8 @@ class Batch {
   int seenNext = 0;
   bool useGraphs = true;
   int64_t graphCaptures = 0, graphReplays = 0, eagerSteps = 0;
+  int nSegments = 0;          // of the rebuilding runs: segments, nodes
+  int64_t nBuild = 0;
   int* dflags = nullptr;      // kFlags
   int* hOverflowG = nullptr;  // the overflow flag of the last step
   // per-class kernel time (ms) summed over the steps since timing was enabled
@@ -265,7 +267,7 @@ class Batch {
     dropGraphs();
     for (void* p : allocs) (void)hipFree(p);
     for (void* p : {(void*)hgrids, (void*)hsc, (void*)hext, (void*)hstate, (void*)hinit, (void*)hOverflow,
-                    (void*)htiles, (void*)hbuild, (void*)hdelta, (void*)hsub})
+                    (void*)htiles, (void*)hbuild, (void*)hdelta, (void*)hsub, (void*)hOverflowG})
       if (p) (void)hipHostFree(p);
     if (gstream) (void)hipStreamSynchronize(gstream);
     grav.release();
@@ -748,6 +750,17 @@ class Batch {
     return a;
   }
 
+  // The rebuilding runs' segments, in position order, with their compacted starts.
+  void buildSegments() {
+    nSegments = 0;
+    nBuild = 0;
+    for (int r : runsByOffset()) {
+      if (!hbuild[r]) continue;
+      hseg[nSegments++] = make_int2((int)runs[r].offset, (int)nBuild);
+      nBuild += runs[r].n;
+    }
+  }
+
   // Runs finished by a step: when their segments are the tail of the active range (the
   // estimated-remaining-steps order puts the soonest to finish last), the active range just
   // shrinks and nothing moves; otherwise the next connectivity pass reorders the batch.
@@ -799,10 +812,16 @@ class Batch {
   // Cell grids of the runs that build candidate lists (hbuild), from their current extents;
   // returns the Morton bits per axis needed.
   int setupGrids() {
-    hipLaunchKernelGGL(k_reset_extent, dim3(nblocks((int64_t)maxRuns*kExt)), dim3(kBlock), 0, stream, dext, maxRuns);
-    int64_t nt = 0;
+    int64_t nt = 0, nsub = 0;
+    int nseg = 0;
     for (int r = 0; r < maxRuns; ++r) {
+      hstate[r] = runs[r].state;
+      hsub[3*r] = (int)runs[r].offset;
+      hsub[3*r + 1] = (int)nsub;
+      hsub[3*r + 2] = nseg;
       if (runs[r].state != RUN_ACTIVE || !hbuild[r]) continue;
+      nsub += runs[r].n;
+      ++nseg;
       const int64_t b = runs[r].offset, e = b + runs[r].n;
       for (int64_t t = b; t < e; t += kExtentTile) {
         htiles[3*nt] = r;
@@ -811,14 +830,20 @@ class Batch {
         ++nt;
       }
     }
+    buildSegments();
+    FetchSet fetch{{hbuild, hstate, hsub, htiles, reinterpret_cast<const int*>(hseg)},
+                   {dbuild, dstate, dsub, dtiles, reinterpret_cast<int*>(dseg)},
+                   {maxRuns, maxRuns, 3*maxRuns, (int)(3*nt), 2*nSegments},
+                   5};
+    hipLaunchKernelGGL(k_fetch, dim3(nblocks(std::max<int64_t>(3*nt, (int64_t)maxRuns*kExt))), dim3(kBlock), 0, stream,
+                       fetch, dext, maxRuns*kExt);
     if (nt > 0) {
-      HIP_CHECK(hipMemcpyAsync(dtiles, htiles, 3*nt*sizeof(int), hipMemcpyHostToDevice, stream));
       launchD([&](auto d) {
         constexpr int DD = decltype(d)::value;
         hipLaunchKernelGGL(k_extent<DD>, dim3((unsigned)nt), dim3(kBlock), 0, stream, f, (const int*)dtiles, dext);
       });
-      HIP_CHECK(hipGetLastError());
     }
+    HIP_CHECK(hipGetLastError());
     download(hext, dext, sizeof(unsigned long long)*maxRuns*kExt);
     const int64_t maxAxis = D == 3 ? (1 << 15) : (D == 2 ? (1 << 20) : (1 << 26));
     int64_t base = 0;
@@ -932,11 +957,12 @@ class Batch {
       cellsAlloc = c;
     }
     nCells = base;
-    HIP_CHECK(hipMemcpyAsync(dgrids, hgrids, sizeof(RunGrid)*maxRuns, hipMemcpyHostToDevice, stream));
-    if (base > 0) {
-      HIP_CHECK(hipMemsetAsync(cellStart, 0, base*sizeof(int), stream));
-      HIP_CHECK(hipMemsetAsync(cellEnd, 0, base*sizeof(int), stream));
-    }
+    static_assert(sizeof(RunGrid) % sizeof(int) == 0);
+    const int words = (int)(sizeof(RunGrid)/sizeof(int))*maxRuns;
+    const FetchSet fetchGrids{{reinterpret_cast<const int*>(hgrids)}, {reinterpret_cast<int*>(dgrids)}, {words}, 1};
+    hipLaunchKernelGGL(k_begin_build, dim3(nblocks(std::max<int64_t>({(int64_t)words, base, nActive}))), dim3(kBlock), 0,
+                       stream, fetchGrids, cellStart, cellEnd, base, tcnt, (int)nActive, dOverflow);
+    HIP_CHECK(hipGetLastError());
     return bits;
   }
 
@@ -966,7 +992,8 @@ class Batch {
     launchD([&](auto d) {
       constexpr int DD = decltype(d)::value;
       hipLaunchKernelGGL(k_keys<DD>, dim3(nb), dim3(kBlock), 0, stream, f, geo, (const RunGrid*)dgrids, (const int*)dstate,
-                         (const int*)dorder, (const int*)dbuild, (int)nTotal, wrapPending ? 1 : 0, 1, mortonBits, runBits, keys, vals, dflags);
+                         (const int*)dorder, (const int*)dbuild, (int)nTotal, wrapPending ? 1 : 0, 1, mortonBits, runBits, keys, vals, dflags,
+                         (const int*)nullptr, (uint64_t*)nullptr, (uint32_t*)nullptr);
     });
     HIP_CHECK(hipGetLastError());
     wrapPending = false;
@@ -1044,34 +1071,18 @@ class Batch {
   void sortRebuildingRuns(int bitsPerAxis) {
     mortonBits = D*bitsPerAxis;
     if (mortonBits + runBits + 2 > 64) raise(SPX_ERR_CAPACITY, "sort key exceeds 64 bits");
-    for (int r = 0; r < maxRuns; ++r) hstate[r] = runs[r].state;
-    HIP_CHECK(hipMemcpyAsync(dstate, hstate, sizeof(int)*maxRuns, hipMemcpyHostToDevice, stream));
+    int segBits = 0;
+    while ((1 << segBits) < nSegments) ++segBits;
+    if (mortonBits + segBits > 64) raise(SPX_ERR_CAPACITY, "sort key exceeds 64 bits");
+    const int64_t nsub = nBuild;
     launchD([&](auto d) {
       constexpr int DD = decltype(d)::value;
       hipLaunchKernelGGL(k_keys<DD>, dim3(nblocks(nTotal)), dim3(kBlock), 0, stream, f, geo, (const RunGrid*)dgrids,
                          (const int*)dstate, (const int*)dorder, (const int*)dbuild, (int)nTotal, wrapPending ? 1 : 0, 1,
-                         mortonBits, runBits, keys, vals, dflags);
+                         mortonBits, runBits, keys, vals, dflags, (const int*)dsub, skeys, spos);
     });
     HIP_CHECK(hipGetLastError());
     wrapPending = false;
-    int nseg = 0;
-    int64_t nsub = 0;
-    for (int r = 0; r < maxRuns; ++r) {
-      hsub[3*r] = (int)runs[r].offset;
-      hsub[3*r + 1] = (int)nsub;
-      hsub[3*r + 2] = nseg;
-      if (!hbuild[r]) continue;
-      nsub += runs[r].n;
-      ++nseg;
-    }
-    if (nseg == 0) return;
-    int segBits = 0;
-    while ((1 << segBits) < nseg) ++segBits;
-    if (mortonBits + segBits > 64) raise(SPX_ERR_CAPACITY, "sort key exceeds 64 bits");
-    HIP_CHECK(hipMemcpyAsync(dsub, hsub, sizeof(int)*3*maxRuns, hipMemcpyHostToDevice, stream));
-    hipLaunchKernelGGL(k_subset_keys, dim3(nblocks(nActive)), dim3(kBlock), 0, stream, (const uint64_t*)keys,
-                       (const int32_t*)f.run, (const int*)dbuild, (const int*)dsub, mortonBits, (int)nActive, skeys, spos);
-    HIP_CHECK(hipGetLastError());
     const int endBit = std::max(1, mortonBits + segBits);
     size_t tmp = 0;
     HIP_CHECK(rocprim::radix_sort_pairs(nullptr, tmp, skeys, skeysAlt, spos, sposAlt, (size_t)nsub, 0, endBit, stream));
@@ -1153,8 +1164,9 @@ class Batch {
       hbuild[r] = 1;
       any = true;
     }
+    const bool reordered = orderDirty;
     if (any || orderDirty) {
-      HIP_CHECK(hipMemcpyAsync(dbuild, hbuild, sizeof(int)*maxRuns, hipMemcpyHostToDevice, stream));
+      if (!any) HIP_CHECK(hipMemcpyAsync(dbuild, hbuild, sizeof(int)*maxRuns, hipMemcpyHostToDevice, stream));
       const int bits = any ? setupGrids() : 0;
       // a change of the batch's composition moves segments: full reorder; otherwise only the
       // rebuilding runs are re-sorted, in place
@@ -1176,27 +1188,24 @@ class Batch {
                            cellStart, cellEnd);
       });
       HIP_CHECK(hipGetLastError());
-      // the rebuilding runs' segments, in position order, with their compacted starts
-      int nseg = 0;
-      int64_t nBuild = 0;
-      for (int r : runsByOffset()) {
-        if (!hbuild[r]) continue;
-        hseg[nseg++] = make_int2((int)runs[r].offset, (int)nBuild);
-        nBuild += runs[r].n;
+      if (reordered) {                              // the segments moved
+        buildSegments();
+        HIP_CHECK(hipMemcpyAsync(dseg, hseg, sizeof(int2)*nSegments, hipMemcpyHostToDevice, stream));
       }
-      HIP_CHECK(hipMemcpyAsync(dseg, hseg, sizeof(int2)*nseg, hipMemcpyHostToDevice, stream));
       bool ok = false;
       for (int attempt = 0; attempt < 4 && !ok; ++attempt) {
-        HIP_CHECK(hipMemsetAsync(dOverflow, 0, 2*sizeof(int), stream));
-        HIP_CHECK(hipMemsetAsync(tcnt, 0, nActive*sizeof(int), stream));
+        if (attempt > 0 || reordered) {             // setupGrids cleared them for the first attempt
+          HIP_CHECK(hipMemsetAsync(dOverflow, 0, 2*sizeof(int), stream));
+          HIP_CHECK(hipMemsetAsync(tcnt, 0, nActive*sizeof(int), stream));
+        }
         launchD([&](auto d) {
           constexpr int DD = decltype(d)::value;
           hipLaunchKernelGGL(k_candidates<DD>, dim3(xcd_grid(nBuild*kSearchLanes, kBlock)), dim3(kBlock), 0, stream, f, geo,
-                             (const RunGrid*)dgrids, (const int2*)dseg, nseg, (int)nBuild, (const int*)cellStart,
+                             (const RunGrid*)dgrids, (const int2*)dseg, nSegments, (int)nBuild, (const int*)cellStart,
                              (const int*)cellEnd, tlist, tcnt, tcap, dOverflow);
         });
         hipLaunchKernelGGL(k_candidates_merge, dim3(xcd_grid(nBuild*kMergeLanes, kBlock)), dim3(kBlock), 0, stream, f, (const int2*)dseg,
-                           nseg, (int)nBuild, (const uint32_t*)tlist, (const int*)tcnt, tcap, dOverflow);
+                           nSegments, (int)nBuild, (const uint32_t*)tlist, (const int*)tcnt, tcap, dOverflow);
         HIP_CHECK(hipGetLastError());
         download(hOverflow, dOverflow, 2*sizeof(int));
         if (hOverflow[0] == 0 && hOverflow[1] == 0) { ok = true; break; }
@@ -1262,7 +1271,7 @@ class Batch {
       constexpr int DD = decltype(d)::value;
       hipLaunchKernelGGL(k_keys<DD>, dim3(nblocks(nTotal)), dim3(kBlock), 0, stream, f, geo, (const RunGrid*)nullptr,
                          (const int*)nullptr, (const int*)nullptr, (const int*)nullptr, (int)nTotal, 1, 0, 0, 0, keys,
-                         vals, dflags);
+                         vals, dflags, (const int*)nullptr, (uint64_t*)nullptr, (uint32_t*)nullptr);
     });
     HIP_CHECK(hipGetLastError());
     wrapPending = false;

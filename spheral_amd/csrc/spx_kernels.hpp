@@ -77,7 +77,8 @@ __device__ __forceinline__ double enforce_axis(const Fields& f, const Geo& g, in
 template <int D>
 __global__ void __launch_bounds__(kBlock) k_keys(Fields f, Geo g, const RunGrid* grids, const int* rstate,
                                                  const int* rorder, const int* build, int n, int enforce, int withKeys,
-                                                 int mortonBits, int runBits, uint64_t* keys, uint32_t* vals, int* flags) {
+                                                 int mortonBits, int runBits, uint64_t* keys, uint32_t* vals, int* flags,
+                                                 const int* sub, uint64_t* skeys, uint32_t* spos) {
   const int i = blockIdx.x*blockDim.x + threadIdx.x;
   if (enforce && i == 0) flags[kFlagWrap] = 0;
   if (i >= n) return;
@@ -92,7 +93,15 @@ __global__ void __launch_bounds__(kBlock) k_keys(Fields f, Geo g, const RunGrid*
     }
     if (withKeys && build[r]) key |= spread_bits((uint64_t)cell_coord<D>(grids[r], a, xa), D) << a;
   }
-  if (withKeys) {
+  if (withKeys && sub) {
+    // only the rebuilding runs' nodes, compacted: run r's go to [sub[3r+1], +n) in position order,
+    // keyed [its segment index | Morton] (sub: per run segment start, compacted start, segment index)
+    if (build[r]) {
+      const int k = sub[3*r + 1] + (i - sub[3*r]);
+      skeys[k] = ((uint64_t)sub[3*r + 2] << mortonBits) | key;
+      spos[k] = (uint32_t)i;
+    }
+  } else if (withKeys) {
     // layout: [rank | run | Morton], rank 0 active (runs by their place rorder), 1 done (by
     // slot); removed runs take the maximum key
     const int st = rstate[r];
@@ -235,22 +244,6 @@ __global__ void __launch_bounds__(kBlock) k_cell_bounds(const uint64_t* keys, co
     if (first || (kp >> sh) != q) { unspread<D>(q, mortonBits, c); start[lin_level_cell<D>(gr, l, ncl, c)] = p; }
     if (last || (kn >> sh) != q) { unspread<D>(q, mortonBits, c); end[lin_level_cell<D>(gr, l, ncl, c)] = p + 1; }
   }
-}
-
-// Sort keys of the particles of the runs that rebuild (build[run] != 0), compacted: run r's
-// particles go to [sub[3r+1], +n) in position order, keyed [its segment index | cell Morton
-// code] (sub: 3 ints per run: segment start, compacted start, segment index).
-__global__ void __launch_bounds__(kBlock) k_subset_keys(const uint64_t* keys, const int32_t* run, const int* build,
-                                                        const int* sub, int mortonBits, int n, uint64_t* skeys,
-                                                        uint32_t* spos) {
-  const int p = blockIdx.x*blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  const int r = run[p];
-  if (!build[r]) return;
-  const int k = sub[3*r + 1] + (p - sub[3*r]);
-  const uint64_t mask = (1ull << mortonBits) - 1ull;
-  skeys[k] = ((uint64_t)sub[3*r + 2] << mortonBits) | (keys[p] & mask);
-  spos[k] = (uint32_t)p;
 }
 
 // Gather over a list of positions: dst[a][pos[k]] = src[a][from ? from[k] : pos[k]], oid alike;
@@ -1201,10 +1194,28 @@ __global__ void __launch_bounds__(kBlock) k_extent(Fields f, const int* tiles, u
   }
 }
 
-__global__ void k_reset_extent(unsigned long long* ext, int nruns) {
-  const int k = blockIdx.x*blockDim.x + threadIdx.x;
-  if (k >= nruns*kExt) return;
-  ext[k] = ext_is_min(k % kExt) ? ~0ull : 0ull;
+// A candidate build's small host arrays into device memory in one launch, read from the host's pinned
+// memory (each copy by itself was 5 to 10 us of a small run's build), and the extents cleared.
+struct FetchSet {
+  const int* src[6];
+  int* dst[6];
+  int n[6];
+  int count;
+};
+__global__ void __launch_bounds__(kBlock) k_fetch(FetchSet s, unsigned long long* ext, int next) {
+  const int i = blockIdx.x*kBlock + threadIdx.x;
+  for (int k = 0; k < s.count; ++k)
+    if (i < s.n[k]) s.dst[k][i] = s.src[k][i];
+  if (i < next) ext[i] = ext_is_min(i % kExt) ? ~0ull : 0ull;
+}
+// Its cell tables, handed-over counts and overflow counts cleared, the grids fetched.
+__global__ void __launch_bounds__(kBlock) k_begin_build(FetchSet grids, int* start, int* end, int64_t cells, int* tcnt,
+                                                        int n, int* overflow) {
+  const int64_t i = (int64_t)blockIdx.x*kBlock + threadIdx.x;
+  if (i < grids.n[0]) grids.dst[0][i] = grids.src[0][i];
+  if (i < cells) start[i] = end[i] = 0;
+  if (i < n) tcnt[i] = 0;
+  if (i < 2) overflow[i] = 0;
 }
 
 // Non-finite guard on the state (NaN/Inf -> per-run status word).
