@@ -66,6 +66,12 @@ static inline double choose_skin(double rate, int D) {
 // mixed 118 -> 118, Taylor-Green 96^3 mixed 170 -> 185, 128^3 FP64 392 -> 493 (the kernel table is
 // staged by four times the blocks, and one lane per node already fills the GPU).
 constexpr int64_t kOmegaWideNodes = 250000;
+// Active particles up to which a step's mixed-precision SPH pass takes four lanes per node (two
+// beyond, the same bits).  2 / 4 lanes: KH 2-D 4096 29.5 / 17.8 us, 32768 37.5 / 28.3, 131072 77.5 /
+// 69.9; Sod 3-D 25k 79.5 / 64.8, 120k 193 / 181; Taylor-Green 3-D 32^3 34.4 / 31.2, 40^3 46.3 / 57.0,
+// 96^3 511 / 625 (lists of 45 leave the fourth lane idle in the last round, and the exchanges cost
+// vector instructions that a full GPU has no slots for).
+static inline int64_t sph_wide_nodes(int D) { return D == 3 ? 40000 : 150000; }
 // Entries in flight per lane of the package-level calls' passes.
 constexpr int kFilterLoads = 2, kUpdateLoads = 2;
 
@@ -1459,8 +1465,9 @@ class Batch {
   // what Integrator::postStateUpdate left: tensor images with grad-h on (SPH asks for boundaries
   // after the Q's copy), zero with it off.  Package calls see boundaries applied.
   void sphPass(bool full, bool withV12 = false, bool stepMid = false) {
-    // lanes per node: from dimension and precision alone
-    const int64_t lanes = mixed ? kSphLanesMixed : D == 1 ? kSphLanes64<1> : D == 2 ? kSphLanes64<2> : kSphLanes64<3>;
+    // lanes per node: from dimension and precision alone, except where the bits do not show them
+    const bool wide = mixed && !full && !limitedQ() && nActive <= sph_wide_nodes(D);
+    const int64_t lanes = wide ? 4 : mixed ? kSphLanesMixed : D == 1 ? kSphLanes64<1> : D == 2 ? kSphLanes64<2> : kSphLanes64<3>;
     const int nb = (int)xcd_grid(nActive*lanes, kBlock);
     Phys ph = this->ph;
     ph.qImages = stepMid ? (cfg.gradh_correction ? 1 : 0) : 1;
@@ -1483,7 +1490,8 @@ class Batch {
         if (mixed) hipLaunchKernelGGL((k_sph<DD, true, float>), dim3(nb), dim3(kBlock), shm, stream, f, geo, ph, dtab, (int)nActive, useLds, sc);
         else hipLaunchKernelGGL((k_sph<DD, true, double>), dim3(nb), dim3(kBlock), shm, stream, f, geo, ph, dtab, (int)nActive, useLds, sc);
       } else {
-        if (mixed) hipLaunchKernelGGL((k_sph<DD, false, float>), dim3(nb), dim3(kBlock), shm, stream, f, geo, ph, dtab, (int)nActive, useLds, sc);
+        if (wide) hipLaunchKernelGGL(k_sph_wide<DD>, dim3(nb), dim3(kBlock), shm, stream, f, geo, ph, dtab, (int)nActive, useLds, sc);
+        else if (mixed) hipLaunchKernelGGL((k_sph<DD, false, float>), dim3(nb), dim3(kBlock), shm, stream, f, geo, ph, dtab, (int)nActive, useLds, sc);
         else hipLaunchKernelGGL((k_sph<DD, false, double>), dim3(nb), dim3(kBlock), shm, stream, f, geo, ph, dtab, (int)nActive, useLds, sc);
       }
     });

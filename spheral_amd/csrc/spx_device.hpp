@@ -84,6 +84,11 @@ __device__ __forceinline__ double quad_swap(double v) {
   return __hiloint2double(hi, lo);
 }
 
+template <int CTRL>
+__device__ __forceinline__ float quad_lane_f(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+
 // A node's sum over its list, L lanes per node.  Ordered: terms are added in list order, as one lane
 // alone would add them, so the lane count never shows in the bits (every lane of the quad adds all
 // four lanes' terms, passed along by DPP).  Otherwise each lane keeps its own partial sum and the

@@ -41,8 +41,12 @@ __device__ __forceinline__ void load_raw(const Fields& f, int j, NbrRaw<D>& q) {
 template <int D, typename R>
 __device__ __forceinline__ void finish_mid(const Geo& g, int code, const NbrRaw<D>& r, Nbr<D, R>& q) {
 #pragma unroll
-  for (int a = 0; a < D; ++a) { q.x[a] = r.x[a]; q.v[a] = refl_sign<D>(g, code, a)*r.v[a]; }
-  if (code) image_pos<D>(g, code, q.x);
+  for (int a = 0; a < D; ++a) { q.x[a] = r.x[a]; q.v[a] = r.v[a]; }
+  if (code) {
+    image_pos<D>(g, code, q.x);
+#pragma unroll
+    for (int a = 0; a < D; ++a) q.v[a] *= refl_sign<D>(g, code, a);
+  }
   q.m = (R)r.m;
   q.rho = (R)r.rho;
   q.cs = (R)r.cs;
@@ -312,7 +316,8 @@ __device__ __forceinline__ void sph_node(const Fields& f, const Geo& g, const Ph
   load_self<D, R>(f, i, S);
   const double Sm = f.m[i], Srho = f.rhom[i], Sh = f.hinvm[i];
 
-  double dvdt[D], dvdx[D*D], Mc[D*D], depsdt = 0.0, maxq = 0.0, m0 = 0.0;
+  double dvdt[D], dvdx[D*D], Mc[D*D], depsdt = 0.0, m0 = 0.0;
+  R maxqr = (R)0;
   double rhosum = 0.0, nrm = 0.0, effq = 0.0, grho[D], m1[D];
 #pragma unroll
   for (int a = 0; a < D; ++a) { dvdt[a] = 0.0; grho[a] = 0.0; m1[a] = 0.0; }
@@ -325,20 +330,21 @@ __device__ __forceinline__ void sph_node(const Fields& f, const Geo& g, const Ph
     for (int a = 0; a < D*D; ++a) TS[a] = (R)f.DvDxQ[a*ld + i];
   }
   const int nn = f.cnt[i];
-  // the next ELL entry and its neighbour's record are fetched one pair ahead
-  uint32_t en = 0;
+  // A neighbour's record is fetched one pair ahead, and its ELL entry two: the record's address is
+  // at hand when its turn comes, instead of a wait for the entry (and all before it) in every pair.
+  uint32_t en = 0, en2 = 0;
   NbrRaw<D> rn;
   if (sub < nn) {
     en = f.nbr[ell_at(sub, i, ld)];
+    if (sub + L < nn) en2 = f.nbr[ell_at(sub + L, i, ld)];
     load_raw<D>(f, (int)(en & kIdxMask), rn);
   }
   for (int k = sub; k < nn; k += L) {
     const uint32_t ent = en;
     const NbrRaw<D> rc = rn;
-    if (k + L < nn) {
-      en = f.nbr[ell_at(k + L, i, ld)];
-      load_raw<D>(f, (int)(en & kIdxMask), rn);
-    }
+    en = en2;
+    if (k + 2*L < nn) en2 = f.nbr[ell_at(k + 2*L, i, ld)];
+    if (k + L < nn) load_raw<D>(f, (int)(en & kIdxMask), rn);
     const int j = (int)(ent & kIdxMask);
     const int code = (int)(ent >> kImgShift);
     Nbr<D, R> O;
@@ -375,7 +381,7 @@ __device__ __forceinline__ void sph_node(const Fields& f, const Geo& g, const Ph
       }
     }
     depsdt += mo*(double)(S.prho*e.vdg + e.workQs);
-    maxq = fmax(maxq, (double)e.Qs);
+    maxqr = fmax(maxqr, e.Qs);
     const R wsph = e.wsphS;
     m0 += (double)wsph;
     if (FULL) {
@@ -391,6 +397,7 @@ __device__ __forceinline__ void sph_node(const Fields& f, const Geo& g, const Ph
     }
   }
 
+  double maxq = (double)maxqr;
   {
     // the pair's partial sums: each lane forms (own + partner's), the same bits on both
 #pragma unroll
@@ -476,20 +483,20 @@ __device__ __forceinline__ void sph_node64(const Fields& f, const Geo& g, const 
       for (int a = 0; a < D*D; ++a) TS[a] = f.DvDxQ[a*ld + i];
     }
     const int nn = f.cnt[i];
-    // the next entry and its neighbour's record are fetched one pair ahead
-    uint32_t en = 0;
+    // the neighbour's record is fetched one pair ahead, its entry two (sph_node)
+    uint32_t en = 0, en2 = 0;
     NbrRaw<D> rn;
     if (sub < nn) {
       en = f.nbr[ell_at(sub, i, ld)];
+      if (sub + L < nn) en2 = f.nbr[ell_at(sub + L, i, ld)];
       load_raw<D>(f, (int)(en & kIdxMask), rn);
     }
     for (int k = sub; k < nn; k += L) {
       const uint32_t ent = en;
       NbrRaw<D> O = rn;
-      if (k + L < nn) {
-        en = f.nbr[ell_at(k + L, i, ld)];
-        load_raw<D>(f, (int)(en & kIdxMask), rn);
-      }
+      en = en2;
+      if (k + 2*L < nn) en2 = f.nbr[ell_at(k + 2*L, i, ld)];
+      if (k + L < nn) load_raw<D>(f, (int)(en & kIdxMask), rn);
       const int code = (int)(ent >> kImgShift);
       if (code) {
         image_pos<D>(g, code, O.x);
@@ -634,16 +641,127 @@ __device__ __forceinline__ void sph_node64(const Fields& f, const Geo& g, const 
   sph_finalize<D, FULL>(f, ph, tab, j, f.cnt[j], t, sc);
 }
 
+// The mixed-precision pass of a step on four lanes per node, with the two-lane pass's bits (above):
+// lanes 0 and 2 form the pairs k = 0, 4, .. and 2, 6, .., lanes 1 and 3 the odd ones, and the sums
+// of the even and of the odd pairs are accumulated in order of k.  To that end each of the two lanes
+// of a parity adds both lanes' terms, but only to half of the sums: the lower to DvDx and DvDt, the
+// upper to M, DepsDt and the zeroth moment.  The pairs' values pass by DPP, 32 exchanges and 12
+// selects per pair; twice the lanes per node halve a node's chain of pairs, which is what a small
+// run waits for.
+template <int D, typename CP>
+__device__ __forceinline__ void sph_node4(const Fields& f, const Geo& g, const Phys& ph, const DevTable& tab, CP coef,
+                                          int n, const Scalars* sc) {
+  using R = float;
+  constexpr int L = 4, LOW = 0x44, UP = 0xEE;       // quad_perm [0,1,0,1] and [2,3,2,3]
+  const int gl = xcd_block()*blockDim.x + threadIdx.x;
+  const int i = gl >> 2, sub = gl & 3;
+  if (i >= n) return;
+  const bool upper = sub >= 2;
+  const size_t ld = (size_t)f.ld;
+  R* pdd = (R*)f.pdd;
+  Nbr<D, R> S;
+  load_self<D, R>(f, i, S);
+  double acc[D*D], ext[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+  for (int a = 0; a < D*D; ++a) acc[a] = 0.0;
+  R maxqr = (R)0;
+  const int nn = f.cnt[i];
+  uint32_t en = 0, en2 = 0;
+  NbrRaw<D> rn;
+  if (sub < nn) {
+    en = f.nbr[ell_at(sub, i, ld)];
+    if (sub + L < nn) en2 = f.nbr[ell_at(sub + L, i, ld)];
+    load_raw<D>(f, (int)(en & kIdxMask), rn);
+  }
+  for (int k = sub; k - sub < nn; k += L) {
+    const uint32_t ent = en;
+    const NbrRaw<D> rc = rn;
+    en = en2;
+    if (k + 2*L < nn) en2 = f.nbr[ell_at(k + 2*L, i, ld)];
+    if (k + L < nn) load_raw<D>(f, (int)(en & kIdxMask), rn);
+    double mo = 0.0;
+    R vso[D], r[D], gs[D], cr[D], dep = (R)0, wsph = (R)0;
+#pragma unroll
+    for (int c = 0; c < D; ++c) vso[c] = r[c] = gs[c] = cr[c] = (R)0;
+    if (k < nn) {
+      const int j = (int)(ent & kIdxMask), code = (int)(ent >> kImgShift);
+      Nbr<D, R> O;
+      finish_mid<D, R>(g, code, rc, O);
+      PairS<D, R> e;
+      pair_eval<D, R>(tab, coef, ph, S, O, code != 0 || i < j, e);
+      pdd[(size_t)k*ld + i] = e.C;
+      mo = rc.m;
+#pragma unroll
+      for (int c = 0; c < D; ++c) { vso[c] = e.vso[c]; r[c] = e.r[c]; gs[c] = e.gs[c]; cr[c] = rounded_product(e.C, e.r[c]); }
+      dep = fused(S.prho, e.vdg, e.workQs);
+      wsph = e.wsphS;
+      maxqr = fmax(maxqr, e.Qs);
+    }
+    auto add = [&](auto from) {
+      const double m = quad_swap<from>(mo);
+      double gd[D];
+#pragma unroll
+      for (int c = 0; c < D; ++c) gd[c] = (double)quad_lane_f<from>(gs[c]);
+#pragma unroll
+      for (int c = 0; c < D; ++c) {
+        const R v = quad_lane_f<from>(vso[c]), x = quad_lane_f<from>(r[c]);
+        const double w = rounded_product(m, (double)(upper ? x : v));
+#pragma unroll
+        for (int d = 0; d < D; ++d) acc[c*D + d] = fused(-w, gd[d], acc[c*D + d]);
+      }
+      // lower: DvDt -= m C r; upper: DepsDt += m dep, m0 += wsph
+      const R de = quad_lane_f<from>(dep), ws = quad_lane_f<from>(wsph);
+#pragma unroll
+      for (int c = 0; c < D; ++c) {
+        const R q = quad_lane_f<from>(cr[c]);
+        if (c == 0) ext[0] = fused(-m, (double)(upper ? -de : q), ext[0]);
+        else if (c == 1) ext[1] = fused(upper ? -1.0 : -m, (double)(upper ? -ws : q), ext[1]);
+        else ext[2] = fused(-m, (double)q, ext[2]);
+      }
+      if (D == 1) ext[1] = fused(-1.0, (double)(upper ? -ws : (R)0), ext[1]);
+    };
+    add(std::integral_constant<int, LOW>{});
+    add(std::integral_constant<int, UP>{});
+  }
+  // even + odd, then the upper lanes' half to the lower ones
+  double maxq = (double)maxqr;
+  maxq = fmax(maxq, quad_swap<0xB1>(maxq));
+  maxq = fmax(maxq, quad_swap<0x4E>(maxq));
+  SphSums<D> q;
+#pragma unroll
+  for (int a = 0; a < D*D; ++a) {
+    acc[a] += quad_swap<0xB1>(acc[a]);
+    q.dvdx[a] = acc[a];
+    q.M[a] = quad_swap<0x4E>(acc[a]);
+  }
+#pragma unroll
+  for (int a = 0; a < 3; ++a) ext[a] += quad_swap<0xB1>(ext[a]);
+  q.depsdt = quad_swap<0x4E>(ext[0]);
+  q.m0 = quad_swap<0x4E>(ext[1]);
+  if (sub != 0) return;
+#pragma unroll
+  for (int a = 0; a < D; ++a) { q.dvdt[a] = ext[a]; q.grho[a] = 0.0; q.m1[a] = 0.0; }
+  q.maxq = maxq;
+  q.rhosum = q.nrm = q.effq = 0.0;
+  sph_finalize<D, false>(f, ph, tab, i, nn, q, sc);
+}
+
 // Lanes per node of the SPH pass.  The choice depends only on the configuration (dimension,
 // precision), never on the particle count, so a run gives the same bits in any batch.  FP64, us per
 // pass with 1 / 2 / 4 lanes: Sod 1-D 400 9.2 / 7.5 / 6.5, Noh 1-D 100 14.3 / 10.4 / 7.8, KH 2-D 65536
-// 71.9 / 46.7 / 41.5, Taylor-Green 37^3 56.4 / 39.8 / 41.8, 128^3 1451 / 1309 / 1385 (before, with two
+// 71.9 / 46.7 / 41.5, Taylor-Green 37^3 56.4 / 39.8 / 41.8, 128^3 1451 / 1309 / 1385; with the list
+// entries read two pairs ahead 6.3, 7.5, 40.2, 37.7 and 1269 (before, with two
 // sides' divisions, two reciprocal square roots and canonical-order selects per pair: 8.0, 10.6,
 // 53.8, 64 and 1406).  On large 3-D runs the pass is bound by the records' gathers: 96 bytes per
 // neighbour, 9 GB through the L1s of which most misses them.
 template <int D>
 constexpr int kSphLanes64 = D == 3 ? 2 : 4;
 constexpr int kSphLanesMixed = 2;
+template <int D>
+__global__ void __launch_bounds__(kBlock, 3) k_sph_wide(Fields f, Geo g, Phys ph, DevTable tab, int n, int ldsTable,
+                                                        const Scalars* sc) {
+  with_table<float>(tab, ldsTable, [&](auto coef) { sph_node4<D>(f, g, ph, tab, coef, n, sc); });
+}
 template <int D, bool FULL, typename R, bool LQ = false>
 __global__ void __launch_bounds__(kBlock, 3) k_sph(Fields f, Geo g, Phys ph, DevTable tab, int n, int ldsTable,
                                                    const Scalars* sc) {
