@@ -1509,11 +1509,9 @@ class Batch {
     grav.stream = forked ? gstream : stream;
     double* xs[3] = {mid ? f.xm[0] : f.x[0], mid ? f.xm[1] : f.x[1], mid ? f.xm[2] : f.x[2]};
     grav.build(xs, f.m, (int)nActive);
+    grav.prepareWalk(cfg.opening, cfg.softening);
     if (!forked) mark("tree_build");
-    if (forked) {
-      grav.prepareWalk(cfg.opening, cfg.softening);
-      HIP_CHECK(hipEventRecord(evTree, gstream));
-    }
+    else HIP_CHECK(hipEventRecord(evTree, gstream));
     grav.evaluate(f.DvDtG, f.pot, (int)nActive, cfg.G, cfg.softening, cfg.opening, dsc, cfg.ftimestep);
     if (toState)
       HIP_CHECK(hipMemcpyAsync(f.potS, f.pot, nActive*sizeof(double), hipMemcpyDeviceToDevice, grav.stream));

@@ -761,7 +761,7 @@ __global__ void __launch_bounds__(kBlock) k_tree_walk(
       phi = DIM == 3 ? fused(-Mc, ri, phi) : phi - Mc*(0.5*log(rs));
       if (COUNT) ++nCell;
     }
-    if (COUNT && mine && !acts && kind == kCellPoint && r2 > self2) ++nPoint;
+    if (COUNT && mine && own < ncells && !acts && kind == kCellPoint && r2 > self2) ++nPoint;
     if (list) {
       const int q1 = last[own];
       for (int q = first[own]; q <= q1; ++q) {

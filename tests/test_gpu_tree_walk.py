@@ -13,7 +13,7 @@ ALONE = 98304          # largest count whose points walk by themselves
 SOFT = 0.01
 
 
-def evaluate(gpu, x, m, opening, hinv=None):
+def tree_run(gpu, x, m, opening, hinv=None):
     n, dim = x.shape
     hinv = hinv or n**(1.0/dim)
     cfg = abi.default_config(dim, nperh=2.01)
@@ -24,6 +24,11 @@ def evaluate(gpu, x, m, opening, hinv=None):
     r = gpu.make_run(cfg, dict(x=x, v=np.zeros((n, dim)), m=m, rho=np.ones(n), eps=np.zeros(n), H=H))
     r.initialize()
     r.evaluate_derivatives()
+    return r
+
+
+def evaluate(gpu, x, m, opening, hinv=None):
+    r = tree_run(gpu, x, m, opening, hinv)
     return r.field("delta velocity"), r.field("gravitational potential")
 
 
@@ -129,3 +134,17 @@ def test_the_two_sorts_give_the_same_bits(gpu):
     a, p = evaluate(gpu, x, m, 1.0)
     a1, p1 = evaluate(gpu, np.concatenate([x, [[-0.9, 0.9, 0.9]]]), np.append(m, 1.0e-200), 1.0)
     assert np.array_equal(a, a1[:-1]) and np.array_equal(p, p1[:-1])
+
+
+@pytest.mark.parametrize("n", [3, 65, 2051])
+def test_interaction_counts(gpu, n):
+    """Opened all the way, a walk's interactions are the pairs of points farther apart than the screen."""
+    print(f"[case] counts of {n} points", flush=True)
+    x = ball(n, 3, seed=n)
+    x[n//2] = x[0]
+    r = tree_run(gpu, x, np.full(n, 1.0/n), 1.0e-9)
+    r2 = ((x[:, None, :] - x[None, :, :])**2).sum(2)
+    before = r.field("delta velocity")
+    assert tuple(r.gravity_interactions()) == (0, int((r2/SOFT**2 > 1.0e-10).sum()))
+    r.evaluate_derivatives()
+    assert np.array_equal(r.field("delta velocity"), before)
