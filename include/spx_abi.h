@@ -298,10 +298,10 @@ int spx_run_gravity_interactions(spx_run* run, int64_t* out2);
 /* Step execution (no counterpart in the reference, whose Integrator::step is plain host
    calls).  A CheapSynchronousRK2 step in which no candidate list is rebuilt, no run is
    admitted, finished or removed and no field was read since the previous step is replayed
-   from a HIP graph captured on its first occurrence (one launch instead of about fifteen);
+   from a HIP graph captured on its first occurrence (one launch instead of seven or more);
    its results are the eager step's bit for bit.  Enabled by default; enable = 0 runs every
-   step eagerly (and drops the captured graphs).  TreeGravity, the Limited Q and
-   SynchronousRK2 steps always run eagerly. */
+   step eagerly (and drops the captured graphs).  SynchronousRK2 steps and steps
+   with TreeGravity over more than 262144 points always run eagerly. */
 int spx_run_set_step_graphs(spx_run* run, int32_t enable);
 /* No counterpart in the reference (an evaluation-schedule switch).  The grad-h Omega that
    SPHBase::postStateUpdate leaves at the end of a CheapSynchronousRK2 step (SPHBase.cc:526-551)
