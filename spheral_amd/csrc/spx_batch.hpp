@@ -22,6 +22,7 @@
 #include <rocprim/rocprim.hpp>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -228,7 +229,7 @@ class Batch {
   int nSegments = 0;          // of the rebuilding runs: segments, nodes
   int64_t nBuild = 0;
   int* dflags = nullptr;      // kFlags
-  int* hOverflowG = nullptr;  // the overflow flag of the last step
+  int* hflags = nullptr;      // the last step's, written by its last kernel
   // per-class kernel time (ms) summed over the steps since timing was enabled
   bool timing = false;
   // TreeGravity's own stream and its fork / join events (gravity runs only)
@@ -273,7 +274,7 @@ class Batch {
     dropGraphs();
     for (void* p : allocs) (void)hipFree(p);
     for (void* p : {(void*)hgrids, (void*)hsc, (void*)hext, (void*)hstate, (void*)hinit, (void*)hOverflow,
-                    (void*)htiles, (void*)hbuild, (void*)hdelta, (void*)hsub, (void*)hOverflowG})
+                    (void*)htiles, (void*)hbuild, (void*)hdelta, (void*)hsub, (void*)hflags})
       if (p) (void)hipHostFree(p);
     if (gstream) (void)hipStreamSynchronize(gstream);
     grav.release();
@@ -503,7 +504,7 @@ class Batch {
     dOverflow = dalloc<int>(2);
     dflags = dalloc<int>(kFlags);
     HIP_CHECK(hipMemsetAsync(dflags, 0, kFlags*sizeof(int), stream));
-    hOverflowG = halloc<int>(1);
+    hflags = halloc<int>(kFlags);
     dbuild = dalloc<int>(maxRuns);
     dsub = dalloc<int>(3*(size_t)maxRuns);
     skeys = dalloc<uint64_t>(ld);
@@ -1690,7 +1691,7 @@ class Batch {
     HIP_CHECK(hipGetLastError());
     mark("update");
     hipLaunchKernelGGL(k_advance_time, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns, hsc, dflags,
-                       hOverflowG);
+                       hflags);
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipStreamSynchronize(stream));        // k_advance_time wrote the runs' scalars to hsc
     collectTimes();
@@ -1848,7 +1849,7 @@ class Batch {
     mark("energy_update");
     wrapPending = true;
     hipLaunchKernelGGL(k_advance_time, dim3(nblocks(maxRuns)), dim3(kBlock), 0, stream, dsc, maxRuns, hsc, dflags,
-                       hOverflowG);
+                       hflags);
     HIP_CHECK(hipGetLastError());
   }
   // Host bookkeeping once the step's run scalars are downloaded.
@@ -1879,8 +1880,8 @@ class Batch {
   // active particle count is unchanged (the velocity arrays alternate between two buffers).  That
   // part is captured as a HIP graph per buffer parity and replayed: one launch instead of seven
   // (seventeen with gravity), and the end of the step reaches the host's memory from its last
-  // kernel.  A small run's step is these launches: 1-D Limited-Q Noh of 100 nodes 172 -> 102 us per
-  // step, 1-D Sod of 400 137 -> 107.  The graph holds no memset, no copy and no host
+  // kernel.  A small run's step is these launches: 1-D Limited-Q Noh of 100 nodes 104 -> 61 us per
+  // step, 1-D Sod of 400 82 -> 64.  The graph holds no memset, no copy and no host
   // synchronisation, and with the neighbour lists sized to the candidate lists' capacity the filter
   // cannot overflow (a node's neighbours are a subset of its candidates).  Results are the eager
   // step's bit for bit.  Steps with newly admitted runs, trees whose build waits on the host,
@@ -1905,11 +1906,12 @@ class Batch {
     put(&ph, sizeof(ph));
     put(&geo, sizeof(geo));
     put(&dtab, sizeof(dtab));
-    const void* bufs[] = {keys, vals, dsc, dflags, hsc, hOverflowG};
+    const void* bufs[] = {keys, vals, dsc, dflags, hsc, hflags};
     put(bufs, sizeof(bufs));
     return k;
   }
   void dropGraphs() {
+    if (stream) (void)hipStreamSynchronize(stream);
     for (auto& g : graphs) {
       if (g.exec) (void)hipGraphExecDestroy(g.exec);
       if (g.graph) (void)hipGraphDestroy(g.graph);
@@ -1935,7 +1937,24 @@ class Batch {
     midpointDerivatives();
     fullStepLaunches();
   }
+  // Waits for the steady step queued when the host's step count was `before`: polls that count for
+  // up to a millisecond, then waits on the stream.  A wait on the stream returns some 10 us after the
+  // last kernel's end, a sixth of a small run's step (Sod 1-D 400 59 -> 50 us, KH 4k 117 -> 107,
+  // Taylor-Green 37^3 195 -> 185).  Every 64th step waits on the stream, so that the runtime's
+  // bookkeeping of finished launches stays bounded.
+  void awaitStep(int before) {
+    if (nblocks(maxRuns) == 1 && (before & 63) != 0) {
+      const auto start = std::chrono::steady_clock::now();
+      for (int spin = 1; __atomic_load_n(&hflags[kFlagStep], __ATOMIC_ACQUIRE) == before; ++spin) {
+        __builtin_ia32_pause();
+        if (spin % 256 == 0 && std::chrono::steady_clock::now() - start > std::chrono::milliseconds(1)) break;
+      }
+      if (__atomic_load_n(&hflags[kFlagStep], __ATOMIC_ACQUIRE) != before) return;
+    }
+    HIP_CHECK(hipStreamSynchronize(stream));
+  }
   void graphStep() {
+    const int before = hflags[kFlagStep];
     connectivityPrep(false, true);
     if (nActive == 0) { applyPendingBoundaries(); return; }
     ensureNbrCapacity(f.ccap);          // every candidate fits: the filter cannot overflow
@@ -1959,8 +1978,8 @@ class Batch {
       connValid = true;
       npairsCache = -1;
       wrapPending = true;
-      HIP_CHECK(hipStreamSynchronize(stream));
-      if (*hOverflowG != 0) raise(SPX_ERR_STATE, "neighbour list overflow in a steady step");
+      awaitStep(before);
+      if (hflags[kFlagOverflow] != 0) raise(SPX_ERR_STATE, "neighbour list overflow in a steady step");
       tunerStepDone();
       endOfStep();
       return;
@@ -1968,7 +1987,10 @@ class Batch {
     if (!g) {
       StepGraph& c = graphs[graphNext];
       graphNext ^= 1;
-      if (c.exec) HIP_CHECK(hipGraphExecDestroy(c.exec));
+      if (c.exec) {
+        HIP_CHECK(hipStreamSynchronize(stream));      // its last replay was polled for, not waited on
+        HIP_CHECK(hipGraphExecDestroy(c.exec));
+      }
       if (c.graph) HIP_CHECK(hipGraphDestroy(c.graph));
       c.exec = nullptr;
       c.graph = nullptr;
@@ -1999,8 +2021,8 @@ class Batch {
     connValid = true;
     npairsCache = -1;
     wrapPending = true;
-    HIP_CHECK(hipStreamSynchronize(stream));
-    if (*hOverflowG != 0) raise(SPX_ERR_STATE, "neighbour list overflow in a replayed step");
+    awaitStep(before);
+    if (hflags[kFlagOverflow] != 0) raise(SPX_ERR_STATE, "neighbour list overflow in a replayed step");
     tunerStepDone();
     endOfStep();
   }

@@ -327,9 +327,9 @@ struct Scalars {
   int nonfinite, pad;
 };
 
-// A batch's device flags: the filter's overflow in steady steps, and whether the last step's
-// positions still await the boundaries.
-enum : int { kFlagOverflow = 0, kFlagWrap = 1, kFlags = 2 };
+// A batch's device flags: the filter's overflow in steady steps, whether the last step's positions
+// still await the boundaries, and the count of steps (32 bits, wraps).
+enum : int { kFlagOverflow = 0, kFlagWrap = 1, kFlagStep = 2, kFlags = 3 };
 
 // Order-preserving map between doubles and unsigned 64-bit integers (for atomic min/max).
 __device__ __forceinline__ unsigned long long ord_bits(double d) {

@@ -914,30 +914,33 @@ __global__ void k_reset_dt(Scalars* sc, int nruns) {
 }
 
 // Time bookkeeping after a step; a run is done when it reaches its end time.
-// End of the step: time advance, and the runs' scalars and the overflow flag into the host's memory
-// (the host waits for the stream and reads them: no copies behind the step).
-__global__ void k_advance_time(Scalars* sc, int nruns, Scalars* host, int* flags, int* hostOverflow) {
+// End of the step: time advance, and the runs' scalars and the overflow flag into the host's memory,
+// then the number of the step, which tells a host that polls for it that all of it is there (one
+// block writes them; with more than one, the host waits for the stream).
+__global__ void k_advance_time(Scalars* sc, int nruns, Scalars* host, int* flags, int* hostFlags) {
   const int r = blockIdx.x*blockDim.x + threadIdx.x;
   if (r == 0) {
     flags[kFlagWrap] = 1;
-    *hostOverflow = flags[kFlagOverflow];
+    hostFlags[kFlagOverflow] = flags[kFlagOverflow];
   }
-  if (r >= nruns) return;
-  Scalars& s = sc[r];
-  if (s.active) {
-    s.t = s.t + s.dt;
-    s.lastDt = s.dt;
-    s.cycle = s.cycle + 1;
+  if (r < nruns) {
+    Scalars& s = sc[r];
+    if (s.active) {
+      s.t = s.t + s.dt;
+      s.lastDt = s.dt;
+      s.cycle = s.cycle + 1;
+    }
+    host[r] = s;
   }
-  host[r] = s;
+  if (gridDim.x > 1) return;
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int step = flags[kFlagStep] + 1;
+    flags[kFlagStep] = step;
+    __hip_atomic_store(&hostFlags[kFlagStep], step, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
-
-// ---------------------------------------------------------------------------
-// CheapSynchronousRK2 mid-step: state.update with timeAdvanceOnly (increments with
-// the previous step's derivatives), then the EOS policies
-// (Integrator/CheapSynchronousRK2.cc:74-77; DataBase/IncrementStateInline.hh:42-80,
-// IncrementBoundedStateInline.hh; ReplaceBoundedState::updateAsIncrement; GammaLawGas).
-// ---------------------------------------------------------------------------
 template <int D>
 __global__ void __launch_bounds__(kBlock) k_midstep(Fields f, Phys ph, Scalars* sc, int nruns, DtLimits lim, int n) {
   const int i = blockIdx.x*blockDim.x + threadIdx.x;

@@ -41,3 +41,21 @@ def test_replayed_steps_equal_launched_steps(gpu, name):
             assert np.array_equal(a.field("gravitational potential"), b.field("gravitational potential"))
     sa, sb = a.step_stats(), b.step_stats()
     assert sa["graph_replays"] > 0 and sb["graph_replays"] == 0
+
+
+def test_a_batch_of_many_slots_waits_on_the_stream(gpu):
+    """The host polls for a step's end when one block writes the runs' scalars; with more than 256
+    slots several do, and it waits on the stream.  The same steps either way."""
+    print("[case] 1 and 300 slots", flush=True)
+    cfg, st = problems.kelvin_helmholtz_2d(4096)
+    out = []
+    for slots in (1, 300):
+        b = gpu.Batch(cfg, capacity=len(st["m"]), max_runs=slots)
+        rid = b.add_run(st, 1.0)
+        for _ in range(70):                      # past a step that waits on the stream by its number
+            b.step()
+        assert b.step_stats()["graph_replays"] > 0
+        out.append([b.field(rid, f) for f in FIELDS] + [b.status(rid)["t"]])
+        b.close()
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
