@@ -1284,6 +1284,13 @@ class Batch {
     wrapPending = false;
   }
 
+  // A state that replaces the stepped one has no boundaries pending: the device's flag, which a steady
+  // step reads, goes with the host's.
+  void dropPendingBoundaries() {
+    wrapPending = false;
+    HIP_CHECK(hipMemsetAsync(dflags + kFlagWrap, 0, sizeof(int), stream));
+  }
+
   // ---------------------------------------------------------------- passes (over the active runs)
   template <typename K64, typename K32, typename... Args>
   void launchPrec(K64 k64, K32 k32, int nb, Args... args) {

@@ -260,7 +260,8 @@ int spx_run_set_state(spx_run* run, const double* x, const double* v, const doub
     run->haveState = false;
     B.runs[0] = spx::Batch::RunInfo();
     B.nTotal = B.nActive = 0;
-    B.connValid = B.initialized = B.wrapPending = false;
+    B.connValid = B.initialized = false;
+    B.dropPendingBoundaries();
     B.addRun(x, v, m, rho, eps, H, run->n, std::numeric_limits<double>::infinity(), 0);
     run->haveState = true;
   });
