@@ -343,9 +343,28 @@ __host__ __device__ inline double ord_value(unsigned long long u) {
   return d;
 }
 
-__device__ __forceinline__ double dmul(double a, double b) { return __dmul_rn(a, b); }
-__device__ __forceinline__ double dadd(double a, double b) { return __dadd_rn(a, b); }
-__device__ __forceinline__ double dsub(double a, double b) { return __dsub_rn(a, b); }
+// Each operation rounded by itself, never part of a fused multiply-add (this ROCm's __dmul_rn and
+// __dadd_rn are plain operators, which the compiler contracts).
+__device__ __forceinline__ double dmul(double a, double b) { return rounded_product(a, b); }
+__device__ __forceinline__ double dadd(double a, double b) {
+#pragma clang fp contract(off)
+  return a + b;
+}
+__device__ __forceinline__ double dsub(double a, double b) {
+#pragma clang fp contract(off)
+  return a - b;
+}
+// |h r|^2 as the neighbour criterion rounds it: every product and every sum by itself, in axis order.
+template <int D>
+__device__ __forceinline__ double eta2(double h, const double* r) {
+  double s = 0.0;
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    const double e = dmul(h, r[a]);
+    s = a == 0 ? dmul(e, e) : dadd(s, dmul(e, e));
+  }
+  return s;
+}
 
 // Ghost coordinate of an image along one axis, written in the reference's
 // mapPositionThroughPlanes arithmetic for axis-aligned planes through the origin of

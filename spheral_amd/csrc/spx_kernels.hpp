@@ -564,15 +564,10 @@ __global__ void __launch_bounds__(kBlock, 8) k_candidates(Fields f, Geo g, const
         acc = r2 <= reach2;
       }
       if (acc) {
-        double e[D];
-#pragma unroll
-        for (int a = 0; a < D; ++a) e[a] = dmul(hi, rr[a]);
-        acc = norm2<D>(e) <= ext2c;
+        acc = eta2<D>(hi, rr) <= ext2c;
         if (acc) {
           const double hj = f.hinv[j];
-#pragma unroll
-          for (int a = 0; a < D; ++a) e[a] = dmul(hj, rr[a]);
-          if (!(norm2<D>(e) <= ext2c)) {
+          if (!(eta2<D>(hj, rr) <= ext2c)) {
             // j's own support does not reach i: j receives the pair from here
             const int slot = atomicAdd(&tcnt[j], 1);
             if (slot < tcap) tlist[ell_at(slot, j, ld)] = (uint32_t)i | ((uint32_t)inverse_image(g, code) << kImgShift);
@@ -731,14 +726,7 @@ __device__ __forceinline__ bool neighbor_test(const Geo& g, double ext2, const d
 #pragma unroll
     for (int a = 0; a < D; ++a) rr[a] = dsub(xi[a], xk[a]);
   }
-  const double hm = fmin(hi, hj);
-  double e2 = 0.0;
-#pragma unroll
-  for (int a = 0; a < D; ++a) {
-    const double e = dmul(hm, rr[a]);
-    e2 = a == 0 ? dmul(e, e) : dadd(e2, dmul(e, e));
-  }
-  return e2 <= ext2 && !(self && code == 0);
+  return eta2<D>(fmin(hi, hj), rr) <= ext2 && !(self && code == 0);
 }
 
 // U: entries in flight per lane.
