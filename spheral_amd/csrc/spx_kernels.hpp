@@ -408,6 +408,12 @@ __device__ __forceinline__ int build_pos(const int2* seg, int nseg, int k) {
 // 3041 (instruction issue: 8 waves per SIMD and the test's ~80 instructions per candidate; at 79
 // VGPRs and 6 waves 3167).  8 lanes: Sod 451, Evrard 2494, Taylor-Green 4245.
 constexpr int kSearchLanes = 16, kSearchCells = 32;
+// The largest capacity that a pass with too short lists asks for.  Read first: where most nodes
+// overflow, as in a run's first build, an atomic per wavefront of 4 or 16 nodes queued at one word
+// (KH 2-D 262144, first build: search 770 -> 215 us, filter 206 -> 48).
+__device__ __forceinline__ void ask_capacity(int* need, int v) {
+  if (v > __hip_atomic_load(need, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(need, v);
+}
 template <int D>
 __global__ void __launch_bounds__(kBlock, 8) k_candidates(Fields f, Geo g, const RunGrid* grids, const int2* seg, int nseg,
                                                        int nBuild, const int* cstart, const int* cend, uint32_t* tlist,
@@ -583,7 +589,7 @@ __global__ void __launch_bounds__(kBlock, 8) k_candidates(Fields f, Geo g, const
   }
   if (sub == 0) {
     f.ccnt[i] = count;
-    if (count > cap) atomicMax(overflow, count);
+    if (count > cap) ask_capacity(overflow, count);
   }
 }
 
@@ -617,12 +623,12 @@ __global__ void __launch_bounds__(kBlock) k_candidates_merge(Fields f, const int
   const int t = tcnt[i];
   if (t == 0) return;
   if (t > tcap) {
-    if (sub == 0) atomicMax(&overflow[1], t);
+    if (sub == 0) ask_capacity(&overflow[1], t);
     return;
   }
   const int c0 = f.ccnt[i];
   if (c0 + t > f.ccap) {
-    if (sub == 0) atomicMax(&overflow[0], c0 + t);
+    if (sub == 0) ask_capacity(&overflow[0], c0 + t);
     return;
   }
   const size_t ld = (size_t)f.ld;
@@ -826,7 +832,7 @@ __device__ __forceinline__ void density_dt_node(const Fields& f, const Geo& g, c
     }
     if (FILT && sub == 0) {
       f.cnt[i] = count;
-      if (count > f.cap) atomicMax(overflow, count);
+      if (count > f.cap) ask_capacity(overflow, count);
     }
     double rho = rhos.total();
     if (DT) {
