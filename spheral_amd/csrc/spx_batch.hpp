@@ -589,7 +589,7 @@ class Batch {
   }
 
   template <typename F>
-  void launchD(F&& fn) {
+  void launchD(F&& fn) const {
     switch (D) {
       case 1: fn(std::integral_constant<int, 1>{}); break;
       case 2: fn(std::integral_constant<int, 2>{}); break;
@@ -656,17 +656,25 @@ class Batch {
     HIP_CHECK(hipStreamSynchronize(stream));
   }
   // The caller's state checked (H isotropic and positive, mass and density positive); returns h^-1.
-  std::vector<double> checkState(const double* m, const double* rho, const double* H, int64_t n) const {
-    std::vector<double> hinv((size_t)n);
+  // The dimension is a constant of the loop: with it at run time, Taylor-Green 128^3's update_state
+  // took 29.0 ms instead of 13.0.
+  template <int DD>
+  static bool stateValid(const double* m, const double* rho, const double* H, int64_t n, double* hinv) {
     bool ok = true;
     for (int64_t i = 0; i < n; ++i) {
-      const double* Hi = H + i*D*D;
+      const double* Hi = H + i*DD*DD;
       const double h = Hi[0];
       bool iso = true;
-      for (int c = 0; c < D*D; ++c) iso &= Hi[c] == (c % (D + 1) == 0 ? h : 0.0);
+      for (int c = 0; c < DD*DD; ++c) iso &= Hi[c] == (c % (DD + 1) == 0 ? h : 0.0);
       ok &= iso & (h > 0.0) & (h <= 1.7976931348623157e308) & (m[i] > 0.0) & (rho[i] > 0.0);
       hinv[i] = h;
     }
+    return ok;
+  }
+  std::vector<double> checkState(const double* m, const double* rho, const double* H, int64_t n) const {
+    std::vector<double> hinv((size_t)n);
+    bool ok = false;
+    launchD([&](auto d) { ok = stateValid<decltype(d)::value>(m, rho, H, n, hinv.data()); });
     if (ok) return hinv;
     for (int64_t i = 0; i < n; ++i) {
       const double* Hi = H + i*D*D;
@@ -1287,8 +1295,8 @@ class Batch {
   // A state that replaces the stepped one has no boundaries pending: the device's flag, which a steady
   // step reads, goes with the host's.
   void dropPendingBoundaries() {
+    if (wrapPending) HIP_CHECK(hipMemsetAsync(dflags + kFlagWrap, 0, sizeof(int), stream));
     wrapPending = false;
-    HIP_CHECK(hipMemsetAsync(dflags + kFlagWrap, 0, sizeof(int), stream));
   }
 
   // ---------------------------------------------------------------- passes (over the active runs)
