@@ -131,7 +131,6 @@ __global__ void __launch_bounds__(kBlock) k_gather(GatherSet s, const uint32_t* 
 struct RecordSet {
   double* a[9];
   int nc;          // components per record
-  int iso;         // > 0: the record is a[0] times the iso x iso identity (NC = iso^2)
 };
 __device__ __forceinline__ int64_t node_of(const int64_t* oid, int64_t slot0, int64_t k) {
   return oid ? oid[slot0 + k] & (((int64_t)1 << 40) - 1) : k;
@@ -144,12 +143,7 @@ __global__ void __launch_bounds__(kBlock) k_to_records(RecordSet s, double* __re
   const int64_t node = node_of(oid, slot0, k);
   if (node < c0 || node >= c1) return;
   double* out = stage + (node - c0)*s.nc;
-  if (s.iso) {
-    const double h = s.a[0][slot0 + k];
-    for (int c = 0; c < s.nc; ++c) out[c] = c % (s.iso + 1) == 0 ? h : 0.0;
-  } else {
-    for (int c = 0; c < s.nc; ++c) out[c] = s.a[c][slot0 + k];
-  }
+  for (int c = 0; c < s.nc; ++c) out[c] = s.a[c][slot0 + k];
 }
 __global__ void __launch_bounds__(kBlock) k_from_records(RecordSet s, const double* __restrict__ stage,
                                                          const int64_t* __restrict__ oid, int64_t slot0, int64_t n,
