@@ -762,8 +762,17 @@ __global__ void __launch_bounds__(kBlock, 3) k_sph_wide(Fields f, Geo g, Phys ph
                                                         const Scalars* sc) {
   with_table<float>(tab, ldsTable, [&](auto coef) { sph_node4<D>(f, g, ph, tab, coef, n, sc); });
 }
+// Wavefronts per SIMD that a variant's registers are cut for: three (168 VGPRs), or two where three
+// spill and two measured faster.  Three / two: evaluate_derivatives with the Limited Q, Taylor-Green
+// 48^3 mixed 449 / 231 us, FP64 679 / 218, 96^3 2540 / 1450 and 4810 / 1380, without it 713 / 659
+// and 801 / 764, KH 65536 FP64 with it 143 / 119; the step's 3-D FP64 pass with it 48^3 414 / 160,
+// 96^3 2540 / 1145.  The step's other variants with the Limited Q (2-D FP64: 8 spilled, 3-D mixed:
+// 38) stay at three: KH 262144 190 / 196, Taylor-Green 96^3 1135 / 1334.
+constexpr int sph_waves(int D, bool full, bool fp64, bool lq) {
+  return (D == 3 && (full || (fp64 && lq))) || (D == 2 && full && fp64 && lq) ? 2 : 3;
+}
 template <int D, bool FULL, typename R, bool LQ = false>
-__global__ void __launch_bounds__(kBlock, 3) k_sph(Fields f, Geo g, Phys ph, DevTable tab, int n, int ldsTable,
+__global__ void __launch_bounds__(kBlock, (sph_waves(D, FULL, sizeof(R) == sizeof(double), LQ))) k_sph(Fields f, Geo g, Phys ph, DevTable tab, int n, int ldsTable,
                                                    const Scalars* sc) {
   if constexpr (sizeof(R) == sizeof(float)) {
     with_table<float>(tab, ldsTable, [&](auto coef) { sph_node<D, FULL, LQ>(f, g, ph, tab, coef, n, sc); });
