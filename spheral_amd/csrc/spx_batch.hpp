@@ -1923,6 +1923,7 @@ class Batch {
     put(&dtab, sizeof(dtab));
     const void* bufs[] = {keys, vals, dsc, dflags, hsc, hflags};
     put(bufs, sizeof(bufs));
+    put(&grav.cellsAllocs, sizeof(grav.cellsAllocs));       // its other arrays stay as constructed
     return k;
   }
   void dropGraphs() {

@@ -24,6 +24,7 @@
 
 #include <rocprim/rocprim.hpp>
 
+#include <algorithm>
 #include <vector>
 
 #include "spx_device.hpp"
@@ -846,6 +847,7 @@ class GravityTree {
   int64_t cellCap = 0;
   TreeCell* cells = nullptr;        // the walk's cell records
   int *first = nullptr, *last = nullptr;
+  int cellsAllocs = 0;              // how often they were allocated
   int npts = 0;                     // points of the tree (0: none yet)
   // opening^2 (< 0: none) and self-screen radius^2 that the cell records were formed for
   double cellsOpen2 = -1.0, cellsSelf2 = 0.0;
@@ -912,9 +914,22 @@ class GravityTree {
     allocs.clear();
   }
 
+  // Room for `need` cells.  The arrays that became too small are given back (the tree's launches on
+  // them have been waited for), and cellsAllocs tells a captured step that its pointers are old.
   void ensureCells(int64_t need) {
     if (need <= cellCap) return;
     const int64_t cap = cellCap ? need + need/4 + 1024 : need;
+    HIP_CHECK(hipStreamSynchronize(stream));
+    for (void* p : {(void*)cells, (void*)first, (void*)last}) {
+      if (!p) continue;
+      allocs.erase(std::find(allocs.begin(), allocs.end(), p));
+      HIP_CHECK(hipFree(p));
+    }
+    bytes -= cellCap*(int64_t)(sizeof(TreeCell) + 2*sizeof(int));
+    cellCap = 0;
+    cells = nullptr;
+    first = last = nullptr;
+    ++cellsAllocs;
     first = alloc<int>(cap);
     last = alloc<int>(cap);
     cells = alloc<TreeCell>(cap);
