@@ -807,7 +807,10 @@ __device__ __forceinline__ void density_dt_node(const Fields& f, const Geo& g, c
             R d[D], gw, graw;
 #pragma unroll
             for (int a = 0; a < D; ++a) d[a] = (R)hj[u]*(R)rr[u][a];
-            kernel_wgw_c<R>(coef, tab, sqrt(norm2<D>(d)), hdet_iso<D, R>((R)hj[u]), w, gw, graw);
+            // (in mixed precision the package-level sum starts most chains from the second axis:
+            // the last FP32 bit it has always had)
+            const R s = !FILT && sizeof(R) == sizeof(float) && !(D == 3 && sub == 0) ? norm2_second<D>(d) : norm2<D>(d);
+            kernel_wgw_c<R>(coef, tab, sqrt(s), hdet_iso<D, R>((R)hj[u]), w, gw, graw);
           }
           if (DT) {
             double d[D];
