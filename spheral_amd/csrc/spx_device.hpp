@@ -446,8 +446,8 @@ __device__ __forceinline__ void kernel_wgw_c(CP coef, const DevTable& t, R eta, 
   b = b < t.n1 ? b : t.n1;
   const CP c = coef + 6*b;
   const bool in = eta < (R)t.extent;
-  const R wv = hdet*(c[0] + (c[1] + c[2]*eta)*eta);
-  const R gr = c[3] + (c[4] + c[5]*eta)*eta;
+  const R wv = hdet*fused(fused(c[2], eta, c[1]), eta, c[0]);
+  const R gr = fused(fused(c[5], eta, c[4]), eta, c[3]);
   w = in ? wv : (R)0;
   graw = in ? gr : (R)0;
   gw = in ? hdet*gr : (R)0;

@@ -76,11 +76,16 @@ __device__ __forceinline__ void load_self(const Fields& f, int i, Nbr<D, R>& s) 
 // the identity, so the pairwise acceleration (SPH.cc:428) is one scalar times r:
 //   pacc_ab / (-m_b) = C r_ab,   C = ((P_a k_a + P_b k_b) + Q_a k_a / 2) + Q_b k_b / 2
 // (P = safeInv(Omega) P / rho^2, Q = the Q's QPi).  C is formed in that canonical order from
-// quantities both lanes compute with the same operations on the same operands (r and the
-// velocity jump change sign exactly), so both lanes hold the same C bits and each lane's
-// C*r_lane is the exact negation of the other's: the pairwise acceleration is bitwise
-// antisymmetric.  C per neighbour entry is all the compatible-energy update needs besides the
-// positions, which it re-forms with the same operations.
+// quantities both lanes compute on the same operands (r and the velocity jump change sign exactly),
+// so without viscosity both lanes hold the same C bits and each lane's C*r_lane is the exact negation
+// of the other's.  The Q's own term is fused the one way and the partner's the other (the results
+// programs have had are held to the bit), so an approaching pair's two C differ by FP32 rounding: the
+// momentum rate of a Gresho vortex is 2e-9 of the sum of m|a|, KH 4096 1e-10.  (FP64 forms C by
+// operations that commute in the two nodes, sph_node64.)  C per neighbour entry is all the
+// compatible-energy update needs besides the positions, which it re-forms with the same operations.
+//
+// Sums whose contraction the compiler may choose are spelled out here, in kernel_wgw_c and in the
+// accumulations of sph_node: sph_node4, chosen by the count of active nodes, has the same bits.
 template <int D, typename R>
 struct PairS {
   R r[D], vso[D], gs[D], es[D];
@@ -134,16 +139,15 @@ template <int D, typename R, bool LQ = false, typename CP>
 __device__ __forceinline__ void pair_eval(const DevTable& tab, CP coef, const Phys& ph, const Nbr<D, R>& S,
                                           const Nbr<D, R>& O, bool aFirst, PairS<D, R>& e,
                                           const R* TS = nullptr, const R* TO = nullptr) {
-  R e2s = (R)0, e2o = (R)0;
+  R eo[D];
 #pragma unroll
   for (int c = 0; c < D; ++c) {
     e.r[c] = (R)(S.x[c] - O.x[c]);
     e.es[c] = S.h*e.r[c];
-    const R eoc = O.h*e.r[c];
-    e2s += e.es[c]*e.es[c];
-    e2o += eoc*eoc;
+    eo[c] = O.h*e.r[c];
     e.vso[c] = (R)(S.v[c] - O.v[c]);
   }
+  const R e2s = norm2<D>(e.es), e2o = norm2<D>(eo);
   // |eta| and safeInvVar(|eta|) = 1/max(1e-30, |eta|) from one reciprocal square root each
   const R tiny = (R)1.0e-30f;
   const R is = e2s > tiny*tiny ? rsqrt(e2s) : (R)1/tiny, io = e2o > tiny*tiny ? rsqrt(e2o) : (R)1/tiny;
@@ -158,7 +162,7 @@ __device__ __forceinline__ void pair_eval(const DevTable& tab, CP coef, const Ph
 #pragma unroll
   for (int c = 0; c < D; ++c) {
     e.gs[c] = ks*e.r[c];
-    vsr += e.vso[c]*e.r[c];
+    vsr = fused(e.vso[c], e.r[c], vsr);
   }
   // velocity jump the Q sees: the plain difference, or the limited midpoint extrapolation
   R vqr = vsr;
@@ -169,14 +173,14 @@ __device__ __forceinline__ void pair_eval(const DevTable& tab, CP coef, const Ph
   const R mus = (S.h*vqr)/(e2s + (R)1.0e-2), muo = (O.h*vqr)/(e2o + (R)1.0e-2);
   const R mms = fmin((R)0, mus), mmo = fmin((R)0, muo);
   const R Cl = (R)ph.Cl, Cq = (R)ph.Cq;
-  const R es_ = -Cl*S.cs*mms + Cq*(mms*mms);
-  const R eo_ = -Cl*O.cs*mmo + Cq*(mmo*mmo);
+  const R es_ = fused(-Cl*S.cs, mms, Cq*(mms*mms));
+  const R eo_ = fused(Cq, mmo*mmo, -(Cl*O.cs*mmo));
   const R QPs = es_*S.irho, QPo = eo_*O.irho;
   e.Qs = S.rho*es_;
   const R p1 = aFirst ? S.prho : O.prho, p2 = aFirst ? O.prho : S.prho;
   const R k1 = aFirst ? ks : ko, k2 = aFirst ? ko : ks;
   const R q1 = aFirst ? QPs : QPo, q2 = aFirst ? QPo : QPs;
-  e.C = ((p1*k1 + p2*k2) + (R)0.5*(q1*k1)) + (R)0.5*(q2*k2);
+  e.C = fused((R)0.5, q2*k2, fused((R)0.5, q1*k1, fused(p1, k1, p2*k2)));
   e.vdg = ks*vsr;                                            // v_so . gradW_s
   e.workQs = (R)0.5*(QPs*e.vdg);                             // v_so . (QPi_s gradW_s / 2)
 }
@@ -371,16 +375,16 @@ __device__ __forceinline__ void sph_node(const Fields& f, const Geo& g, const Ph
     const double mo = rc.m;
 #pragma unroll
     for (int c = 0; c < D; ++c) {
-      dvdt[c] -= mo*(double)(e.C*e.r[c]);
+      dvdt[c] = fused(-mo, (double)(e.C*e.r[c]), dvdt[c]);
       const double mv = mo*(double)e.vso[c], mr = mo*(double)e.r[c];
 #pragma unroll
       for (int d = 0; d < D; ++d) {
-        dvdx[c*D + d] -= mv*(double)e.gs[d];
+        dvdx[c*D + d] = fused(-mv, (double)e.gs[d], dvdx[c*D + d]);
         // (the FP32 pair terms round r_c g_d and r_d g_c differently: all of M is accumulated)
-        Mc[c*D + d] -= mr*(double)e.gs[d];
+        Mc[c*D + d] = fused(-mr, (double)e.gs[d], Mc[c*D + d]);
       }
     }
-    depsdt += mo*(double)(S.prho*e.vdg + e.workQs);
+    depsdt = fused(mo, (double)fused(S.prho, e.vdg, e.workQs), depsdt);
     maxqr = fmax(maxqr, e.Qs);
     const R wsph = e.wsphS;
     m0 += (double)wsph;
