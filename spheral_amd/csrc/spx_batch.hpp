@@ -62,11 +62,18 @@ static inline double choose_skin(double rate, int D) {
   return best;
 }
 
-// Active particles up to which the grad-h pass takes four lanes per node (one lane beyond): KH 2-D
-// 4096 mixed 24 -> 11.6 us, Sod 3-D 25k mixed 71 -> 32.5, KH 65536 FP64 27.4 -> 20.4, Evrard 250k
-// mixed 118 -> 118, Taylor-Green 96^3 mixed 170 -> 185, 128^3 FP64 392 -> 493 (the kernel table is
-// staged by four times the blocks, and one lane per node already fills the GPU).
-constexpr int64_t kOmegaWideNodes = 250000;
+// Active particles up to which the grad-h pass takes four lanes per node (one lane beyond, the same
+// bits).  With 65536 nodes one lane per node is one wavefront per SIMD; four lanes gain where one
+// leaves a node's chain of pairs exposed, and lose where the GPU is full, by staging the kernel table
+// four times as often.  The lines are two wavefronts per SIMD in 1-D and 2-D and below four in 3-D,
+// whose lists are longer.  One / four lanes, us per pass, FP64: KH 65544 30.1 / 22.1, 131798 33.9 /
+// 32.4, 165562 35.6 / 36.5, 262716 44.0 / 51.1; Sod 2-D 100217 21.0 / 23.4, 199763 27.9 / 34.6;
+// Taylor-Green 48^3 38.1 / 35.5, 56^3 43.5 / 43.6, 63^3 52.0 / 56.2, 64^3 53.0 / 58.8, 80^3 105 /
+// 121; Evrard 220000 111 / 104, 250000 114 / 116, 280000 139 / 130; Sod 3-D 122018 76.4 / 64.1,
+// 248832 119 / 111, 395136 186 / 175.  Mixed: KH 131798 31.5 / 29.5, 165562 32.1 / 32.1, 262716 38.9 /
+// 43.4; Sod 2-D 149781 22.8 / 25.8; Taylor-Green 56^3 41.1 / 39.4, 64^3 51.9 / 53.7, 80^3 103 / 109;
+// Evrard 250000 113 / 112; Sod 3-D 248832 118 / 102, 802797 338 / 310.
+static inline int64_t omega_wide_nodes(int D) { return D == 3 ? (1 << 18) - 1 : 1 << 17; }
 // Active particles up to which a step's mixed-precision SPH pass takes four lanes per node (two
 // beyond, the same bits).  2 / 4 lanes: KH 2-D 4096 29.5 / 17.8 us, 32768 37.5 / 28.3, 131072 77.5 /
 // 69.9; Sod 3-D 25k 79.5 / 64.8, 120k 193 / 181; Taylor-Green 3-D 32^3 34.4 / 31.2, 40^3 46.3 / 57.0,
@@ -1356,7 +1363,7 @@ class Batch {
                         geo, dtab, (int)nActive, (const double*)(M ? f.xhm : f.xh), M ? f.omegam : f.omega, runMask);
       };
       auto pick = [&](auto m) {
-        if (nActive <= kOmegaWideNodes) go(std::integral_constant<int, kNodeLanes>{}, m);
+        if (nActive <= omega_wide_nodes(D)) go(std::integral_constant<int, kNodeLanes>{}, m);
         else go(std::integral_constant<int, 1>{}, m);
       };
       if (mid) pick(std::true_type{});

@@ -1004,7 +1004,7 @@ __global__ void __launch_bounds__(kBlock) k_eos(Fields f, Phys ph, int n) {
 // (optional): only nodes of runs with a non-zero entry are updated.
 // ---------------------------------------------------------------------------
 // L lanes per node, U entries in flight per lane; the sums are in list order for either L, so the
-// choice by particle count (kOmegaWideNodes) changes no bit.
+// choice by particle count (omega_wide_nodes) changes no bit.
 template <int D, typename R, bool MID, int U, int L, typename CP>
 __device__ __forceinline__ void omega_node(const Fields& f, const Geo& g, const DevTable& tab, CP coef, int n,
                                            const double* xh, double* omega, const int* runMask) {
