@@ -75,11 +75,14 @@ static inline double choose_skin(double rate, int D) {
 // Evrard 250000 113 / 112; Sod 3-D 248832 118 / 102, 802797 338 / 310.
 static inline int64_t omega_wide_nodes(int D) { return D == 3 ? (1 << 18) - 1 : 1 << 17; }
 // Active particles up to which a step's mixed-precision SPH pass takes four lanes per node (two
-// beyond, the same bits).  2 / 4 lanes: KH 2-D 4096 29.5 / 17.8 us, 32768 37.5 / 28.3, 131072 77.5 /
-// 69.9; Sod 3-D 25k 79.5 / 64.8, 120k 193 / 181; Taylor-Green 3-D 32^3 34.4 / 31.2, 40^3 46.3 / 57.0,
-// 96^3 511 / 625 (lists of 45 leave the fourth lane idle in the last round, and the exchanges cost
-// vector instructions that a full GPU has no slots for).
-static inline int64_t sph_wide_nodes(int D) { return D == 3 ? 40000 : 150000; }
+// beyond, the same bits).  In 3-D its registers allow three wavefronts per SIMD, 49152 nodes at 16
+// per wavefront: up to there all of them run at once, and one more node is another round, while two
+// lanes hold twice as many.  2 / 4 lanes, us per pass: Sod 3-D 25k 79.5 / 64.8, 48608 93.6 / 77.5,
+// 49392 96.1 / 96.0, 55303 99.4 / 102.9, 120k 176 / 173, 250k 310 / 341; Evrard 49000 95.6 / 80.1,
+// 52000 94.2 / 103.0; Taylor-Green 32^3 34.4 / 31.2, 36^3 45.5 / 39.8, 37^3 45.8 / 52.7, 96^3 511 / 625.
+// In 2-D the line is a mean over lists: KH 4096 29.5 / 17.8, 131798 76.3 / 68.5, 262716 120 / 116,
+// 600k 276 / 287; Sod 2-D 109850 46.0 / 44.8, 149781 52.5 / 53.7, 262064 76.8 / 83.3.
+static inline int64_t sph_wide_nodes(int D) { return D == 3 ? 49152 : 150000; }
 // Entries in flight per lane of the package-level calls' passes.
 constexpr int kFilterLoads = 2, kUpdateLoads = 2;
 
