@@ -287,7 +287,8 @@ class Batch {
     dropGraphs();
     for (void* p : allocs) (void)hipFree(p);
     for (void* p : {(void*)hgrids, (void*)hsc, (void*)hext, (void*)hstate, (void*)hinit, (void*)hOverflow,
-                    (void*)htiles, (void*)hbuild, (void*)hdelta, (void*)hsub, (void*)hflags})
+                    (void*)htiles, (void*)hbuild, (void*)hdelta, (void*)hsub, (void*)hflags, (void*)hseg,
+                    (void*)horder})
       if (p) (void)hipHostFree(p);
     if (gstream) (void)hipStreamSynchronize(gstream);
     grav.release();
