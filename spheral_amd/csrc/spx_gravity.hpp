@@ -39,8 +39,8 @@ struct TreeBox { double lo[3], box; };       // cube of the tree: lower corner, 
 
 // Points up to which the keys are sorted by the sample sort below, and cells are allocated for the
 // worst case (kTreeBits per point): building then takes no wait on the host, and the step is replayed
-// from a graph.  The line bounds that worst case, 1.1 KB per point of which a usual tree fills a
-// twelfth: 294 MB at 2^18.  Beyond it, the library's radix sort and a download of the cell count.
+// from a graph.  The line bounds that worst case, 1.1 KB per point (usual trees have 1.4 to 1.7 of
+// its 20 cells), 294 MB at 2^18.  Beyond it, the library's radix sort and a download of the cell count.
 // It is no crossover: own / library, Evrard, build 117 / 177 us at 131k, 146 / 232 at 262k, 155 / 259
 // at 300k, 286 / 381 at 800k, a step 1.34 / 1.47, 2.22 / 2.40, 2.55 / 2.83 and 6.41 / 6.65 ms.
 constexpr int kTreeOwnSort = 1 << 18;
