@@ -76,16 +76,15 @@ template <int Q>
 __device__ __forceinline__ double quad_lane(double v) {
   return __hiloint2double(quad_lane<Q>(__double2hiint(v)), quad_lane<Q>(__double2loint(v)));
 }
-// quad_perm CTRL of a double: 0xB1 swaps neighbouring lanes, 0x4E swaps the halves of a quad.
+// quad_perm CTRL: 0xB1 swaps neighbouring lanes, 0x4E swaps the halves of a quad.
 template <int CTRL>
 __device__ __forceinline__ double quad_swap(double v) {
   const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, false);
   const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, false);
   return __hiloint2double(hi, lo);
 }
-
 template <int CTRL>
-__device__ __forceinline__ float quad_lane_f(float v) {
+__device__ __forceinline__ float quad_swap(float v) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, false));
 }
 

@@ -195,13 +195,6 @@ __device__ __forceinline__ void pair_eval(const DevTable& tab, CP coef, const Ph
 // pair loop makes three lookups per pair at scattered intervals).  sc != nullptr (the step):
 // the node's half-step velocity record for the compatible-energy update is written too (as
 // k_v12 would, with the run's dt/2).
-__device__ __forceinline__ double lane_pair_swap(double v) {
-  const int lo = __double2loint(v), hi = __double2hiint(v);
-  // quad_perm [1, 0, 3, 2]: lane 2m reads lane 2m+1 and vice versa
-  const int lo2 = __builtin_amdgcn_mov_dpp(lo, 0xB1, 0xf, 0xf, false);
-  const int hi2 = __builtin_amdgcn_mov_dpp(hi, 0xB1, 0xf, 0xf, false);
-  return __hiloint2double(hi2, lo2);
-}
 
 // A node's sums over its pairs.
 template <int D>
@@ -405,23 +398,23 @@ __device__ __forceinline__ void sph_node(const Fields& f, const Geo& g, const Ph
   {
     // the pair's partial sums: each lane forms (own + partner's), the same bits on both
 #pragma unroll
-    for (int a = 0; a < D; ++a) dvdt[a] += lane_pair_swap(dvdt[a]);
+    for (int a = 0; a < D; ++a) dvdt[a] += quad_swap<0xB1>(dvdt[a]);
 #pragma unroll
     for (int c = 0; c < D; ++c)
 #pragma unroll
       for (int d = 0; d < D; ++d) {
-        dvdx[c*D + d] += lane_pair_swap(dvdx[c*D + d]);
-        Mc[c*D + d] += lane_pair_swap(Mc[c*D + d]);
+        dvdx[c*D + d] += quad_swap<0xB1>(dvdx[c*D + d]);
+        Mc[c*D + d] += quad_swap<0xB1>(Mc[c*D + d]);
       }
-    depsdt += lane_pair_swap(depsdt);
-    m0 += lane_pair_swap(m0);
-    maxq = fmax(maxq, lane_pair_swap(maxq));
+    depsdt += quad_swap<0xB1>(depsdt);
+    m0 += quad_swap<0xB1>(m0);
+    maxq = fmax(maxq, quad_swap<0xB1>(maxq));
     if (FULL) {
-      rhosum += lane_pair_swap(rhosum);
-      nrm += lane_pair_swap(nrm);
-      effq += lane_pair_swap(effq);
+      rhosum += quad_swap<0xB1>(rhosum);
+      nrm += quad_swap<0xB1>(nrm);
+      effq += quad_swap<0xB1>(effq);
 #pragma unroll
-      for (int a = 0; a < D; ++a) { grho[a] += lane_pair_swap(grho[a]); m1[a] += lane_pair_swap(m1[a]); }
+      for (int a = 0; a < D; ++a) { grho[a] += quad_swap<0xB1>(grho[a]); m1[a] += quad_swap<0xB1>(m1[a]); }
     }
     if (sub != 0) return;
   }
@@ -705,19 +698,19 @@ __device__ __forceinline__ void sph_node4(const Fields& f, const Geo& g, const P
       const double m = quad_swap<from>(mo);
       double gd[D];
 #pragma unroll
-      for (int c = 0; c < D; ++c) gd[c] = (double)quad_lane_f<from>(gs[c]);
+      for (int c = 0; c < D; ++c) gd[c] = (double)quad_swap<from>(gs[c]);
 #pragma unroll
       for (int c = 0; c < D; ++c) {
-        const R v = quad_lane_f<from>(vso[c]), x = quad_lane_f<from>(r[c]);
+        const R v = quad_swap<from>(vso[c]), x = quad_swap<from>(r[c]);
         const double w = rounded_product(m, (double)(upper ? x : v));
 #pragma unroll
         for (int d = 0; d < D; ++d) acc[c*D + d] = fused(-w, gd[d], acc[c*D + d]);
       }
       // lower: DvDt -= m C r; upper: DepsDt += m dep, m0 += wsph
-      const R de = quad_lane_f<from>(dep), ws = quad_lane_f<from>(wsph);
+      const R de = quad_swap<from>(dep), ws = quad_swap<from>(wsph);
 #pragma unroll
       for (int c = 0; c < D; ++c) {
-        const R q = quad_lane_f<from>(cr[c]);
+        const R q = quad_swap<from>(cr[c]);
         if (c == 0) ext[0] = fused(-m, (double)(upper ? -de : q), ext[0]);
         else if (c == 1) ext[1] = fused(upper ? -1.0 : -m, (double)(upper ? -ws : q), ext[1]);
         else ext[2] = fused(-m, (double)q, ext[2]);
