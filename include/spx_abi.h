@@ -312,12 +312,12 @@ int spx_run_set_step_graphs(spx_run* run, int32_t enable);
    every step, as the reference's integrator does. */
 int spx_run_set_end_of_step_omega(spx_run* run, int32_t eager);
 /* Neighbour-group sizes of the filtering sum-density pass, the grad-h passes and the
-   compatible-energy update (sizes[0..3), each 4 or 8: how many neighbours' loads a lane
-   issues before using them).  Every size gives the same result bits.  By default (sizes null
-   or sizes[0] <= 0) the engine measures: after two warm-up steps it alternates 4 and 8 per
-   pass over six steps, timing each, moves a pass off its default (8, 8, 8) only when the
-   other size is at least 3 % faster, and measures again once the active particle count has
-   changed by more than 2x. */
+   compatible-energy update (sizes[0..3), each 4 or 8: how many neighbours' loads a node's
+   lanes issue between them before using any).  Every size gives the same result bits.  By
+   default (sizes null or sizes[0] <= 0) the engine measures: after two warm-up steps it
+   alternates 4 and 8 per pass over six steps, timing each, moves a pass off its default
+   (8, 8, 8) only when the other size is at least 3 % faster, and measures again once the
+   active particle count has changed by more than 2x. */
 int spx_run_set_group_sizes(spx_run* run, const int32_t* sizes);
 /* out9: graph captures, graph replays, eager steps, group-size measurements, current sizes of
    the three passes, whole-batch reorders, steps whose finished runs retired without a reorder

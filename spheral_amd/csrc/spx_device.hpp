@@ -29,8 +29,8 @@ __host__ __device__ __forceinline__ size_t ell_at(int k, int i, size_t ld) {
 // requested before any is used, so a wavefront waits on memory once per group instead of twice per
 // neighbour.  With four lanes per node a group is G/4 entries of each lane.  Defaults of the
 // filtering sum-density pass, the energy update and the grad-h passes (a batch measures 4 against 8);
-// Taylor-Green 128^3 FP64 per step: filter 8 -> 1.08 ms, 4 -> 1.40; update 0.82 / 0.83; grad-h (one
-// lane per node there) 0.39 / 0.44.
+// Taylor-Green 128^3 FP64 per step, 8 / 4: connectivity with the filter 1.13 / 1.33 ms; update 0.82 /
+// 0.83; grad-h (one lane per node there) 0.39 / 0.43.
 constexpr int kGroup = 8;
 constexpr int kGroupUpdate = 8;
 constexpr int kGroupOmega = 8;

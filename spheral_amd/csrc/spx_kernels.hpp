@@ -1,11 +1,12 @@
 // spx_kernels.hpp -- neighbour build and the light pair passes of the SPH hot path.
 //
-// Every pair pass is a gather: one lane per target particle walks its ELLPACK
-// neighbour list and accumulates only its own sums, so no atomics touch the
-// conserved quantities.  Where a pair term must be bitwise antisymmetric (the
-// pairwise acceleration and the compatible-energy partition) both lanes evaluate
-// the pair in one canonical (a, b) order: an image partner makes the gathering
-// node "a" (the reference's internal-ghost pair), otherwise the lower slot is "a".
+// Every pair pass is a gather: one to four lanes per target particle walk its ELLPACK
+// neighbour list and accumulate only its own sums, so no atomics touch the
+// conserved quantities.  Where a pair term must agree from both sides (the pairwise
+// acceleration and the compatible-energy partition) FP64 forms it by operations that
+// commute in the two nodes; mixed precision evaluates the pair in one canonical (a, b)
+// order: an image partner makes the gathering node "a" (the reference's internal-ghost
+// pair), otherwise the lower slot is "a".
 //
 // A batch holds independent runs of one problem type; particle i belongs to run
 // f.run[i] with its own cell grid (RunGrid) and time step (Scalars).  Pairs never
@@ -332,8 +333,8 @@ __device__ __forceinline__ void load_vm(const double* vm, int j, double* v, doub
 //
 // Two stages.  k_candidates builds, for the runs whose list is stale, a candidate list
 // with the criterion widened to ext (1 + skin): a few lanes per particle walk the cells its
-// widened support reaches.  It records the positions and h^-1 the list was built from.  The filtering pass (k_density_dt) applies the exact criterion to the
-// candidates every step.  The candidates stay complete while no pair can have closed in from beyond the
+// widened support reaches.  It records the positions and h^-1 the list was built from.  The
+// filtering pass (k_density_dt) applies the exact criterion to the candidates every step.  The candidates stay complete while no pair can have closed in from beyond the
 // widened radius: with D = max |x - xb| hb/ext and G = max hb/h^-1 over the run's nodes,
 // |rij(now)| <= max(Si, Sj)(now) implies |rij(built)| <= max(Si, Sj)(built) (G + 2D), so a
 // list is valid while G + 2D <= 1 + skin (the full update measures both after every step).
@@ -901,8 +902,7 @@ __global__ void k_reset_dt(Scalars* sc, int nruns) {
   if (r < nruns) sc[r].dtBits = kNoVote;
 }
 
-// Time bookkeeping after a step; a run is done when it reaches its end time.
-// End of the step: time advance, and the runs' scalars and the overflow flag into the host's memory,
+// End of the step: time advance (a run is done when it reaches its end time), and the runs' scalars and the overflow flag into the host's memory,
 // then the number of the step, which tells a host that polls for it that all of it is there (one
 // block writes them; with more than one, the host waits for the stream).
 __global__ void k_advance_time(Scalars* sc, int nruns, Scalars* host, int* flags, int* hostFlags) {
@@ -929,6 +929,14 @@ __global__ void k_advance_time(Scalars* sc, int nruns, Scalars* host, int* flags
     __hip_atomic_store(&hostFlags[kFlagStep], step, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
+
+// ---------------------------------------------------------------------------
+// CheapSynchronousRK2 mid-step: state.update with timeAdvanceOnly (increments with
+// the previous step's derivatives), then the EOS policies
+// (Integrator/CheapSynchronousRK2.cc:74-77; DataBase/IncrementStateInline.hh:42-80,
+// IncrementBoundedStateInline.hh; ReplaceBoundedState::updateAsIncrement; GammaLawGas),
+// preceded by the dt selection.
+// ---------------------------------------------------------------------------
 template <int D>
 __global__ void __launch_bounds__(kBlock) k_midstep(Fields f, Phys ph, Scalars* sc, int nruns, DtLimits lim, int n) {
   const int i = blockIdx.x*blockDim.x + threadIdx.x;

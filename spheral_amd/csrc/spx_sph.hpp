@@ -80,8 +80,8 @@ __device__ __forceinline__ void load_self(const Fields& f, int i, Nbr<D, R>& s) 
 // so without viscosity both lanes hold the same C bits and each lane's C*r_lane is the exact negation
 // of the other's.  The Q's own term is fused the one way and the partner's the other (the results
 // programs have had are held to the bit), so an approaching pair's two C differ by FP32 rounding: the
-// momentum rate of a Gresho vortex is 2e-9 of the sum of m|a|, KH 4096 1e-10.  (FP64 forms C by
-// operations that commute in the two nodes, sph_node64.)  C per neighbour entry is all the
+// momentum rate of a Gresho vortex is 2e-9 of the sum of m|a|, of KH 4096 with random velocities 1e-10.
+// (FP64 forms C by operations that commute in the two nodes, sph_node64.)  C per neighbour entry is all the
 // compatible-energy update needs besides the positions, which it re-forms with the same operations.
 //
 // Sums whose contraction the compiler may choose are spelled out here, in kernel_wgw_c and in the
@@ -744,7 +744,8 @@ __device__ __forceinline__ void sph_node4(const Fields& f, const Geo& g, const P
 }
 
 // Lanes per node of the SPH pass.  The choice depends only on the configuration (dimension,
-// precision), never on the particle count, so a run gives the same bits in any batch.  FP64, us per
+// precision), so a run gives the same bits in any batch; k_sph_wide, which a mixed-precision step takes
+// by the particle count, has the two-lane pass's bits.  FP64, us per
 // pass with 1 / 2 / 4 lanes: Sod 1-D 400 9.2 / 7.5 / 6.5, Noh 1-D 100 14.3 / 10.4 / 7.8, KH 2-D 65536
 // 71.9 / 46.7 / 41.5, Taylor-Green 37^3 56.4 / 39.8 / 41.8, 128^3 1451 / 1309 / 1385; with the list
 // entries read two pairs ahead 6.3, 7.5, 40.2, 37.7 and 1269 (before, with two
@@ -894,7 +895,7 @@ __global__ void __launch_bounds__(kBlock) k_full_update(Fields f, Geo g, Phys ph
   const int gl = xcd_block()*blockDim.x + threadIdx.x;
   const int i = gl/kNodeLanes, sub = gl & (kNodeLanes - 1);
   const bool valid = i < n && sub == 0;
-  int skr = 0;                       // candidate-list check (k_skin_check's measure, fused)
+  int skr = 0;                       // candidate-list check: how far the run has used up its skin
   double skd = 0.0, skg = 0.0;
   double du = 0.0;
   if (i < n) du = compatible_rate<D, R, U>(f, g, i, sub);
